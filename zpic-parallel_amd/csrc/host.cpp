@@ -198,7 +198,7 @@ void swap_buffers( Particles & a, Particles & b ) {
 }
 
 ParticleSort::ParticleSort( uint2 const nt2, uint32_t const max_part )
-    : buf{}, ntiles( nt2.x * nt2.y ), idx_size( max_part ) {
+    : buf{}, ntiles( nt2.x * nt2.y ), idx_size( max_part ), in_parts( false ), listed( false ) {
     buf.idx = device_alloc<int>( max_part );
     buf.npt = device_alloc<int>( 9 * (size_t) ntiles );
     buf.new_np = device_alloc<int>( ntiles );
@@ -215,9 +215,26 @@ void ParticleSort::grow( uint32_t max_part ) {
     buf.idx = nullptr;
     buf.idx = device_alloc<int>( max_part );
     idx_size = max_part;
+    if ( parts.on ) parts.size = part_size( max_part );
+    listed = false;
+}
+
+void ParticleSort::init_parts( uint32_t max_part, int tile_vol ) {
+    parts.on = part_rule( ntiles );
+    if ( !parts.on ) return;
+    parts.size = part_size( max_part );
+    parts.cap = ntiles + PART_TARGET;
+    parts.seg = device_alloc<int>( (size_t) PART_SEG * ntiles );
+    parts.item = device_alloc<int>( 2 * (size_t) parts.cap );
+    parts.total = device_alloc<int>( 1 );
+    parts.npt = device_alloc<int>( 9 * (size_t) parts.cap );
+    parts.energy = device_alloc<double>( parts.cap );
+    parts.J = device_alloc<float>( 3 * (size_t) parts.cap * tile_vol );
 }
 
 ParticleSort::~ParticleSort() {
+    device_free( parts.J ); device_free( parts.energy ); device_free( parts.npt );
+    device_free( parts.total ); device_free( parts.item ); device_free( parts.seg );
     device_free( buf.nmove );
     device_free( buf.total ); device_free( buf.tmp_np ); device_free( buf.seg );
     device_free( buf.new_np ); device_free( buf.npt ); device_free( buf.idx );
@@ -678,6 +695,11 @@ void Species::initialize( float2 const box_, uint2 const ntiles, uint2 const nx,
     particles->periodic = make_int2( bc.x.lower == species::bc::periodic, bc.y.lower == species::bc::periodic );
     tmp = new Particles( ntiles, nx, max_part );
     sort = new ParticleSort( ntiles, max_part );
+    {
+        zpic_geom g{};
+        check( zpic_geom_init( &g, (int) ntiles.x, (int) ntiles.y, (int) nx.x, (int) nx.y, 1, 2 ) );
+        sort->init_parts( max_part, g.tile_vol );
+    }
     const int nt = ntiles.x * ntiles.y;
     d_tile_energy = device_alloc<double>( nt );
     d_energy_dev = device_alloc<double>( 1 );
@@ -727,17 +749,21 @@ void Species::move( vec3grid<float3> * const J ) {
     zpic_geom g = J->geom();
     zpic_particles p = particles->view();
     set_staging( sort->buf );  // the following tile_sort places what this pass stages
+    sort->in_parts = false;
     check( zpic_move_deposit( &p, &g, J->fbuf(), dt_dx.x, dt_dx.y, q, qnx.x, qnx.y, &sort->buf, deterministic,
                               stream() ) );
 }
 
 void Species::tile_sort() { tile_sort( nullptr, 0 ); }
 
-void Species::tile_sort( const int * extra, uint64_t max_extra ) {
+void Species::tile_sort( const int * extra, uint64_t max_extra, bool energy ) {
     zpic_particles p = particles->view(), t = tmp->view();
     const uint2 nt = particles->ntiles, nx = particles->nx;
     const int2 per = particles->periodic;
-    check( zpic_tile_sort_count( &p, &t, &sort->buf, nt.x, nt.y, nx.x, nx.y, per.x, per.y, extra, stream() ) );
+    check( tile_sort_count( &p, &t, &sort->buf, nt.x, nt.y, nx.x, nx.y, per.x, per.y, extra,
+                            sort->in_parts ? &sort->parts : nullptr, energy ? d_tile_energy : nullptr, d_energy_dev,
+                            stream() ) );
+    sort->listed = sort->in_parts;
     int mode = 0;
     int total = 0;
     if ( extra ) {
@@ -752,7 +778,8 @@ void Species::tile_sort( const int * extra, uint64_t max_extra ) {
         }
     }
     if ( mode == 0 ) {
-        check( zpic_tile_sort_copy( &p, &t, &sort->buf, nt.x, nt.y, nx.x, nx.y, per.x, per.y, 0, stream() ) );
+        check( tile_sort_copy( &p, &t, &sort->buf, nt.x, nt.y, nx.x, nx.y, per.x, per.y, 0,
+                               sort->in_parts ? &sort->parts : nullptr, stream() ) );
         return;
     }
     // copy_sorted path (particles.cpp:868-881): grow the staging buffer, copy
@@ -797,6 +824,7 @@ void Species::reinject() {
     inject( range );
     sync();
     np_bound = total;
+    sort->listed = false;
 }
 
 int Species::set_moving_window() {
@@ -834,6 +862,12 @@ void Species::set_staging( zpic_sort & s, bool window ) const {
     s.stage_u = staged ? reinterpret_cast<float *>( tmp->u ) : nullptr;
 }
 
+void Species::list_parts() {
+    if ( !sort->parts.on || sort->listed ) return;
+    check( part_list( particles->np, sort->ntiles, sort->parts, stream() ) );
+    sort->listed = true;
+}
+
 void Species::particle_pass( EMF const & emf, Current & current, bool shift, bool set_j ) {
     const float alpha = 0.5 * dt / m_q;
     const float2 dt_dx = make_float2( dt / dx.x, dt / dx.y );
@@ -841,10 +875,12 @@ void Species::particle_pass( EMF const & emf, Current & current, bool shift, boo
     zpic_geom g = emf.E->geom();
     zpic_particles p = particles->view();
     set_staging( sort->buf, shift );
-    if ( set_j && !deterministic )
-        check( zpic_push_move_deposit_overwrite( &p, &g, emf.E->fbuf(), emf.B->fbuf(), current.J->fbuf(), alpha,
-                                                 dt_dx.x, dt_dx.y, q, qnx.x, qnx.y, d_tile_energy, &sort->buf,
-                                                 reflect_mask(), shift ? -1 : 0, 0, stream() ) );
+    sort->in_parts = sort->buf.stage_ix && sort->parts.on;
+    if ( sort->in_parts ) list_parts();
+    if ( !deterministic )
+        check( push_move_deposit_parts( &p, &g, emf.E->fbuf(), emf.B->fbuf(), current.J->fbuf(), alpha, dt_dx.x,
+                                        dt_dx.y, q, qnx.x, qnx.y, d_tile_energy, &sort->buf, reflect_mask(),
+                                        shift ? -1 : 0, set_j, sort->in_parts ? &sort->parts : nullptr, stream() ) );
     else
         check( zpic_push_move_deposit_shift( &p, &g, emf.E->fbuf(), emf.B->fbuf(), current.J->fbuf(), alpha,
                                              dt_dx.x, dt_dx.y, q, qnx.x, qnx.y, d_tile_energy, &sort->buf,
@@ -857,15 +893,15 @@ void Species::finish_step( bool shift ) {
         const uint2 gd = particles->dims;
         const int range[4] = { (int) gd.x - 1, (int) gd.x - 1, 0, (int) gd.y - 1 };
         np_inject( range, d_np_inj );
-        tile_sort( d_np_inj, (uint64_t) gd.y * ppc.x * ppc.y );
+        tile_sort( d_np_inj, (uint64_t) gd.y * ppc.x * ppc.y, !deterministic );
         inject( range );
         moving_window.advance();
     } else {
-        tile_sort();
+        tile_sort( nullptr, 0, !deterministic );
     }
     iter++;
     const uint2 nt = particles->ntiles;
-    check( zpic_sum_tiles( d_tile_energy, (int) ( nt.x * nt.y ), d_energy_dev, deterministic, stream() ) );
+    if ( deterministic ) check( zpic_sum_tiles( d_tile_energy, (int) ( nt.x * nt.y ), d_energy_dev, 1, stream() ) );
 }
 
 // species.cpp:2088: the window time is (iter + 1) * dt in float
@@ -932,6 +968,7 @@ void Species::set_particles( const int * np, const int * ix, const float * x, co
     to_device( particles->u, reinterpret_cast<const float3 *>( u ), n );
     sync();
     np_bound = n;
+    sort->listed = false;
 }
 
 void Species::subsample_from( const Species & src, int stride, int phase ) {
@@ -946,6 +983,7 @@ void Species::subsample_from( const Species & src, int stride, int phase ) {
                            (int) particles->nx.y, 0, 0 ) );
     check( zpic_subsample( &s, &gs, &d, &gd, stride, phase, stream() ) );
     np_bound = particles->np_total();
+    sort->listed = false;
 }
 
 // Particles::gather (particles.cpp:88-150) with Species::gather's scales
@@ -1253,28 +1291,32 @@ void Batch::build() {
     const size_t nsp = sims[0]->species.size();
     if ( persistent ) {
         std::vector<zpic_batch_species> items;
+        std::vector<PartScratch> parts;
         for ( size_t k = 0; k < nsp; k++ )
             for ( size_t i = 0; i < sims.size(); i++ ) {
                 Simulation * s = sims[i];
                 items.push_back( s->species[k]->batch_item( s->emf, s->current ) );
                 items.back().threads = sim_threads[i];
+                parts.push_back( s->species[k]->part_scratch() );
             }
         std::vector<zpic_batch_fields_item> fitems;
         for ( auto * s : sims ) fitems.push_back( s->batch_fields() );
-        check( zpic_batch_step_create( &persistent_step, items.data(), (int) nsp, fitems.data(), (int) fitems.size(),
-                                       threads ) );
+        check( batch_step_new( &persistent_step, items.data(), (int) nsp, fitems.data(), (int) fitems.size(), threads,
+                               parts.data() ) );
         bound = buffers();
         return;
     }
     for ( size_t k = 0; k < nsp; k++ ) {
         std::vector<zpic_batch_species> items;
+        std::vector<PartScratch> parts;
         for ( size_t i = 0; i < sims.size(); i++ ) {
             Simulation * s = sims[i];
             items.push_back( s->species[k]->batch_item( s->emf, s->current ) );
             items.back().threads = sim_threads[i];
+            parts.push_back( s->species[k]->part_scratch() );
         }
         zpic_batch_particles * plan = nullptr;
-        check( zpic_batch_particles_create( &plan, items.data(), (int) items.size(), threads ) );
+        check( batch_particles_new( &plan, items.data(), (int) items.size(), threads, parts.data() ) );
         slots.push_back( plan );
     }
     std::vector<zpic_batch_fields_item> fitems;
@@ -1301,6 +1343,8 @@ void Batch::advance() {
     // exchange the current's buffers and may grow or swap particle buffers)
     if ( ( fields || persistent_step ) && buffers() != bound ) build();
     if ( !fields && !persistent_step ) build();
+    for ( auto * s : sims )
+        for ( auto * sp : s->species ) sp->list_parts();
     if ( use_graph ) {
         if ( !exec ) {
             hip_check( hipStreamBeginCapture( stream(), hipStreamCaptureModeThreadLocal ), "hipStreamBeginCapture" );

@@ -19,6 +19,7 @@
 // order, which reproduces the reference's single-thread results exactly.
 #include "common.h"
 #include "grid_ops.h"
+#include "parts.h"
 
 #include <algorithm>
 #include <memory>
@@ -50,6 +51,7 @@ struct SortView {
     int2 * stage_ix;  // order-free sort staging (fast mode), or null
     float2 * stage_x;
     float3 * stage_u;
+    int seg_stride;   // ints per tile of seg: 16, or PART_SEG where tiles are taken in parts
 };
 
 struct Geo {
@@ -398,6 +400,13 @@ constexpr int PREFETCH = 2;  // iterations of 64 particles loaded ahead
 constexpr int LBCAP = 32;
 constexpr int LBWORDS = 7;
 
+// A tile's segment table is 16 ints (at most 13 segments), or PART_SEG where
+// tiles are taken in parts (at most PART_MAX_SEG).  Places from its end: the
+// chunk, the tile's old count and old offset; of a tile in parts, parts |
+// segments << 8 and the place of its first part in the list.
+constexpr int SEG_CHUNK = 1, SEG_OLD_NP = 2, SEG_OLD_OFF = 3, SEG_COUNT = 4, SEG_FIRST = 5;
+constexpr int SEG16 = 13;
+
 // LDS of the particle pass: E and B planes (PUSH), W private J triples, W
 // tag arrays and W crossing queues (MOVE), W leaver buffers (lbuf).
 __host__ __device__ inline size_t particles_lds_bytes( int vol, int W, bool push, bool move, bool lbuf = false ) {
@@ -420,6 +429,7 @@ struct PartArgs {
     int waves;  // waves of the workgroup that take particles (0: all)
     int lbuf;   // order-free sort: leavers buffered in LDS (LDS sized for it)
     int jset;   // fast mode: the tile's J region is written, not added to
+    PartScratch parts;  // parts.on (order-free sort): workgroup y takes part y of the list
 };
 
 struct PartG {
@@ -500,9 +510,20 @@ __device__ inline int select_item( A & a, const A * tab, const int2 * map, int g
 // The particle pass of tile t (one workgroup).  `smem` is the workgroup's
 // LDS of particles_lds_bytes( vol, W ) bytes, W = the waves that take
 // particles: all of the workgroup's, or a.waves if that is smaller (the
-// other waves then only join the workgroup barriers).
+// other waves then only join the workgroup barriers).  Where tiles are taken
+// in parts, y is a place in the list of parts, which may be shorter.
 template <bool PUSH, bool MOVE, bool DET>
-__device__ inline void particles_tile( const PartArgs & a, const int t, float * smem ) {
+__device__ inline void particles_tile( const PartArgs & a, const int y, float * smem ) {
+    const bool in_parts = MOVE && !DET && a.parts.on;
+    int t = y, part = 0, nparts = 1;
+    if ( in_parts ) {
+        const gptr<const int> item = gbl( (const int *) a.parts.item ) + 2 * y;
+        const int total = gbl( a.parts.total )[0];
+        t = item[0];
+        part = item[1] & 255;
+        nparts = item[1] >> 8;
+        if ( y >= total ) return;
+    }
     const PartView P = a.P;
     const Geo g = a.g;
     const float3 * __restrict__ E = a.E;
@@ -538,6 +559,11 @@ __device__ inline void particles_tile( const PartArgs & a, const int t, float * 
     __shared__ int s_cnt[9];
     __shared__ double s_en[FAST_BLOCK / WAVE];
     __shared__ int s_nl[FAST_BLOCK / WAVE];
+    const int off = gbl( P.off )[t];
+    const int np = gbl( P.np )[t];
+    // no more segments (waves of all parts) than the tile's table holds
+    nparts = min( nparts, PART_MAX_SEG / W );
+    if ( part >= nparts ) return;
 
     if constexpr ( PUSH ) {
         const gptr<const float> Et = gbl( reinterpret_cast<const float *>( E + (size_t) t * vol ) );
@@ -554,11 +580,10 @@ __device__ inline void particles_tile( const PartArgs & a, const int t, float * 
     }
     __syncthreads();
 
-    const int off = gbl( P.off )[t];
-    const int np = gbl( P.np )[t];
-    const int chunk = ( ( np + W - 1 ) / W + WAVE - 1 ) & ~( WAVE - 1 );
-    const int beg = w * chunk;
-    const int end = min( np, beg + chunk );
+    const int nseg = nparts * W;  // segments of the tile; this wave's is part * W + w
+    const int chunk = ( ( np + nseg - 1 ) / nseg + WAVE - 1 ) & ~( WAVE - 1 );
+    const int beg = ( part * W + w ) * chunk;
+    const int end = w < W ? min( np, beg + chunk ) : beg;  // the waves past W take none
 
     // tile base pointers (uniform) + 32-bit particle index
     const TileArray<int2> pix{ (gptr<char>) gbl( P.ix + off ) };
@@ -855,7 +880,8 @@ __device__ inline void particles_tile( const PartArgs & a, const int t, float * 
     if constexpr ( MOVE ) {
         // flush: J(tile) += sum of the waves' J (LDS), guard cells included
         // (species.cpp:1488-1492)
-        const gptr<float> Jt = gbl( reinterpret_cast<float *>( J + (size_t) t * vol ) );
+        const gptr<float> Jt = gbl( nparts > 1 ? a.parts.J + (size_t) y * 3 * vol
+                                               : reinterpret_cast<float *>( J + (size_t) t * vol ) );
         for ( int k = tid; k < 3 * g.ext_x * g.ext_y; k += nthr ) {
             const int el = k / 3, c = k - 3 * el;
             float s = Jall[c * vol + el];
@@ -863,28 +889,38 @@ __device__ inline void particles_tile( const PartArgs & a, const int t, float * 
             // jset (the first species of a step, fast mode): the region is
             // written instead of zeroed and added to; the same value, since
             // s is never -0 (every plane element starts at +0)
-            if ( !DET && a.jset ) Jt[k] = s;
+            if ( !DET && ( a.jset || nparts > 1 ) ) Jt[k] = s;
             else Jt[k] += s;
         }
         if ( tid == 0 ) {
-            const gptr<int> seg = gbl( S.seg + 16 * t );
-            const gptr<int> npt = gbl( S.npt + 9 * t );
+            const gptr<int> seg = gbl( S.seg + S.seg_stride * t + part * W );
+            const gptr<int> npt = gbl( nparts > 1 ? a.parts.npt + 9 * y : S.npt + 9 * t );
             int tot = 0;
             for ( int v = 0; v < W; v++ ) {
                 seg[v] = s_nl[v];
                 tot += s_nl[v];
             }
-            for ( int v = W; v < MAX_SEG; v++ ) seg[v] = 0;
-            seg[MAX_SEG] = chunk;
+            if ( in_parts ) {
+                if ( part == 0 ) {
+                    seg[PART_SEG - SEG_FIRST] = y;
+                    seg[PART_SEG - SEG_COUNT] = nparts | nseg << 8;
+                    seg[PART_SEG - SEG_CHUNK] = chunk;
+                }
+            } else {
+                for ( int v = W; v < MAX_SEG; v++ ) seg[v] = 0;
+                seg[MAX_SEG] = chunk;
+            }
             for ( int d = 0; d < 9; d++ ) npt[d] = s_cnt[d];
-            npt[4] = np - tot;
+            const int first = min( np, part * W * chunk ), last = min( np, ( part + 1 ) * W * chunk );
+            npt[4] = last - first - tot;
         }
     }
     if constexpr ( PUSH ) {
         if ( tid == 0 ) {
             double s = 0.0;
             for ( int v = 0; v < W; v++ ) s += s_en[v];
-            gbl( tile_energy )[t] = s;
+            if ( nparts > 1 ) gbl( a.parts.energy )[y] = s;
+            else gbl( tile_energy )[t] = s;
         }
     }
 }
@@ -895,6 +931,50 @@ __global__ void __launch_bounds__( FAST_BLOCK ) k_particles( PartArgs a, const P
     const int t = select_instance( a, tab, map );
     particles_tile<PUSH, MOVE, DET>( a, t, smem );
 }
+
+// A tile taken in parts: their J regions, direction counts and energies into
+// the tile's own, in part order (a tile of one part wrote its own).  Slice
+// `slice` of `slices` workgroups of the tile.
+constexpr int MERGE_LOADS = 5;
+__device__ inline void part_merge_tile( const PartArgs & a, const int t, const int slice, const int slices ) {
+    const gptr<const int> end = gbl( (const int *) a.S.seg ) + PART_SEG * ( t + 1 );
+    const int nparts = end[-SEG_COUNT] & 255, first = end[-SEG_FIRST], vol3 = 3 * a.g.vol;
+    if ( nparts < 2 ) return;
+    const gptr<const float> src = gbl( (const float *) a.parts.J ) + (size_t) first * vol3;
+    const gptr<float> Jt = gbl( reinterpret_cast<float *>( a.J ) ) + (size_t) t * vol3;
+    const int n = 3 * a.g.ext_x * a.g.ext_y;
+    for ( int k = slice * blockDim.x + threadIdx.x; k < n; k += slices * blockDim.x ) {
+        float s = a.jset ? 0.0f : Jt[k], sum = 0.0f;
+        for ( int p = 0; p < nparts; p += MERGE_LOADS ) {
+            float v[MERGE_LOADS];
+#pragma unroll
+            for ( int i = 0; i < MERGE_LOADS; i++ ) v[i] = p + i < nparts ? src[(size_t) ( p + i ) * vol3 + k] : 0.0f;
+#pragma unroll
+            for ( int i = 0; i < MERGE_LOADS; i++ ) sum += v[i];
+        }
+        Jt[k] = s + sum;
+    }
+    if ( slice != 0 ) return;
+    if ( threadIdx.x < 9 ) {
+        const gptr<const int> m = gbl( (const int *) a.parts.npt ) + 9 * first + threadIdx.x;
+        int s = 0;
+        for ( int p = 0; p < nparts; p++ ) s += m[9 * p];
+        gbl( a.S.npt )[9 * t + threadIdx.x] = s;
+    } else if ( threadIdx.x == 64 ) {
+        const gptr<const double> e = gbl( (const double *) a.parts.energy ) + first;
+        double s = 0.0;
+        for ( int p = 0; p < nparts; p++ ) s += e[p];
+        gbl( a.tile_energy )[t] = s;
+    }
+}
+
+constexpr int MERGE_BLOCK = 256;
+__global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge( PartArgs a, const PartArgs * tab, const int2 * map ) {
+    const int t = select_instance( a, tab, map );
+    if ( a.parts.on ) part_merge_tile( a, t, blockIdx.y, gridDim.y );
+}
+// workgroups per tile: a tile's elements over several where the tiles are few
+int merge_slices( int ntiles ) { return ntiles <= 256 ? 4 : 1; }
 
 // ---------------------------------------------------------------------------
 // Tile sort.  Directions d = 0..8 encode the motion (d%3-1, d/3-1) of a
@@ -928,6 +1008,7 @@ struct SortArgs {
     SortGeo q;
     int ntiles;
     const int * extra;  // free slots reserved after each tile (may be null)
+    PartScratch parts;  // parts.on: the scan also lists the parts of the next particle pass
 };
 
 // New particle count per tile (bnd_check's new_np, particles.cpp:212-303):
@@ -959,29 +1040,35 @@ __global__ void k_sort_newnp( SortArgs a, const SortArgs * tab ) {
 // carry.  All loads of a round are issued before its scan.
 // BLOCK: the workgroup size (a multiple of 64, at most 64 waves).
 constexpr int SCAN_BLOCK = 1024;
-constexpr int SCAN_K = 16;
-template <int BLOCK>
+// NEWNP: forms the new counts (k_sort_newnp) as well.
+// With parts.on the tiles' parts are scanned along (in the upper half of the
+// 64-bit sums) and the list of parts is written; PARTS_ONLY writes nothing
+// else, from the counts in S.new_np.
+template <int BLOCK, bool PARTS_ONLY = false, int SCAN_K = 16, bool NEWNP = false>
 __device__ inline void sort_count_body( const SortArgs & a ) {
+    typedef unsigned long long u64;
     const SortG S = gview( a.S );
     const gptr<int> new_off = gbl( a.T.off );
     const gptr<const int> extra = gbl( a.extra );
     const gptr<const int> np_old = gbl( (const int *) a.P.np );
-    const bool count_moved = a.S.nmove != nullptr;
+    const bool count_moved = !PARTS_ONLY && a.S.nmove != nullptr;
+    const int psize = a.parts.on ? a.parts.size : 0;
+    auto parts_of = [&]( int n ) { return min( PART_MAX, max( 1, ( n + psize - 1 ) / psize ) ); };
     const int ntiles = a.ntiles;
     const int tid = threadIdx.x, lane = tid % WAVE, w = tid / WAVE;
-    __shared__ int s_wave[BLOCK / WAVE];
+    __shared__ u64 s_wave[BLOCK / WAVE];
     __shared__ unsigned long long s_moved;
     if ( tid == 0 ) s_moved = 0;
     // 16-byte accesses need every array 16-byte aligned (tile starts are
     // multiples of SCAN_K)
     const bool vec = ( ( reinterpret_cast<uintptr_t>( a.S.new_np ) | reinterpret_cast<uintptr_t>( a.T.off ) |
                          reinterpret_cast<uintptr_t>( a.extra ) | reinterpret_cast<uintptr_t>( a.P.np ) ) & 15 ) == 0;
-    int carry = 0;
+    u64 carry = 0;
     unsigned long long moved = 0;
     for ( int base = 0; base < ntiles; base += BLOCK * SCAN_K ) {
         const int t0 = base + tid * SCAN_K;
         int v[SCAN_K];
-        if ( vec && t0 + SCAN_K <= ntiles ) {
+        if ( SCAN_K % 4 == 0 && !NEWNP && vec && t0 + SCAN_K <= ntiles ) {
 #pragma unroll
             for ( int q = 0; q < SCAN_K / 4; q++ ) {
                 const int4 n4 = *(const gptr<int4>) ( S.new_np + t0 + 4 * q );
@@ -1002,39 +1089,56 @@ __device__ inline void sort_count_body( const SortArgs & a ) {
                 const int t = t0 + k;
                 v[k] = 0;
                 if ( t < ntiles ) {
+                    if constexpr ( NEWNP ) sort_newnp_tile( a, t );
                     v[k] = S.new_np[t] + ( a.extra ? extra[t] : 0 );
                     if ( count_moved ) moved += (unsigned) np_old[t];
                 }
             }
         }
-        int sum = 0;
+        u64 sum = 0;
 #pragma unroll
-        for ( int k = 0; k < SCAN_K; k++ ) sum += v[k];
+        for ( int k = 0; k < SCAN_K; k++ ) {
+            sum += (u64) v[k];
+            if ( psize && t0 + k < ntiles ) sum += (u64) parts_of( v[k] ) << 32;
+        }
         // inclusive scan of the thread sums within the wave
-        int x = sum;
+        u64 x = sum;
         for ( int o = 1; o < WAVE; o <<= 1 ) {
-            const int y = __shfl_up( x, o );
+            const u64 y = __shfl_up( x, o );
             if ( lane >= o ) x += y;
         }
         if ( lane == WAVE - 1 ) s_wave[w] = x;
         __syncthreads();
         if ( w == 0 ) {
-            int z = lane < BLOCK / WAVE ? s_wave[lane] : 0;
+            u64 z = lane < BLOCK / WAVE ? s_wave[lane] : 0;
             for ( int o = 1; o < BLOCK / WAVE; o <<= 1 ) {
-                const int y = __shfl_up( z, o );
+                const u64 y = __shfl_up( z, o );
                 if ( lane >= o ) z += y;
             }
             if ( lane < BLOCK / WAVE ) s_wave[lane] = z;  // inclusive wave totals
         }
         __syncthreads();
-        int off = carry + ( w > 0 ? s_wave[w - 1] : 0 ) + x - sum;
+        const u64 start = carry + ( w > 0 ? s_wave[w - 1] : 0 ) + x - sum;
+        int off = (int) (unsigned) start;
+        if ( psize ) {
+            const gptr<int2> item = gbl( reinterpret_cast<int2 *>( a.parts.item ) );
+            int i = (int) ( start >> 32 );
+#pragma unroll
+            for ( int k = 0; k < SCAN_K; k++ ) {
+                if ( t0 + k >= ntiles ) break;
+                const int n = parts_of( v[k] );
+                for ( int p = 0; p < n; p++ ) item[i + p] = make_int2( t0 + k, p | n << 8 );
+                i += n;
+            }
+        }
         int o[SCAN_K];
 #pragma unroll
         for ( int k = 0; k < SCAN_K; k++ ) {
             o[k] = off;
             off += v[k];
         }
-        if ( vec && t0 + SCAN_K <= ntiles ) {
+        if constexpr ( PARTS_ONLY ) {
+        } else if ( SCAN_K % 4 == 0 && vec && t0 + SCAN_K <= ntiles ) {
 #pragma unroll
             for ( int q = 0; q < SCAN_K / 4; q++ )
                 *(gptr<int4>) ( new_off + t0 + 4 * q ) = make_int4( o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3] );
@@ -1046,7 +1150,10 @@ __device__ inline void sort_count_body( const SortArgs & a ) {
         carry += s_wave[BLOCK / WAVE - 1];
         __syncthreads();  // s_wave is rewritten by the next round
     }
-    if ( tid == 0 ) S.total[0] = carry;
+    if ( tid == 0 ) {
+        if constexpr ( !PARTS_ONLY ) S.total[0] = (int) (unsigned) carry;
+        if ( psize ) gbl( a.parts.total )[0] = (int) ( carry >> 32 );
+    }
     // Species::move's d_nmove += np (species.cpp:2162): the counts the
     // particle pass just moved, i.e. before this sort
     if ( count_moved ) {
@@ -1061,6 +1168,48 @@ __device__ inline void sort_count_body( const SortArgs & a ) {
 __global__ void __launch_bounds__( SCAN_BLOCK ) k_sort_count( SortArgs a, const SortArgs * tab ) {
     if ( tab ) a = gbl( tab )[blockIdx.x];
     sort_count_body<SCAN_BLOCK>( a );
+}
+
+__global__ void __launch_bounds__( SCAN_BLOCK ) k_part_list( SortArgs a ) { sort_count_body<SCAN_BLOCK, true>( a ); }
+
+// Per entry: sum of its per-tile push energies (parallel tree, fast mode),
+// written to the entry's energy output.  One workgroup per entry.
+struct EnergyArgs {
+    const double * tile;
+    int n;
+    double * out;
+};
+
+// Sum of an entry's per-tile push energies: per-thread runs, a butterfly
+// within each wave, then the wave sums in wave order (any workgroup size).
+__device__ inline void batch_energy_body( const EnergyArgs & a ) {
+    __shared__ double s_wsum[SCAN_BLOCK / WAVE];
+    const gptr<const double> tile = gbl( a.tile );
+    double acc = 0;
+    for ( int t = threadIdx.x; t < a.n; t += blockDim.x ) acc += tile[t];
+    for ( int o = WAVE / 2; o > 0; o >>= 1 ) acc += __shfl_xor( acc, o );
+    if ( threadIdx.x % WAVE == 0 ) s_wsum[threadIdx.x / WAVE] = acc;
+    __syncthreads();
+    if ( threadIdx.x == 0 ) {
+        double s = 0;
+        for ( int v = 0; v < (int) blockDim.x / WAVE; v++ ) s += s_wsum[v];
+        gbl( a.out )[0] = s;
+    }
+    __syncthreads();  // s_wsum may be reused by the next body in the workgroup
+}
+
+// New counts, offsets and the push energy of an instance of at most
+// SCAN_BLOCK tiles, a thread per tile: three launches' work in one.  (With
+// more tiles the nine counts each tile gathers are too many for one
+// workgroup.)
+__global__ void __launch_bounds__( SCAN_BLOCK ) k_sort_plan( SortArgs a, const SortArgs * tab, EnergyArgs e,
+                                                             const EnergyArgs * etab ) {
+    if ( tab ) {
+        a = gbl( tab )[blockIdx.x];
+        e = gbl( etab )[blockIdx.x];
+    }
+    sort_count_body<SCAN_BLOCK, false, 1, true>( a );
+    if ( e.tile ) batch_energy_body( e );
 }
 
 // Stayers that move to the staging buffer because the tile's range moved
@@ -1376,9 +1525,8 @@ __global__ void __launch_bounds__( SORT_BLOCK ) k_sort_in( SortArgs a, const Sor
 // multisets are).  One wave sorts one tile: the work per tile is a few
 // hundred records behind a chain of dependent loads, so the kernels are
 // bound by latency and gain from as many tiles in flight as possible.
-constexpr int SEG_OLD_OFF = 13, SEG_OLD_NP = 14;
 constexpr int SORT_WAVES = 4;       // tiles per workgroup of k_sort_shift / k_sort_in_fast
-constexpr int SORT_WAVE_LDS = 384;  // ints of LDS per wave
+constexpr int SORT_WAVE_LDS = 512;  // ints of LDS per wave
 constexpr int SORT_BATCH = 4;       // records per lane loaded before any is stored
 
 // Exclusive prefix sum of x over the wave's lanes; `total` gets the sum.
@@ -1402,12 +1550,11 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
 }
 
-// Segment v of a prefix table pre[0..MAX_SEG] (non-decreasing) that holds
-// position k (the last v with pre[v] <= k).
-__device__ inline int segment_of( int k, const int * pre ) {
+// Segment of a prefix table pre[0..n) (non-decreasing) that holds position k
+// (the last v with pre[v] <= k).
+__device__ inline int segment_of( int k, const int * pre, int n ) {
     int w = 0;
-#pragma unroll
-    for ( int v = 1; v < MAX_SEG; v++ ) w += pre[v] <= k;
+    for ( int v = 1; v < n; v++ ) w += pre[v] <= k;
     return w;
 }
 
@@ -1416,11 +1563,14 @@ __device__ inline int cell_dir( int2 c, const SortGeo & q ) {
     return ( ( c.y >= q.ny ) - ( c.y < 0 ) + 1 ) * 3 + ( ( c.x >= q.nx ) - ( c.x < 0 ) + 1 );
 }
 
-// k_sort_shift for tile t by one wave; L = the wave's SORT_WAVE_LDS ints.
-__device__ inline void sort_shift_wave( const SortArgs & a, const int t, int * L ) {
-    int * const seg = L;        // [16] leavers per chunk, [MAX_SEG] = chunk
-    int * const gpre = L + 16;  // [16] free-slot prefix of the staging region
-    int * const pre = L + 32;   // [16] prefix of the leaver counts
+// k_sort_shift for tile t by one wave, or slice `slice` of `slices` waves: a
+// slice takes rounds of the shifted stayers and, of a tile in parts, the
+// leavers of a run of parts, whose direction counts are known.  L = the
+// wave's SORT_WAVE_LDS ints.
+__device__ inline void sort_shift_wave( const SortArgs & a, const int t, int * L, const int slice, const int slices ) {
+    int * const seg = L;         // [64] leavers per chunk
+    int * const gpre = L + 64;   // [64] free-slot prefix of the staging region
+    int * const pre = L + 128;   // [64] prefix of the leaver counts
     const PartG P = gview( a.P );
     const SortG S = gview( a.S );
     const gptr<int2> Gix = gbl( a.S.stage_ix );
@@ -1428,51 +1578,69 @@ __device__ inline void sort_shift_wave( const SortArgs & a, const int t, int * L
     const gptr<float3> Gu = gbl( a.S.stage_u );
     const gptr<const int> new_off = gbl( (const int *) a.T.off );
     const int lane = threadIdx.x % WAVE;
+    const int stride = a.S.seg_stride;
     wave_sync();  // the wave's previous tile has read L
 
-    // lanes 0-15: seg; 16-19: old offset, old count, new offset, new count;
-    // 20-28: direction counts
-    int val = 0;
-    if ( lane <= MAX_SEG ) val = S.seg[16 * t + lane];
-    else if ( lane == 16 ) val = P.off[t];
-    else if ( lane == 17 ) val = P.np[t];
-    else if ( lane == 18 ) val = new_off[t];
-    else if ( lane == 19 ) val = S.new_np[t];
-    else if ( lane < 29 ) val = S.npt[9 * t + lane - 20];
-    const int o = __builtin_amdgcn_readlane( val, 16 ), np = __builtin_amdgcn_readlane( val, 17 );
-    const int no = __builtin_amdgcn_readlane( val, 18 ), nn = __builtin_amdgcn_readlane( val, 19 );
-    const int chunk = __builtin_amdgcn_readlane( val, MAX_SEG );
+    // val: the segment table; hdr: lanes 0-3 old offset, old count, new
+    // offset, new count, 4-12 direction counts
+    const int val = lane < stride ? S.seg[stride * t + lane] : 0;
+    int hdr = 0;
+    if ( lane == 0 ) hdr = P.off[t];
+    else if ( lane == 1 ) hdr = P.np[t];
+    else if ( lane == 2 ) hdr = new_off[t];
+    else if ( lane == 3 ) hdr = S.new_np[t];
+    else if ( lane < 13 ) hdr = S.npt[9 * t + lane - 4];
+    const int o = __builtin_amdgcn_readlane( hdr, 0 ), np = __builtin_amdgcn_readlane( hdr, 1 );
+    const int no = __builtin_amdgcn_readlane( hdr, 2 ), nn = __builtin_amdgcn_readlane( hdr, 3 );
+    const int chunk = __builtin_amdgcn_readlane( val, stride - SEG_CHUNK );
+    const int nseg = stride == PART_SEG ? __builtin_amdgcn_readlane( val, stride - SEG_COUNT ) >> 8 : SEG16;
+    int nl;
     {
         // chunk v = [v chunk, min(np, (v + 1) chunk)), its first seg[v]
         // staging slots hold leavers, the rest are free
         const int v = lane;
-        const int s = v < MAX_SEG ? val : 0;
-        const int len = v < MAX_SEG ? min( max( np - v * chunk, 0 ), chunk ) : 0;
-        int nl, nfree;
+        const int s = v < nseg ? val : 0;
+        const int len = v < nseg ? min( max( np - v * chunk, 0 ), chunk ) : 0;
+        int nfree;
         const int p = wave_excl_scan( s, nl );
-        const int f = wave_excl_scan( v < MAX_SEG ? max( len - s, 0 ) : 0, nfree );
-        if ( v <= MAX_SEG ) {
-            seg[v] = val;
-            pre[v] = v < MAX_SEG ? p : nl;
-            gpre[v] = v < MAX_SEG ? f : nfree;
-        }
+        const int f = wave_excl_scan( max( len - s, 0 ), nfree );
+        seg[v] = s;
+        pre[v] = p;
+        gpre[v] = f;
     }
-    if ( lane == 0 ) {
-        S.seg[16 * t + SEG_OLD_OFF] = o;
-        S.seg[16 * t + SEG_OLD_NP] = np;
+    if ( slice == 0 && lane == 0 ) {
+        S.seg[stride * t + stride - SEG_OLD_OFF] = o;
+        S.seg[stride * t + stride - SEG_OLD_NP] = np;
     }
-    // bucket starts: the leavers of the directions before (lane 20 + d)
+    // the slice's leavers [j_beg, j_end): those of parts [p0, p1)
+    int p0 = 0, first = 0, j_beg = 0, j_end = nl;
+    if ( slices > 1 ) {
+        const int nparts = stride == PART_SEG ? __builtin_amdgcn_readlane( val, stride - SEG_COUNT ) & 255 : 1;
+        const int waves = nseg / nparts;
+        first = __builtin_amdgcn_readlane( val, stride - SEG_FIRST );
+        p0 = slice * nparts / slices;
+        const int p1 = ( slice + 1 ) * nparts / slices;
+        wave_sync();
+        j_beg = p0 > 0 ? pre[p0 * waves] : 0;
+        j_end = p1 == p0 ? j_beg : p1 < nparts ? pre[p1 * waves] : nl;
+    }
+    // bucket starts: the leavers of the directions before, then those of the
+    // parts before (lane 4 + d)
     int dstart, dtot;
     {
-        const int d = lane - 20;
-        dstart = wave_excl_scan( ( d >= 0 && d < 9 && d != 4 ) ? val : 0, dtot );
+        const int d = lane - 4;
+        const bool dir = d >= 0 && d < 9 && d != 4;
+        dstart = wave_excl_scan( dir ? hdr : 0, dtot );
+        if ( p0 > 0 && dir ) {
+            const gptr<const int> m = gbl( (const int *) a.parts.npt ) + 9 * first + d;
+            for ( int p = 0; p < p0; p++ ) dstart += m[9 * p];
+        }
     }
     wave_sync();
 
     // the leavers' cells, SORT_BATCH per lane at a time; the first batch is
     // loaded before the stayer copies below (which write other staging
     // slots), so that the two round trips overlap
-    const int nl = pre[MAX_SEG];
     int pos[SORT_BATCH];
     int2 cl[SORT_BATCH];
     auto load_batch = [&]( int j0 ) {
@@ -1481,52 +1649,54 @@ __device__ inline void sort_shift_wave( const SortArgs & a, const int t, int * L
             const int j = j0 + i * WAVE + lane;
             pos[i] = -1;
             cl[i] = make_int2( 0, 0 );
-            if ( j < nl ) {
-                const int v = segment_of( j, pre );
+            if ( j < j_end ) {
+                const int v = segment_of( j, pre, nseg );
                 pos[i] = v * chunk + ( j - pre[v] );
                 cl[i] = Gix[o + pos[i]];
             }
         }
     };
-    load_batch( 0 );
+    load_batch( j_beg );
 
     // stayers at old-range positions below and above the new range: to the
     // free staging slots in order
     const int a0 = o, la = max( min( o + np, no ) - o, 0 );
     const int b0 = max( o, no + nn ), lb = max( o + np - b0, 0 );
     const int nout = la + lb;
-    int ns = 0;
-    for ( int j0 = 0; j0 < nout; j0 += WAVE ) {
+    // stayers among the old range's first r positions: chunk v holds
+    // len - seg[v] of them, at its front
+    auto stayers_before = [&]( int r ) {
+        if ( r <= 0 ) return 0;
+        const int v = min( r / chunk, nseg - 1 ), len = min( np - v * chunk, chunk );
+        return gpre[v] + min( r - v * chunk, max( len - seg[v], 0 ) );
+    };
+    const int below = stayers_before( la ), skip = stayers_before( lb > 0 ? b0 - o : np );
+    for ( int j0 = slice * WAVE; j0 < nout; j0 += slices * WAVE ) {
         const int j = j0 + lane;
-        bool stay = false;
-        int p = 0;
         if ( j < nout ) {
-            p = j < la ? a0 + j : b0 + ( j - la );
+            const int p = j < la ? a0 + j : b0 + ( j - la );
             const int r = p - o, v = r / chunk, len = min( np - v * chunk, chunk );
-            stay = r - v * chunk < len - seg[v];
+            if ( r - v * chunk < len - seg[v] ) {
+                const int k = j < la ? stayers_before( r ) : below + stayers_before( r ) - skip;
+                const int w = segment_of( k, gpre, nseg );
+                const int dst = o + w * chunk + seg[w] + ( k - gpre[w] );
+                const int2 c = P.ix[p];
+                const float2 x = P.x[p];
+                const float3 u = ld3( P.u + p );
+                Gix[dst] = c;
+                Gx[dst] = x;
+                st3( Gu + dst, u );
+            }
         }
-        const unsigned long long m = __ballot( stay );
-        if ( stay ) {
-            const int k = ns + count_below( m );
-            const int w = segment_of( k, gpre );
-            const int dst = o + w * chunk + seg[w] + ( k - gpre[w] );
-            const int2 c = P.ix[p];
-            const float2 x = P.x[p];
-            const float3 u = ld3( P.u + p );
-            Gix[dst] = c;
-            Gx[dst] = x;
-            st3( Gu + dst, u );
-        }
-        ns += __popcll( m );
     }
-    if ( lane == 0 ) S.tmp_np[t] = ns;
+    if ( slice == 0 && lane == 0 ) S.tmp_np[t] = below + stayers_before( np ) - skip;
 
     // direction buckets of the leavers, staging order kept in each
     int run[9];
 #pragma unroll
-    for ( int d = 0; d < 9; d++ ) run[d] = __builtin_amdgcn_readlane( dstart, 20 + d );
-    for ( int j0 = 0; j0 < nl; j0 += SORT_BATCH * WAVE ) {
-        if ( j0 > 0 ) load_batch( j0 );
+    for ( int d = 0; d < 9; d++ ) run[d] = __builtin_amdgcn_readlane( dstart, 4 + d );
+    for ( int j0 = j_beg; j0 < j_end; j0 += SORT_BATCH * WAVE ) {
+        if ( j0 > j_beg ) load_batch( j0 );
         int dir[SORT_BATCH];
 #pragma unroll
         for ( int i = 0; i < SORT_BATCH; i++ ) dir[i] = pos[i] >= 0 ? cell_dir( cl[i], a.q ) : 4;
@@ -1545,34 +1715,36 @@ __device__ inline void sort_shift_wave( const SortArgs & a, const int t, int * L
     }
 }
 
-__global__ void __launch_bounds__( SORT_WAVES * WAVE ) k_sort_shift( SortArgs a, const SortArgs * tab, const int2 * map, int n ) {
+__global__ void __launch_bounds__( SORT_WAVES * WAVE ) k_sort_shift( SortArgs a, const SortArgs * tab, const int2 * map, int n,
+                                                                   int slices ) {
     __shared__ int s_lds[SORT_WAVES][SORT_WAVE_LDS];
     const int w = __builtin_amdgcn_readfirstlane( (int) threadIdx.x / WAVE );
     const int g = blockIdx.x * SORT_WAVES + w;
-    if ( g >= n ) return;
-    const int t = select_item( a, tab, map, g );
-    sort_shift_wave( a, t, s_lds[w] );
+    if ( g >= n * slices ) return;
+    const int t = select_item( a, tab, map, g / slices );
+    sort_shift_wave( a, t, s_lds[w], g % slices, slices );
 }
 
-// k_sort_in_fast for tile t by one wave; L = the wave's SORT_WAVE_LDS ints.
+// k_sort_in_fast for tile t by one wave, or slice `slice` of `slices` waves
+// (rounds of the ranks below); L = the wave's SORT_WAVE_LDS ints.
 // The slots of the new range [no, no + nn) that none of the tile's stayers
 // holds are runs: the part before the old range, the tail of every chunk
 // (behind its compacted stayers) and the part after the old range.  They
 // are filled in order with the tile's staged stayers, then with its eight
 // sources' leavers towards it, source by source (each in its staging order,
 // from the source's direction bucket).
-__device__ inline void sort_in_fast_wave( const SortArgs & a, const int t, int * L ) {
-    int * const seg = L;          // [9][16] leavers per chunk of the 9 sources (e = 4: the tile)
-    int * const so_s = L + 144;   // [9] source tile
-    int * const so_o = L + 153;   // [9] its old offset
-    int * const so_n = L + 162;   // [9] its old count
-    int * const npt = L + 171;    // [9][9] direction counts of the 9 sources
-    int * const hdr = L + 252;    // [4] new offset, new count, staged stayers
-    int * const gpre = L + 256;   // [16] free-slot prefix of the tile's staging region
-    int * const rb = L + 272;     // [17] hole run starts, in position order
-    int * const rpre = L + 289;   // [18] prefix of their lengths
-    int * const bst = L + 307;    // [9] start of source e's bucket towards the tile
-    int * const ebase = L + 316;  // [10] first rank of source e's particles; [9] = all
+__device__ inline void sort_in_fast_wave( const SortArgs & a, const int t, int * L, const int slice,
+                                          const int slices ) {
+    int * const seg = L;          // [64] the tile's leavers per chunk
+    int * const gpre = L + 64;    // [64] free-slot prefix of the tile's staging region
+    int * const rb = L + 128;     // [64] hole run starts, in position order
+    int * const rpre = L + 192;   // [64] prefix of their lengths
+    int * const npt = L + 256;    // [9][9] direction counts of the 9 sources
+    int * const so_o = L + 337;   // [9] old offset of each source
+    int * const so_n = L + 346;   // [9] its old count
+    int * const hdr = L + 355;    // [3] new offset, new count, staged stayers
+    int * const bst = L + 358;    // [9] start of source e's bucket towards the tile
+    int * const ebase = L + 367;  // [10] first rank of source e's particles; [9] = all
     const PartG P = gview( a.P );
     const SortG S = gview( a.S );
     const gptr<const int2> Gix = gbl( (const int2 *) a.S.stage_ix );
@@ -1581,32 +1753,32 @@ __device__ inline void sort_in_fast_wave( const SortArgs & a, const int t, int *
     const gptr<const int> new_off = gbl( (const int *) a.T.off );
     const SortGeo q = a.q;
     const int lane = threadIdx.x % WAVE;
+    const int stride = a.S.seg_stride;
     wave_sync();  // the wave's previous tile has read L
 
-    // set-up: every load at once (228 values, four per lane)
+    // set-up: every load at once (the tile's segment table; the sources' old
+    // ranges, the tile's header, the sources' direction counts)
+    const int val = lane < stride ? S.seg[stride * t + lane] : 0;
 #pragma unroll
-    for ( int i = 0; i < 4; i++ ) {
+    for ( int i = 0; i < 2; i++ ) {
         const int k = i * WAVE + lane;
-        if ( k < 144 ) {
-            const int e = k / 16, v = k % 16;
-            const int s = ( e == 4 ) ? t : source_of( t, e, q );
-            const int x = s >= 0 ? S.seg[16 * s + v] : 0;
-            seg[k] = ( v == SEG_OLD_OFF || v == SEG_OLD_NP ) ? 0 : x;
-            if ( v == SEG_OLD_OFF ) so_o[e] = x;
-            if ( v == SEG_OLD_NP ) so_n[e] = x;
-            if ( v == 0 ) so_s[e] = s;
-        } else if ( k < 144 + 81 ) {
-            const int e = ( k - 144 ) / 9, d = ( k - 144 ) % 9;
+        if ( k < 81 ) {
+            const int e = k / 9, d = k % 9;
             const int s = source_of( t, e, q );
-            npt[k - 144] = ( e != 4 && s >= 0 ) ? S.npt[9 * s + d] : 0;
-        } else if ( k < 144 + 81 + 3 ) {
-            const int h = k - 225;
-            hdr[h] = h == 0 ? new_off[t] : h == 1 ? S.new_np[t] : S.tmp_np[t];
+            npt[k] = ( e != 4 && s >= 0 ) ? S.npt[9 * s + d] : 0;
+        } else if ( k < 99 ) {
+            const int e = ( k - 81 ) % 9, which = ( k - 81 ) / 9;
+            const int s = ( e == 4 ) ? t : source_of( t, e, q );
+            const int x = s >= 0 ? S.seg[stride * s + stride - ( which ? SEG_OLD_NP : SEG_OLD_OFF )] : 0;
+            ( which ? so_n : so_o )[e] = x;
+        } else if ( k < 102 ) {
+            hdr[k - 99] = k == 99 ? new_off[t] : k == 100 ? S.new_np[t] : S.tmp_np[t];
         }
     }
     wave_sync();
 
-    const int o = so_o[4], np = so_n[4], chunk = seg[4 * 16 + MAX_SEG];
+    const int o = so_o[4], np = so_n[4], chunk = __builtin_amdgcn_readlane( val, stride - SEG_CHUNK );
+    const int nseg = stride == PART_SEG ? __builtin_amdgcn_readlane( val, stride - SEG_COUNT ) >> 8 : SEG16;
     const int no = hdr[0], nn = hdr[1], ns = hdr[2];
     {
         // lanes 0-8: source e's bucket towards the tile and its first rank
@@ -1624,57 +1796,50 @@ __device__ inline void sort_in_fast_wave( const SortArgs & a, const int t, int *
         }
         if ( e == 9 ) ebase[9] = ns + all;
     }
+    int nholes;
     {
-        // lanes 0-14: chunk v's free staging slots (behind its leavers)
+        // lane v: chunk v's free staging slots (behind its leavers)
         const int v = lane;
-        const int len = v < MAX_SEG && chunk > 0 ? min( max( np - v * chunk, 0 ), chunk ) : 0;
-        const int sv = v < MAX_SEG ? seg[4 * 16 + v] : 0;
+        const int sv = v < nseg ? val : 0;
+        const int len = v < nseg ? min( max( np - v * chunk, 0 ), chunk ) : 0;
         int nfree;
-        const int f = wave_excl_scan( v < MAX_SEG ? max( len - sv, 0 ) : 0, nfree );
-        if ( v <= MAX_SEG ) gpre[v] = v < MAX_SEG ? f : nfree;
-    }
-    {
-        // lanes 0-16: hole runs of the new range, clipped to it: before the
-        // old range, behind chunk r - 1's stayers, after the old range
+        const int f = wave_excl_scan( max( len - sv, 0 ), nfree );
+        seg[v] = sv;
+        gpre[v] = f;
+        // hole runs of the new range, clipped to it: before the old range,
+        // behind chunk r - 1's stayers, after the old range (lane r)
         const int r = lane;
+        const int sl = __shfl_up( sv, 1 ), ll = __shfl_up( len, 1 );
         int b = 0, en = 0;
         if ( r == 0 ) {
             b = no;
             en = o;
-        } else if ( r <= MAX_SEG ) {
-            const int v = r - 1;
-            const int len = chunk > 0 ? min( max( np - v * chunk, 0 ), chunk ) : 0;
-            b = o + v * chunk + ( len - seg[4 * 16 + v] );
-            en = o + v * chunk + len;
-        } else if ( r == MAX_SEG + 1 ) {
+        } else if ( r <= nseg ) {
+            b = o + ( r - 1 ) * chunk + ( ll - sl );
+            en = o + ( r - 1 ) * chunk + ll;
+        } else if ( r == nseg + 1 ) {
             b = o + np;
             en = no + nn;
         }
         b = max( b, no );
         en = min( en, no + nn );
-        int nholes;
-        const int rp = wave_excl_scan( r <= MAX_SEG + 1 ? max( en - b, 0 ) : 0, nholes );
-        if ( r <= MAX_SEG + 1 ) {
-            rb[r] = b;
-            rpre[r] = rp;
-        }
-        if ( r == MAX_SEG + 2 ) rpre[r] = nholes;
+        const int rp = wave_excl_scan( r <= nseg + 1 ? max( en - b, 0 ) : 0, nholes );
+        rb[r] = b;
+        rpre[r] = rp;
     }
     wave_sync();
 
-    const int nholes = rpre[MAX_SEG + 2], ntot = ebase[9];
+    const int ntot = ebase[9];
     // position of fill rank k (-1 past the holes: the counts always balance)
     auto slot = [&]( int k ) {
         if ( k >= nholes ) return -1;
-        int r = 0;
-#pragma unroll
-        for ( int v = 1; v < MAX_SEG + 2; v++ ) r += rpre[v] <= k;
+        const int r = segment_of( k, rpre, nseg + 2 );
         return rb[r] + ( k - rpre[r] );
     };
     // ranks [0, ns): the tile's staged stayers; [ebase[e], ebase[e + 1]):
     // source e's bucket towards the tile.  SORT_BATCH ranks per lane are
     // resolved and loaded before any is written.
-    for ( int k0 = 0; k0 < ntot; k0 += SORT_BATCH * WAVE ) {
+    for ( int k0 = slice * SORT_BATCH * WAVE; k0 < ntot; k0 += slices * SORT_BATCH * WAVE ) {
         int src[SORT_BATCH], dst[SORT_BATCH], sh[SORT_BATCH];
 #pragma unroll
         for ( int i = 0; i < SORT_BATCH; i++ ) {
@@ -1685,8 +1850,8 @@ __device__ inline void sort_in_fast_wave( const SortArgs & a, const int t, int *
             if ( k < ntot ) {
                 dst[i] = slot( k );
                 if ( k < ns ) {
-                    const int v = segment_of( k, gpre );
-                    src[i] = o + v * chunk + seg[4 * 16 + v] + ( k - gpre[v] );
+                    const int v = segment_of( k, gpre, nseg );
+                    src[i] = o + v * chunk + seg[v] + ( k - gpre[v] );
                 } else {
                     int e = 0;
 #pragma unroll
@@ -1723,19 +1888,24 @@ __device__ inline void sort_in_fast_wave( const SortArgs & a, const int t, int *
             }
         }
     }
-    if ( lane == 0 ) {
+    if ( slice == 0 && lane == 0 ) {
         P.np[t] = nn;
         P.off[t] = no;
     }
 }
 
-__global__ void __launch_bounds__( SORT_WAVES * WAVE ) k_sort_in_fast( SortArgs a, const SortArgs * tab, const int2 * map, int n ) {
+// Waves per tile of the two kernels above: one fills the device from 8192
+// tiles on, and a crowded tile's wave holds up fewer.
+int sort_slices( int ntiles ) { return std::max( 1, std::min( 16, 8192 / std::max( ntiles, 1 ) ) ); }
+
+__global__ void __launch_bounds__( SORT_WAVES * WAVE ) k_sort_in_fast( SortArgs a, const SortArgs * tab, const int2 * map, int n,
+                                                                   int slices ) {
     __shared__ int s_lds[SORT_WAVES][SORT_WAVE_LDS];
     const int w = __builtin_amdgcn_readfirstlane( (int) threadIdx.x / WAVE );
     const int g = blockIdx.x * SORT_WAVES + w;
-    if ( g >= n ) return;
-    const int t = select_item( a, tab, map, g );
-    sort_in_fast_wave( a, t, s_lds[w] );
+    if ( g >= n * slices ) return;
+    const int t = select_item( a, tab, map, g / slices );
+    sort_in_fast_wave( a, t, s_lds[w], g % slices, slices );
 }
 
 // ---------------------------------------------------------------------------
@@ -1800,6 +1970,7 @@ PartView view( const zpic_particles * p ) {
 
 SortView view( const zpic_sort * s ) {
     SortView v;
+    v.seg_stride = 16;
     if ( s ) {
         v.idx = s->idx; v.npt = s->npt; v.new_np = s->new_np; v.seg = s->seg; v.tmp_np = s->tmp_np; v.total = s->total;
         v.nmove = s->nmove;
@@ -1852,10 +2023,19 @@ int check_threads( int threads ) {
     return ZPIC_OK;
 }
 
+// Tiles in parts need the order-free sort (its segment table).
+bool parts_on( const SortView & S, const PartScratch * parts ) { return parts && parts->on && S.stage_ix; }
+void use_parts( PartArgs & a, const PartScratch * parts ) {
+    if ( !parts_on( a.S, parts ) ) return;
+    a.parts = *parts;
+    a.S.seg = parts->seg;
+    a.S.seg_stride = PART_SEG;
+}
+
 template <bool PUSH, bool MOVE>
 int launch_particles( const zpic_particles * p, const zpic_geom * fld, const float * E, const float * B, float * J,
                       float alpha, MoveArgs m, double * tile_energy, zpic_sort * s, int det, void * stream,
-                      int jset = 0 ) {
+                      int jset = 0, const PartScratch * parts = nullptr ) {
     if ( int rc = check_geom( fld ) ) return rc;
     if ( !p || ( PUSH && ( !E || !B || !tile_energy ) ) || ( MOVE && ( !J || !s ) ) )
         return set_error( ZPIC_EINVAL, "null buffer" );
@@ -1884,20 +2064,34 @@ int launch_particles( const zpic_particles * p, const zpic_geom * fld, const flo
         }
     }
     hipStream_t st = as_stream( stream );
-    if ( det )
-        hipLaunchKernelGGL( ( k_particles<PUSH, MOVE, true> ), dim3( nt ), dim3( threads ), lds, st, a,
-                            (const PartArgs *) nullptr, (const int2 *) nullptr );
-    else
-        hipLaunchKernelGGL( ( k_particles<PUSH, MOVE, false> ), dim3( nt ), dim3( threads ), lds, st, a,
-                            (const PartArgs *) nullptr, (const int2 *) nullptr );
+    const PartArgs * tab = nullptr;
+    const int2 * map = nullptr;
+    if ( det ) {
+        hipLaunchKernelGGL( ( k_particles<PUSH, MOVE, true> ), dim3( nt ), dim3( threads ), lds, st, a, tab, map );
+        ZPIC_LAUNCH_CHECK( "k_particles" );
+        return ZPIC_OK;
+    }
+    use_parts( a, parts );
+    const int blocks = a.parts.on ? a.parts.cap : nt;
+    hipLaunchKernelGGL( ( k_particles<PUSH, MOVE, false> ), dim3( blocks ), dim3( threads ), lds, st, a, tab, map );
     ZPIC_LAUNCH_CHECK( "k_particles" );
+    if ( a.parts.on ) {
+        hipLaunchKernelGGL( k_part_merge, dim3( nt, merge_slices( nt ) ), dim3( MERGE_BLOCK ), 0, st, a, tab, map );
+        ZPIC_LAUNCH_CHECK( "k_part_merge" );
+    }
     return ZPIC_OK;
 }
 
 SortArgs sort_args( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntx, int nty, int nx, int ny, int px,
-                    int py ) {
+                    int py, const PartScratch * parts = nullptr ) {
     SortArgs a;
     a.P = view( p ); a.T = view( tmp ); a.S = view( s );
+    a.parts = PartScratch();
+    if ( parts_on( a.S, parts ) ) {
+        a.S.seg = parts->seg;
+        a.S.seg_stride = PART_SEG;
+        a.parts = *parts;
+    }
     a.q = SortGeo{ ntx, nty, nx, ny, px ? 1 : 0, py ? 1 : 0 };
     a.ntiles = ntx * nty;
     a.extra = nullptr;
@@ -1907,14 +2101,6 @@ SortArgs sort_args( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int
 }  // namespace
 
 // ------------------------------------------------------------------ batches
-// Per entry: sum of its per-tile push energies (parallel tree, fast mode),
-// written to the entry's energy output.  One workgroup per entry.
-struct EnergyArgs {
-    const double * tile;
-    int n;
-    double * out;
-};
-
 // Device tables for one launch per stage over many independent instances:
 // entry e of a table holds the arguments of one (instance, species) pair,
 // map[b] = (entry, tile) for block b.
@@ -1928,12 +2114,22 @@ struct BatchParticlePlan {
     bool staged = false;       // every entry uses the order-free sort
     PartArgs * d_part = nullptr;
     SortArgs * d_sort = nullptr;
-    int2 * d_map = nullptr;
+    int2 * d_map = nullptr;    // block -> (entry, tile)
+    int2 * d_items = nullptr;  // particle pass: block -> (entry, part of a tile)
+    int nitems = 0;
     EnergyArgs * d_energy = nullptr;  // [nentries]
     std::vector<PartArgs> h_part;
 };
 
-int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species * items, int n, int threads ) {
+void batch_particles_destroy( BatchParticlePlan * plan ) {
+    if ( !plan ) return;
+    (void) hipFree( plan->d_part ); (void) hipFree( plan->d_sort ); (void) hipFree( plan->d_map );
+    (void) hipFree( plan->d_items ); (void) hipFree( plan->d_energy );
+    delete plan;
+}
+
+int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species * items, int n, int threads,
+                            const PartScratch * parts ) {
     if ( !out || !items || n < 1 ) return set_error( ZPIC_EINVAL, "empty batch" );
     if ( int rc = check_threads( threads ) ) return rc;
     auto * plan = new BatchParticlePlan();
@@ -1941,7 +2137,7 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
     plan->nentries = n;
     std::vector<SortArgs> sorts( n );
     std::vector<EnergyArgs> energies( n );
-    std::vector<int2> map;
+    std::vector<int2> map, pmap;
     for ( int e = 0; e < n; e++ ) {
         const zpic_batch_species & it = items[e];
         if ( int rc = check_geom( &it.fld ) ) { delete plan; return rc; }
@@ -1952,6 +2148,7 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
         a.tile_energy = it.tile_energy;
         zpic_sort s = it.s;
         a.S = view( &s );
+        use_parts( a, parts ? parts + e : nullptr );
         // each entry runs with the threads that fit its own tiles, as its own
         // single-instance pass does
         if ( it.threads && check_threads( it.threads ) ) { delete plan; return ZPIC_EINVAL; }
@@ -1963,14 +2160,16 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
         plan->h_part.push_back( a );
         zpic_particles p = it.p, t = it.tmp;
         sorts[e] = sort_args( &p, &t, &s, it.fld.ntiles_x, it.fld.ntiles_y, it.fld.nx, it.fld.ny, it.periodic_x,
-                              it.periodic_y );
+                              it.periodic_y, parts ? parts + e : nullptr );
         const int nt = it.fld.ntiles_x * it.fld.ntiles_y;
         energies[e] = EnergyArgs{ it.tile_energy, nt, it.energy_out };
         for ( int t2 = 0; t2 < nt; t2++ ) map.push_back( make_int2( e, t2 ) );
+        for ( int y = 0; y < ( a.parts.on ? a.parts.cap : nt ); y++ ) pmap.push_back( make_int2( e, y ) );
         plan->max_tiles = std::max( plan->max_tiles, nt );
         plan->max_vol = std::max( plan->max_vol, it.fld.tile_vol );
     }
     plan->nblocks = (int) map.size();
+    plan->nitems = (int) pmap.size();
     {
         int nst = 0;
         for ( int e = 0; e < n; e++ ) nst += items[e].s.stage_ix != nullptr;
@@ -1984,69 +2183,35 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
     hipError_t e2 = hipMalloc( (void **) &plan->d_sort, sizeof( SortArgs ) * n );
     hipError_t e3 = hipMalloc( (void **) &plan->d_map, sizeof( int2 ) * map.size() );
     hipError_t e4 = hipMalloc( (void **) &plan->d_energy, sizeof( EnergyArgs ) * n );
-    if ( e1 || e2 || e3 || e4 ) {
-        (void) hipFree( plan->d_part ); (void) hipFree( plan->d_sort ); (void) hipFree( plan->d_map );
-        (void) hipFree( plan->d_energy );
-        delete plan;
+    hipError_t e5 = hipMalloc( (void **) &plan->d_items, sizeof( int2 ) * pmap.size() );
+    if ( e1 || e2 || e3 || e4 || e5 ) {
+        batch_particles_destroy( plan );
         return set_error( ZPIC_EHIP, "hipMalloc failed for batch tables" );
     }
     ZPIC_HIP_TRY( hipMemcpy( plan->d_part, plan->h_part.data(), sizeof( PartArgs ) * n, hipMemcpyHostToDevice ) );
     ZPIC_HIP_TRY( hipMemcpy( plan->d_sort, sorts.data(), sizeof( SortArgs ) * n, hipMemcpyHostToDevice ) );
     ZPIC_HIP_TRY( hipMemcpy( plan->d_map, map.data(), sizeof( int2 ) * map.size(), hipMemcpyHostToDevice ) );
+    ZPIC_HIP_TRY( hipMemcpy( plan->d_items, pmap.data(), sizeof( int2 ) * pmap.size(), hipMemcpyHostToDevice ) );
     ZPIC_HIP_TRY( hipMemcpy( plan->d_energy, energies.data(), sizeof( EnergyArgs ) * n, hipMemcpyHostToDevice ) );
     *out = plan;
     return ZPIC_OK;
-}
-
-void batch_particles_destroy( BatchParticlePlan * plan ) {
-    if ( !plan ) return;
-    (void) hipFree( plan->d_part ); (void) hipFree( plan->d_sort ); (void) hipFree( plan->d_map );
-    (void) hipFree( plan->d_energy );
-    delete plan;
-}
-
-// Sum of an entry's per-tile push energies: per-thread runs, a butterfly
-// within each wave, then the wave sums in wave order (any workgroup size).
-__device__ inline void batch_energy_body( const EnergyArgs & a ) {
-    __shared__ double s_wsum[FAST_BLOCK / WAVE];
-    const gptr<const double> tile = gbl( a.tile );
-    double acc = 0;
-    for ( int t = threadIdx.x; t < a.n; t += blockDim.x ) acc += tile[t];
-    for ( int o = WAVE / 2; o > 0; o >>= 1 ) acc += __shfl_xor( acc, o );
-    if ( threadIdx.x % WAVE == 0 ) s_wsum[threadIdx.x / WAVE] = acc;
-    __syncthreads();
-    if ( threadIdx.x == 0 ) {
-        double s = 0;
-        for ( int v = 0; v < (int) blockDim.x / WAVE; v++ ) s += s_wsum[v];
-        gbl( a.out )[0] = s;
-    }
-    __syncthreads();  // s_wsum may be reused by the next body in the workgroup
 }
 
 __global__ void __launch_bounds__( 256 ) k_batch_energy( const EnergyArgs * tab ) {
     batch_energy_body( gbl( tab )[blockIdx.x] );
 }
 
-int batch_particles_step( BatchParticlePlan * plan, void * stream ) {
-    hipStream_t st = as_stream( stream );
-    PartArgs dummy{};
-    hipLaunchKernelGGL( ( k_particles<true, true, false> ), dim3( plan->nblocks ), dim3( plan->threads ), plan->lds, st,
-                        dummy, (const PartArgs *) plan->d_part, (const int2 *) plan->d_map );
-    ZPIC_LAUNCH_CHECK( "k_particles (batch)" );
-    SortArgs sd{};
-    hipLaunchKernelGGL( k_sort_newnp, dim3( ( plan->max_tiles + 255 ) / 256, plan->nentries ), dim3( 256 ), 0, st, sd,
-                        (const SortArgs *) plan->d_sort );
-    ZPIC_LAUNCH_CHECK( "k_sort_newnp (batch)" );
-    hipLaunchKernelGGL( k_sort_count, dim3( plan->nentries ), dim3( SCAN_BLOCK ), 0, st, sd,
-                        (const SortArgs *) plan->d_sort );
-    ZPIC_LAUNCH_CHECK( "k_sort_count (batch)" );
+// The sort's passes after the new counts and offsets.
+int batch_particles_place( BatchParticlePlan * plan, hipStream_t st ) {
+    const SortArgs sd{};
     if ( plan->staged ) {
-        const dim3 grid( ( plan->nblocks + SORT_WAVES - 1 ) / SORT_WAVES );
+        const int slices = sort_slices( plan->nblocks );
+        const dim3 grid( ( plan->nblocks * slices + SORT_WAVES - 1 ) / SORT_WAVES );
         hipLaunchKernelGGL( k_sort_shift, grid, dim3( SORT_WAVES * WAVE ), 0, st, sd, (const SortArgs *) plan->d_sort,
-                            (const int2 *) plan->d_map, plan->nblocks );
+                            (const int2 *) plan->d_map, plan->nblocks, slices );
         ZPIC_LAUNCH_CHECK( "k_sort_shift (batch)" );
         hipLaunchKernelGGL( k_sort_in_fast, grid, dim3( SORT_WAVES * WAVE ), 0, st, sd, (const SortArgs *) plan->d_sort,
-                            (const int2 *) plan->d_map, plan->nblocks );
+                            (const int2 *) plan->d_map, plan->nblocks, slices );
         ZPIC_LAUNCH_CHECK( "k_sort_in_fast (batch)" );
     } else {
         hipLaunchKernelGGL( k_sort_out<false>, dim3( plan->nblocks ), dim3( SORT_BLOCK ), 0, st, sd,
@@ -2056,9 +2221,36 @@ int batch_particles_step( BatchParticlePlan * plan, void * stream ) {
                             (const SortArgs *) plan->d_sort, (const int2 *) plan->d_map );
         ZPIC_LAUNCH_CHECK( "k_sort_in (batch)" );
     }
+    return ZPIC_OK;
+}
+
+int batch_particles_step( BatchParticlePlan * plan, void * stream ) {
+    hipStream_t st = as_stream( stream );
+    PartArgs dummy{};
+    hipLaunchKernelGGL( ( k_particles<true, true, false> ), dim3( plan->nitems ), dim3( plan->threads ), plan->lds, st,
+                        dummy, (const PartArgs *) plan->d_part, (const int2 *) plan->d_items );
+    ZPIC_LAUNCH_CHECK( "k_particles (batch)" );
+    if ( plan->nitems > plan->nblocks ) {
+        hipLaunchKernelGGL( k_part_merge, dim3( plan->nblocks, merge_slices( plan->nblocks ) ), dim3( MERGE_BLOCK ), 0, st, dummy,
+                            (const PartArgs *) plan->d_part, (const int2 *) plan->d_map );
+        ZPIC_LAUNCH_CHECK( "k_part_merge (batch)" );
+    }
+    SortArgs sd{};
+    if ( plan->max_tiles <= SCAN_BLOCK ) {
+        hipLaunchKernelGGL( k_sort_plan, dim3( plan->nentries ), dim3( SCAN_BLOCK ), 0, st, sd,
+                            (const SortArgs *) plan->d_sort, EnergyArgs{}, (const EnergyArgs *) plan->d_energy );
+        ZPIC_LAUNCH_CHECK( "k_sort_plan (batch)" );
+        return batch_particles_place( plan, st );
+    }
+    hipLaunchKernelGGL( k_sort_newnp, dim3( ( plan->max_tiles + 255 ) / 256, plan->nentries ), dim3( 256 ), 0, st, sd,
+                        (const SortArgs *) plan->d_sort );
+    ZPIC_LAUNCH_CHECK( "k_sort_newnp (batch)" );
+    hipLaunchKernelGGL( k_sort_count, dim3( plan->nentries ), dim3( SCAN_BLOCK ), 0, st, sd,
+                        (const SortArgs *) plan->d_sort );
+    ZPIC_LAUNCH_CHECK( "k_sort_count (batch)" );
     hipLaunchKernelGGL( k_batch_energy, dim3( plan->nentries ), dim3( 256 ), 0, st, (const EnergyArgs *) plan->d_energy );
     ZPIC_LAUNCH_CHECK( "k_batch_energy" );
-    return ZPIC_OK;
+    return batch_particles_place( plan, st );
 }
 
 namespace {
@@ -2079,7 +2271,8 @@ namespace {
 // particle pass.
 enum StepKind : int {
     SK_ZERO = 0,  // Current::zero of tiles [t0, t1)
-    SK_PART,      // particle pass of tiles [t0, t1), one after the other
+    SK_PART,      // particle pass of items [t0, t1) (tiles, or parts of them), one after the other
+    SK_MERGE,     // J regions and counts of tiles taken in parts (tiles [t0, t1))
     SK_NEWNP,     // new per-tile counts of tiles [t0, t1)
     SK_COUNT,     // offsets scan, nmove and push energy of the species
     SK_SHIFT,     // order-free sort: stayers outside the new range staged (tiles [t0, t1))
@@ -2233,6 +2426,11 @@ __global__ void __launch_bounds__( BLOCK, 4 ) k_batch_step( StepTables T ) {
             }
             break;
         }
+        case SK_MERGE: {
+            const PartArgs a = uniform_load( T.part + it.arg );
+            for ( int t = it.t0; t < it.t1; t++ ) part_merge_tile( a, t, 0, 1 );
+            break;
+        }
         case SK_NEWNP: {
             const SortArgs a = uniform_load( T.sort + it.arg );
             for ( int t = it.t0 + (int) threadIdx.x; t < it.t1; t += BLOCK ) sort_newnp_tile( a, t );
@@ -2250,8 +2448,8 @@ __global__ void __launch_bounds__( BLOCK, 4 ) k_batch_step( StepTables T ) {
             const int w = __builtin_amdgcn_readfirstlane( (int) threadIdx.x / WAVE );
             int * L = reinterpret_cast<int *>( smem ) + w * SORT_WAVE_LDS;
             for ( int t = it.t0 + w; t < it.t1; t += BLOCK / WAVE ) {
-                if ( it.kind == SK_SHIFT ) sort_shift_wave( a, t, L );
-                else sort_in_fast_wave( a, t, L );
+                if ( it.kind == SK_SHIFT ) sort_shift_wave( a, t, L, 0, 1 );
+                else sort_in_fast_wave( a, t, L, 0, 1 );
             }
             break;
         }
@@ -2356,7 +2554,7 @@ std::vector<FilterPass> filter_passes( const zpic_batch_fields_item & it ) {
 }
 
 int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int nslots, const zpic_batch_fields_item * fl,
-                       int n, int threads ) {
+                       int n, int threads, const PartScratch * parts ) {
     if ( !out || !sp || !fl || n < 1 || nslots < 1 ) return set_error( ZPIC_EINVAL, "empty batch" );
     if ( int rc = check_threads( threads ) ) return rc;
     auto plan = std::make_unique<BatchStepPlan>();
@@ -2437,10 +2635,12 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
             a.tile_energy = it.tile_energy;
             zpic_sort s = it.s;
             a.S = view( &s );
+            use_parts( a, parts ? parts + k * n + i : nullptr );
             a.waves = waves[i];
             part[k * n + i] = a;
             zpic_particles p = it.p, t = it.tmp;
-            sort[k * n + i] = sort_args( &p, &t, &s, it.fld.ntiles_x, it.fld.ntiles_y, it.fld.nx, it.fld.ny, 1, 1 );
+            sort[k * n + i] = sort_args( &p, &t, &s, it.fld.ntiles_x, it.fld.ntiles_y, it.fld.nx, it.fld.ny, 1, 1,
+                                         parts ? parts + k * n + i : nullptr );
             ener[k * n + i] = EnergyArgs{ it.tile_energy, it.fld.ntiles_x * it.fld.ntiles_y, it.energy_out };
         }
     }
@@ -2452,7 +2652,10 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     };
     std::vector<Stage> stages;
     stages.push_back( { SK_ZERO, 0 } );
-    for ( int k = 0; k < nslots; k++ ) stages.push_back( { SK_PART, k } );
+    for ( int k = 0; k < nslots; k++ ) {
+        stages.push_back( { SK_PART, k } );
+        stages.push_back( { SK_MERGE, k } );
+    }
     for ( int k = 0; k < nslots; k++ ) {
         stages.push_back( { SK_NEWNP, k } );
         stages.push_back( { SK_COUNT, k } );
@@ -2472,7 +2675,6 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
 
     // tiles per item of the light stages
     constexpr int ZERO_TILES = 32, NEWNP_TILES = 1024, GC_TILES = 16;
-    constexpr long long PART_GRAIN = 65536;
     constexpr int CELL_GRAIN = 4096;
     // tiles per item of the per-tile stages: small tiles are grouped so that
     // an item moves at least ~65536 particles (particle pass, sort) or covers
@@ -2481,6 +2683,11 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     // 64-instance scan: 17.8 ms per step at 16384 / 1024, 14.1 ms at 65536 /
     // 4096, 18.7 ms at 262144 / 16384, where too few items remain to fill the
     // device)
+    // (the particles' grain shrinks with the batch, so that each of the device's
+    // workgroups still gets a few of the particle pass's items)
+    long long all = 0;
+    for ( int k = 0; k < nslots * n; k++ ) all += sp[k].p.max_part;
+    const long long PART_GRAIN = std::max( 4096LL, std::min( 65536LL, all / 4096 ) );
     std::vector<int> part_group( n ), cell_group( n );
     for ( int i = 0; i < n; i++ ) {
         const int cells = fl[i].g.nx * fl[i].g.ny;
@@ -2496,7 +2703,7 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     std::vector<int> need( (size_t) ns * n, 0 );  // items per (stage, instance)
     std::vector<std::vector<StepItem>> per_stage( ns );
     std::vector<int> last( n, -1 );  // last stage with items, per instance (current chain)
-    std::vector<int> part_stage( n, -1 );
+    std::vector<int> part_stage( (size_t) nslots * n, -1 );  // a species' last stage before its sort
     for ( int si = 0; si < ns; si++ ) {
         const Stage st = stages[si];
         for ( int oi = 0; oi < n; oi++ ) {
@@ -2520,14 +2727,24 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
                 break;
             case SK_PART:
                 dep = last[i] * n + i;
-                for ( int t = 0; t < nt; t += part_group[i] )
-                    push( SK_PART, st.slot * n + i, t, std::min( nt, t + part_group[i] ), dep );
-                last[i] = si;
-                part_stage[i] = si;
+            {
+                // a tile in parts: each item takes the particles of part_group tiles
+                const PartScratch & pt = part[st.slot * n + i].parts;
+                const int ny = pt.on ? pt.cap : nt;
+                const int step = pt.on ? std::max( part_group[i], (int) ( PART_GRAIN / pt.size ) ) : part_group[i];
+                for ( int y = 0; y < ny; y += step ) push( SK_PART, st.slot * n + i, y, std::min( ny, y + step ), dep );
+                last[i] = part_stage[st.slot * n + i] = si;
+                break;
+            }
+            case SK_MERGE:
+                if ( !part[st.slot * n + i].parts.on ) break;
+                dep = last[i] * n + i;
+                for ( int t = 0; t < nt; t += GC_TILES ) push( SK_MERGE, st.slot * n + i, t, std::min( nt, t + GC_TILES ), dep );
+                last[i] = part_stage[st.slot * n + i] = si;
                 break;
             case SK_NEWNP:
                 // after the species' own particle pass
-                dep = ( 1 + st.slot ) * n + i;
+                dep = part_stage[st.slot * n + i] * n + i;
                 for ( int t = 0; t < nt; t += NEWNP_TILES ) push( SK_NEWNP, st.slot * n + i, t, std::min( nt, t + NEWNP_TILES ), dep );
                 break;
             case SK_COUNT:
@@ -2850,27 +3067,61 @@ int zpic_push_move_deposit_overwrite( const zpic_particles * p, const zpic_geom 
 
 int zpic_tile_sort_count( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx,
                           int ny, int periodic_x, int periodic_y, const int * extra, void * stream ) {
+    return zpic::tile_sort_count( p, tmp, s, ntiles_x, ntiles_y, nx, ny, periodic_x, periodic_y, extra, nullptr, nullptr, nullptr,
+                                  stream );
+}
+
+}  // extern "C"
+
+int zpic::tile_sort_count( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx,
+                           int ny, int periodic_x, int periodic_y, const int * extra, const PartScratch * parts,
+                           const double * tile_energy, double * energy, void * stream ) {
     if ( !p || !tmp || !s || ntiles_x < 1 || ntiles_y < 1 || nx < 1 || ny < 1 )
         return set_error( ZPIC_EINVAL, "invalid tile_sort arguments" );
     const int nt = ntiles_x * ntiles_y;
-    SortArgs a = sort_args( p, tmp, s, ntiles_x, ntiles_y, nx, ny, periodic_x, periodic_y );
+    SortArgs a = sort_args( p, tmp, s, ntiles_x, ntiles_y, nx, ny, periodic_x, periodic_y, parts );
     a.extra = extra;
     const SortArgs * tab = nullptr;
     hipStream_t st = as_stream( stream );
+    if ( nt <= SCAN_BLOCK ) {
+        const EnergyArgs e{ tile_energy, nt, energy }, * etab = nullptr;
+        hipLaunchKernelGGL( k_sort_plan, dim3( 1 ), dim3( SCAN_BLOCK ), 0, st, a, tab, e, etab );
+        ZPIC_LAUNCH_CHECK( "k_sort_plan" );
+        return ZPIC_OK;
+    }
     hipLaunchKernelGGL( k_sort_newnp, dim3( ( nt + 255 ) / 256 ), dim3( 256 ), 0, st, a, tab );
     ZPIC_LAUNCH_CHECK( "k_sort_newnp" );
     hipLaunchKernelGGL( k_sort_count, dim3( 1 ), dim3( SCAN_BLOCK ), 0, st, a, tab );
     ZPIC_LAUNCH_CHECK( "k_sort_count" );
+    return tile_energy ? zpic_sum_tiles( tile_energy, nt, energy, 0, stream ) : ZPIC_OK;
+}
+
+int zpic::part_list( const int * np, int ntiles, const PartScratch & parts, void * stream ) {
+    SortArgs a{};
+    a.S.new_np = const_cast<int *>( np );
+    a.ntiles = ntiles;
+    a.parts = parts;
+    hipLaunchKernelGGL( k_part_list, dim3( 1 ), dim3( SCAN_BLOCK ), 0, as_stream( stream ), a );
+    ZPIC_LAUNCH_CHECK( "k_part_list" );
     return ZPIC_OK;
 }
 
+extern "C" {
+
 int zpic_tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx,
                          int ny, int periodic_x, int periodic_y, int mode, void * stream ) {
+    return zpic::tile_sort_copy( p, tmp, s, ntiles_x, ntiles_y, nx, ny, periodic_x, periodic_y, mode, nullptr, stream );
+}
+
+}  // extern "C"
+
+int zpic::tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx,
+                          int ny, int periodic_x, int periodic_y, int mode, const PartScratch * parts, void * stream ) {
     if ( !p || !tmp || !s || ntiles_x < 1 || ntiles_y < 1 || nx < 1 || ny < 1 )
         return set_error( ZPIC_EINVAL, "invalid tile_sort arguments" );
     if ( mode != 0 && mode != 1 ) return set_error( ZPIC_EINVAL, "tile_sort copy mode must be 0 or 1" );
     const int nt = ntiles_x * ntiles_y;
-    const SortArgs a = sort_args( p, tmp, s, ntiles_x, ntiles_y, nx, ny, periodic_x, periodic_y );
+    const SortArgs a = sort_args( p, tmp, s, ntiles_x, ntiles_y, nx, ny, periodic_x, periodic_y, parts );
     const SortArgs * tab = nullptr;
     const int2 * map = nullptr;
     hipStream_t st = as_stream( stream );
@@ -2884,10 +3135,11 @@ int zpic_tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s
     }
     if ( a.S.stage_ix ) {
         // order-free placement from the particle pass's staging
-        const dim3 grid( ( nt + SORT_WAVES - 1 ) / SORT_WAVES );
-        hipLaunchKernelGGL( k_sort_shift, grid, dim3( SORT_WAVES * WAVE ), 0, st, a, tab, map, nt );
+        const int slices = sort_slices( nt );
+        const dim3 grid( ( nt * slices + SORT_WAVES - 1 ) / SORT_WAVES );
+        hipLaunchKernelGGL( k_sort_shift, grid, dim3( SORT_WAVES * WAVE ), 0, st, a, tab, map, nt, slices );
         ZPIC_LAUNCH_CHECK( "k_sort_shift" );
-        hipLaunchKernelGGL( k_sort_in_fast, grid, dim3( SORT_WAVES * WAVE ), 0, st, a, tab, map, nt );
+        hipLaunchKernelGGL( k_sort_in_fast, grid, dim3( SORT_WAVES * WAVE ), 0, st, a, tab, map, nt, slices );
         ZPIC_LAUNCH_CHECK( "k_sort_in_fast" );
         return ZPIC_OK;
     }
@@ -2897,6 +3149,16 @@ int zpic_tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s
     ZPIC_LAUNCH_CHECK( "k_sort_in" );
     return ZPIC_OK;
 }
+
+int zpic::push_move_deposit_parts( const zpic_particles * p, const zpic_geom * fld, const float * E, const float * B,
+                                   float * J, float alpha, float dt_dx, float dt_dy, float q, float qnx, float qny,
+                                   double * tile_energy, zpic_sort * s, int reflect, int shift_x, int set_j,
+                                   const PartScratch * parts, void * stream ) {
+    const MoveArgs m{ dt_dx, dt_dy, q, qnx, qny, reflect, shift_x, 0 };
+    return launch_particles<true, true>( p, fld, E, B, J, alpha, m, tile_energy, s, 0, stream, set_j, parts );
+}
+
+extern "C" {
 
 int zpic_tile_sort( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx,
                     int ny, int periodic_x, int periodic_y, void * stream ) {
@@ -2933,12 +3195,21 @@ struct zpic_batch_particles {
 
 int zpic_batch_particles_create( zpic_batch_particles ** out, const zpic_batch_species * items, int n,
                                  int threads_per_tile ) {
+    return zpic::batch_particles_new( out, items, n, threads_per_tile, nullptr );
+}
+
+}  // extern "C"
+
+int zpic::batch_particles_new( zpic_batch_particles ** out, const zpic_batch_species * items, int n,
+                               int threads_per_tile, const PartScratch * parts ) {
     if ( !out ) return set_error( ZPIC_EINVAL, "null output" );
     BatchParticlePlan * plan = nullptr;
-    if ( int rc = batch_particles_create( &plan, items, n, threads_per_tile ) ) return rc;
+    if ( int rc = batch_particles_create( &plan, items, n, threads_per_tile, parts ) ) return rc;
     *out = new zpic_batch_particles{ plan };
     return ZPIC_OK;
 }
+
+extern "C" {
 
 int zpic_batch_particles_advance( zpic_batch_particles * b, void * stream ) {
     if ( !b || !b->plan ) return set_error( ZPIC_EINVAL, "null batch" );
@@ -2957,12 +3228,22 @@ struct zpic_batch_step {
 
 int zpic_batch_step_create( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
                             const zpic_batch_fields_item * fields, int n, int threads_per_tile ) {
+    return zpic::batch_step_new( out, species, nslots, fields, n, threads_per_tile, nullptr );
+}
+
+}  // extern "C"
+
+int zpic::batch_step_new( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
+                          const zpic_batch_fields_item * fields, int n, int threads_per_tile,
+                          const PartScratch * parts ) {
     if ( !out ) return set_error( ZPIC_EINVAL, "null output" );
     BatchStepPlan * plan = nullptr;
-    if ( int rc = batch_step_create( &plan, species, nslots, fields, n, threads_per_tile ) ) return rc;
+    if ( int rc = batch_step_create( &plan, species, nslots, fields, n, threads_per_tile, parts ) ) return rc;
     *out = new zpic_batch_step{ plan };
     return ZPIC_OK;
 }
+
+extern "C" {
 
 int zpic_batch_step_advance( zpic_batch_step * b, void * stream ) {
     if ( !b || !b->plan ) return set_error( ZPIC_EINVAL, "null batch step" );

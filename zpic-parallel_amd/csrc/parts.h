@@ -1,0 +1,72 @@
+// Tiles taken by several workgroups in the fast-mode particle pass.
+//
+// A tile's particles are cut into parts of about `size` particles, at most
+// PART_MAX of them, one workgroup each; a part deposits into a J region of
+// its own, and k_part_merge adds the regions of a tile in part order.  Used
+// where the tiles alone do not fill the device, or one crowded tile would
+// hold up the rest (part_rule): with one workgroup per tile, a 128x128 Weibel
+// run (64 tiles, 2 x 1M particles) took 1.18 ms a step over its first
+// thousand steps, as filaments gather up to three times the mean in a tile,
+// and takes 0.20 ms; a 64x64 box of 8x8 tiles and as many particles 1.92 and
+// 0.20 ms.  The list of parts follows the tiles'
+// particle counts: the sort writes it for the next pass, and part_list()
+// where the counts came about in another way.
+#pragma once
+
+#include <algorithm>
+
+#include "zpic_amd.h"
+
+namespace zpic {
+
+constexpr int PART_SEG = 64;      // ints per tile of the segment table
+constexpr int PART_MAX_SEG = 59;  // wave segments of one tile
+constexpr int PART_MAX = 14;
+constexpr int PART_TARGET = 1024;  // parts beyond one per tile, at most
+constexpr unsigned PART_MIN = 1024;
+
+struct PartScratch {
+    int on = 0;    // 0: tiles are not cut, the rest is unused
+    int size = 0;  // particles of a part
+    int cap = 0;   // most parts of all tiles: ntiles + PART_TARGET
+    int * seg = nullptr;    // [PART_SEG * ntiles] segment tables
+    int * item = nullptr;   // [2 * cap] the parts: tile, part | parts of the tile << 8
+    int * total = nullptr;  // [1] their number
+    int * npt = nullptr;    // [9 * cap] direction counts of each part
+    double * energy = nullptr;  // [cap]
+    float * J = nullptr;        // [3 * tile_vol * cap]
+};
+
+// Worth its two launches (the merge, about 5 us, and the list) where one
+// crowded tile bounds the pass: up to 1024 tiles, one workgroup each on the
+// device at once.
+inline bool part_rule( int ntiles ) { return ntiles <= 1024; }
+// Particles of a part for a buffer of max_part: no more than PART_TARGET parts
+// beyond one per tile, and no fewer than PART_MIN particles, which take a
+// workgroup about as long as its staging and its J region.  (512 and 2048
+// parts measured within 3 % on these runs, 4096 of at least 256 particles up
+// to 15 % slower on a 512x512 grid.)
+inline int part_size( unsigned max_part ) {
+    return (int) std::max( PART_MIN, ( max_part / PART_TARGET + 64 ) & ~63u );
+}
+
+// The list of parts for the tiles' particle counts np[ntiles].
+int part_list( const int * np, int ntiles, const PartScratch & parts, void * stream );
+// The stage and batch entry points of zpic_amd.h with such scratch (one per
+// species of a batch, as its items; null: no tile is cut).  The sort's count
+// also sums the tiles' push energies (fast mode) where they are given.
+int push_move_deposit_parts( const zpic_particles * p, const zpic_geom * fld, const float * E, const float * B,
+                             float * J, float alpha, float dt_dx, float dt_dy, float q, float qnx, float qny,
+                             double * tile_energy, zpic_sort * s, int reflect, int shift_x, int set_j,
+                             const PartScratch * parts, void * stream );
+int tile_sort_count( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx, int ny,
+                     int periodic_x, int periodic_y, const int * extra, const PartScratch * parts,
+                     const double * tile_energy, double * energy, void * stream );
+int tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx, int ny,
+                    int periodic_x, int periodic_y, int mode, const PartScratch * parts, void * stream );
+int batch_particles_new( zpic_batch_particles ** out, const zpic_batch_species * items, int n, int threads_per_tile,
+                         const PartScratch * parts );
+int batch_step_new( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
+                    const zpic_batch_fields_item * fields, int n, int threads_per_tile, const PartScratch * parts );
+
+}  // namespace zpic

@@ -17,6 +17,7 @@
 #include <string>
 #include <vector>
 
+#include "parts.h"
 #include "zdf.hpp"
 #include "zpic_amd.h"
 
@@ -389,6 +390,12 @@ class ParticleSort {
     // leaver list sized for max_part particles (grown with the particle buffer)
     void grow( uint32_t max_part );
     uint32_t idx_size;
+    // scratch of tiles taken in parts by the particle pass (tile_vol: elements
+    // of a tile of the current), and whether the last pass took them so
+    zpic::PartScratch parts;
+    bool in_parts;
+    bool listed;  // the list of parts fits the particle counts
+    void init_parts( uint32_t max_part, int tile_vol );
     ParticleSort( const ParticleSort & ) = delete;
     ParticleSort & operator=( const ParticleSort & ) = delete;
 };
@@ -669,7 +676,7 @@ class Species {
     // for extra[t] (device array) more particles after each tile; max_extra
     // bounds their sum.  Takes the copy_sorted path, growing the buffers,
     // when the total exceeds the particle buffer, as the reference does.
-    void tile_sort( const int * extra, uint64_t max_extra );
+    void tile_sort( const int * extra, uint64_t max_extra, bool energy = false );
     virtual void advance( EMF const & emf, Current & current );
     // advance() (window: advance_mov_window()) recording `after_push` (may be
     // null) between the particle pass and the sort
@@ -748,6 +755,10 @@ class Species {
 
     // Arguments of this species for a batched advance with the given fields
     zpic_batch_species batch_item( EMF const & emf, Current & current ) const;
+    zpic::PartScratch part_scratch() const { return sort->parts; }
+    // The list of parts, where the particle counts changed by other means than
+    // a sort that wrote it.
+    void list_parts();
     // device particle buffers (they change when the buffers are swapped)
     void buffers( std::vector<const void *> & out ) const {
         out.push_back( particles->ix );
