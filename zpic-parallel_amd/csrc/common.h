@@ -36,6 +36,10 @@ hipStream_t default_stream_or_null();
 // The stream of a stage entry point: the caller's, or the library's for NULL.
 inline hipStream_t as_stream( void * s ) { return s ? (hipStream_t) s : default_stream_or_null(); }
 
+// zpic_current_update on a grid that need not be periodic (no walls).
+int current_update( const float * dep, float * J, const zpic_geom * g, int passes, const float * coef, int px, int py,
+                    void * stream );
+
 }  // namespace zpic
 
 #define ZPIC_HIP_TRY( call )                                               \

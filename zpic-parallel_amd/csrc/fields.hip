@@ -79,17 +79,24 @@ __global__ void __launch_bounds__( TILE_BLOCK ) k_kernel3( K3Args args, const K3
     kernel3_tile( args, t, A );
 }
 
-// 128 threads and CUR_TILES tiles per workgroup: 104-108 us on the 2048^2
-// grid, against 113 us with one tile per workgroup and 115 / 139 us with
-// 256 / 512 threads (the fixed costs of a workgroup amortised; the same
-// for the Yee update and the guard copy gained nothing or lost)
+// Up to CUR_FEW tiles, a workgroup of 256 threads for each, so that the tiles
+// still reach every compute unit; more tiles, two per workgroup of 128
+// threads, whose fixed costs then halve.  Microseconds a call, tiles of the
+// given cells and passes (in brackets the form that looked the neighbours up
+// for each element, ran the passes in LDS and took four tiles per 128
+// threads): 8x8 of 16x16, 0: 5 (26); 33x45 of 32x16, 5: 18 (123); 256x32 of
+// 16x16, 5: 54 (105); 128x128 of 16x16, 1: 65 (78).  On the largest, 256
+// threads and one tile take 72, 128 threads and one tile 70.
+constexpr int CUR_FEW = 4096;
+constexpr int CUR_BLOCK_FEW = 256;
 constexpr int CUR_BLOCK = 128;
-constexpr int CUR_TILES = 4;
-__global__ void __launch_bounds__( CUR_BLOCK ) k_current( CurArgs a ) {
+constexpr int CUR_TILES = 2;
+template <int NP>
+__global__ void __launch_bounds__( CUR_BLOCK_FEW ) k_current( CurArgs a ) {
     extern __shared__ float sm[];
     for ( int t = blockIdx.x; t < a.g.ntx * a.g.nty; t += gridDim.x ) {
         if ( t != (int) blockIdx.x ) __syncthreads();  // LDS of the previous tile read out
-        current_tile( a, t, sm );
+        current_tile<NP>( a, t, sm );
     }
 }
 
@@ -951,8 +958,15 @@ int zpic_current_advance( float * J, const zpic_geom * g, int kind, int dir, int
     return ZPIC_OK;
 }
 
-int zpic_current_update( const float * dep, float * J, const zpic_geom * gg, int passes, const float * coef,
+int zpic_current_update( const float * dep, float * J, const zpic_geom * g, int passes, const float * coef,
                          void * stream ) {
+    return zpic::current_update( dep, J, g, passes, coef, 1, 1, stream );
+}
+
+}  // extern "C"
+
+int zpic::current_update( const float * dep, float * J, const zpic_geom * gg, int passes, const float * coef, int px,
+                          int py, void * stream ) {
     if ( int rc = check( gg ) ) return rc;
     if ( !dep || !J || ( passes > 0 && !coef ) ) return set_error( ZPIC_EINVAL, "null argument" );
     if ( dep == J ) return set_error( ZPIC_EINVAL, "current update: deposit and current buffers must differ" );
@@ -964,11 +978,13 @@ int zpic_current_update( const float * dep, float * J, const zpic_geom * gg, int
         return set_error( ZPIC_EINVAL, "current update: tiles narrower than both guard bands plus the filter passes" );
     if ( 3 * ( g.vol - g.ext_x * g.ext_y ) > CUR_BLOCK ) return set_error( ZPIC_EINVAL, "current update: tile padding" );
     const size_t lds = current_lds_bytes( g, passes );
-    if ( lds > 65536 ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
+    if ( sizeof( float ) * 6 * ( g.ext_x + 2 * passes ) * g.ext_y > 65536 ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
     CurArgs a{};
     a.dep = dep;
     a.J = J;
     a.g = g;
+    a.px = px ? 1 : 0;
+    a.py = py ? 1 : 0;
     a.passes = passes;
     for ( int p = 0; p < passes; p++ ) {
         a.a[p] = coef[3 * p];
@@ -976,10 +992,23 @@ int zpic_current_update( const float * dep, float * J, const zpic_geom * gg, int
         a.c[p] = coef[3 * p + 2];
     }
     hipStream_t st = as_stream( stream );
-    hipLaunchKernelGGL( k_current, dim3( ( g.ntx * g.nty + CUR_TILES - 1 ) / CUR_TILES ), dim3( CUR_BLOCK ), lds, st, a );
+    const int nt = g.ntx * g.nty;
+    const bool few = nt <= CUR_FEW;
+    const dim3 grid( few ? nt : ( nt + CUR_TILES - 1 ) / CUR_TILES ), block( few ? CUR_BLOCK_FEW : CUR_BLOCK );
+    switch ( passes ) {
+    case 0: hipLaunchKernelGGL( k_current<0>, grid, block, lds, st, a ); break;
+    case 1: hipLaunchKernelGGL( k_current<1>, grid, block, lds, st, a ); break;
+    case 2: hipLaunchKernelGGL( k_current<2>, grid, block, lds, st, a ); break;
+    case 3: hipLaunchKernelGGL( k_current<3>, grid, block, lds, st, a ); break;
+    case 4: hipLaunchKernelGGL( k_current<4>, grid, block, lds, st, a ); break;
+    case 5: hipLaunchKernelGGL( k_current<5>, grid, block, lds, st, a ); break;
+    default: hipLaunchKernelGGL( k_current<-1>, grid, block, lds, st, a ); break;
+    }
     ZPIC_LAUNCH_CHECK( "k_current" );
     return ZPIC_OK;
 }
+
+extern "C" {
 
 int zpic_yee( float * E, float * B, const float * J, const zpic_geom * gg, float dtdx, float dtdy, float dt, int px,
               int py, void * stream ) {

@@ -297,22 +297,28 @@ __device__ inline void yee_tile( const YeeArgs & a, const int t, float * sm ) {
     }
 }
 
-// Current::advance on a grid periodic along x and y (current.cpp:226-246:
-// add_from_gc, copy_to_gc, then the filter's kernel3_x passes, each followed
-// by copy_to_gc_x, grid.h:367-444, 253-340, 495-545) for tile t in one pass,
+// Current::advance without walls (current.cpp:226-246: add_from_gc,
+// copy_to_gc, then the filter's kernel3_x passes, each followed by
+// copy_to_gc_x, grid.h:367-444, 253-340, 495-545) for tile t in one pass,
 // from the deposit buffer `dep` into `J` (distinct buffers: neighbours read
-// `dep` while J is written).  After that sequence on a periodic grid every
-// element of a tile's region, guards included, holds the value of the global
-// cell it stands for, so tile t computes its whole region itself:
+// `dep` while J is written).  After that sequence every element of a tile's
+// region that stands for a cell of the grid, guards included, holds that
+// cell's value, so tile t computes its whole region itself:
 //  * the summed current of every cell in columns [-gl - P, nx + gu + P) and
 //    rows [-gl, ny + gu) (tile-local), with the additions of the x pass
 //    (own value, + lower neighbour's upper guard, + upper neighbour's lower
 //    guard) then the y pass (+ the y neighbours' guard rows as their own x
 //    pass left them), in that order;
-//  * P filter passes in LDS, A[i-1]*a + A[i]*b + A[i+1]*c, the valid columns
-//    shrinking by one on each side per pass;
+//  * P filter passes, A[i-1]*a + A[i]*b + A[i+1]*c: up to CUR_REG_PASSES in
+//    registers, a thread taking CUR_RUN neighbouring columns of a row of one
+//    component and the P columns on either side (the outer values computed
+//    twice cost less than an LDS round trip and a barrier per pass); more in
+//    LDS, pass by pass, the valid columns shrinking by one on each side;
 //  * the region [-gl, nx + gu) x [-gl, ny + gu) written, and the tile's
 //    padding elements copied from `dep` (the sequence never touches them).
+// At the end of a non-periodic axis the guards stand for no cell: guard
+// columns keep their deposit (with the y pass's additions) through the
+// filter, guard rows theirs with the x pass's, and the filter runs on them.
 // With nx >= gl + gu + P and ny >= gl + gu every value a cell of the region
 // needs lies in tile t's 3x3 neighbourhood.  LDS: current_lds_bytes.
 constexpr int CUR_MAX_PASSES = 16;
@@ -320,12 +326,25 @@ struct CurArgs {
     const float * dep;
     float * J;
     G g;
+    int px, py;
     int passes;
     float a[CUR_MAX_PASSES], b[CUR_MAX_PASSES], c[CUR_MAX_PASSES];
 };
 
+constexpr int CUR_REG_PASSES = 5;
+constexpr int CUR_RUN = 5;
+
+// The summed current and, for a filter, its result; odd row strides in the
+// register form, whose lanes walk down the rows.
+__host__ __device__ inline int current_lds_floats( const G & g, int passes ) {
+    const int W = g.nx + g.gl + g.gu + 2 * passes;
+    const int row = passes > CUR_REG_PASSES ? 2 * W : passes > 0 ? ( W | 1 ) + ( g.ext_x | 1 ) : W;
+    return ( 3 * row * g.ext_y + 1 ) & ~1;
+}
+// and the tables of current_tile
 inline size_t current_lds_bytes( const G & g, int passes ) {
-    return sizeof( float ) * 2 * 3 * (size_t) ( g.nx + g.gl + g.gu + 2 * passes ) * g.ext_y;
+    return sizeof( float ) * current_lds_floats( g, passes ) + sizeof( long long ) * 2 * g.ext_y +
+           sizeof( int ) * 2 * ( g.nx + g.gl + g.gu + 2 * passes );
 }
 
 // Loop over the n = rows x len elements of a 2-D range, row-major, thread
@@ -346,72 +365,137 @@ __device__ inline void for_2d( int rows, int len, F && f ) {
     }
 }
 
+// The P passes of one run of columns held in v (v[P] is the first output
+// column's value on entry, v[0] on return); columns outside [lo, hi) of v
+// keep their value if EDGE.
+template <int P, bool EDGE>
+__device__ inline void filter_run( float ( &v )[CUR_RUN + 2 * P], const CurArgs & a, int lo, int hi ) {
+#pragma unroll
+    for ( int p = 0; p < P; p++ ) {
+        const float ca = a.a[p], cb = a.b[p], cc = a.c[p];
+#pragma unroll
+        for ( int i = 0; i < CUR_RUN + 2 * ( P - 1 - p ); i++ ) {
+            // v[i] holds column i + p of the run
+            const float f = v[i] * ca + v[i + 1] * cb + v[i + 2] * cc;
+            v[i] = ( EDGE && ( i + p + 1 < lo || i + p + 1 >= hi ) ) ? v[i + 1] : f;
+        }
+    }
+}
+
+// NP: the filter's passes, or -1 for more than CUR_REG_PASSES.
+template <int NP>
 __device__ inline void current_tile( const CurArgs & a, const int t, float * sm ) {
     const G g = a.g;
-    const int P = a.passes;
+    const int P = NP >= 0 ? NP : a.passes;
     const int E = g.ext_x;
-    const int XW = g.nx + g.gl + g.gu + 2 * P, plane = XW * g.ext_y;
+    const int XW = g.nx + g.gl + g.gu + 2 * P;
+    const int XS = NP > 0 ? XW | 1 : XW, plane = XS * g.ext_y;
     float * A = sm;
     float * Bf = sm + 3 * plane;
     const gptr<const float> dep = gbl( a.dep );
-    // first float of each deposit region of the 3x3 neighbourhood, index
-    // (dy + 1) * 3 + dx + 1
-    __shared__ long long s_nb[9];
-    if ( threadIdx.x < 9 ) {
-        const int k = threadIdx.x;
-        s_nb[k] = (long long) nbr( t % g.ntx, t / g.ntx, k % 3 - 1, k / 3 - 1, g, 1, 1 ) * g.vol * 3;
+    const int tx = t % g.ntx, ty = t / g.ntx;
+    const bool left = a.px || tx > 0, right = a.px || tx < g.ntx - 1;  // x neighbours exist
+    const bool down = a.py || ty > 0, up = a.py || ty < g.nty - 1;
+    // The deposits that make up an element: one or two columns (the cell's
+    // and, next to a tile edge, the x neighbour's guard that holds a share of
+    // it) times one or two rows.  Tables of their offsets in floats, a
+    // column's tile and place plus a row's; -1: none.
+    long long * const rowt = reinterpret_cast<long long *>( sm + current_lds_floats( g, P ) );  // [ext_y][2]
+    int * const colt = reinterpret_cast<int *>( rowt + 2 * g.ext_y );                          // [XW][2]
+    for ( int e = threadIdx.x; e < XW + g.ext_y; e += blockDim.x ) {
+        const bool row = e >= XW;
+        const int xx = row ? e - XW - g.gl : e - g.gl - P;
+        const int n = row ? g.ny : g.nx, nt = row ? g.nty : g.ntx, t0 = row ? ty : tx;
+        const bool lo = row ? down : left, hi = row ? up : right;
+        const int d = xx < 0 ? ( lo ? -1 : 0 ) : ( xx >= n && hi ? 1 : 0 );
+        const int i = xx - d * n;
+        auto tile = [&]( int k ) { return ( t0 + k + nt ) % nt; };
+        const long long per_tile = 3ll * g.vol * ( row ? g.ntx : 1 ), per_el = 3 * ( row ? E : 1 );
+        auto at = [&]( int k, int x ) { return tile( k ) * per_tile + ( x + g.gl ) * per_el; };
+        long long first = -1, second = -1;
+        if ( i >= -g.gl && i < n + g.gu ) {  // past a non-periodic end's guards there is nothing
+            first = at( d, i );
+            if ( i >= 0 && i < g.gu && ( lo || d > 0 ) ) second = at( d - 1, n + i );
+            if ( i >= n - g.gl && i < n && ( hi || d < 0 ) ) second = at( d + 1, i - n );
+        }
+        if ( row ) {
+            rowt[2 * ( e - XW )] = first;
+            rowt[2 * ( e - XW ) + 1] = second;
+        } else {
+            colt[2 * e] = (int) first;
+            colt[2 * e + 1] = (int) second;
+        }
     }
     __syncthreads();
-    // deposit of neighbour k at tile-local (x, y), component c
-    auto raw = [&]( int k, int x, int y, int c ) { return dep[s_nb[k] + ( ( x + g.gl ) + ( y + g.gl ) * E ) * 3 + c]; };
-    // neighbour k (at dx, dy) at interior column i, any row y, after the x
-    // pass; its x neighbours are k - 1 and k + 1 (inside the 3x3 block
-    // whenever the terms apply)
-    auto xsum = [&]( int k, int i, int y, int c ) {
-        float v = raw( k, i, y, c );
-        if ( i < g.gu ) v += raw( k - 1, g.nx + i, y, c );
-        if ( i >= g.nx - g.gl ) v += raw( k + 1, i - g.nx, y, c );
-        return v;
-    };
-    // summed current on the region, SoA planes A[c][row][col]
+    // summed current on the region, SoA planes A[c][row][col]: the x pass's
+    // addition, then the y pass's of sums that their own x pass made
     for_2d( g.ext_y, 3 * XW, [&]( int row, int q ) {
         const int col = q / 3, c = q - 3 * col;
-        const int xx = col - g.gl - P, yy = row - g.gl;
-        const int dx = xx < 0 ? -1 : ( xx >= g.nx ? 1 : 0 );
-        const int dy = yy < 0 ? -1 : ( yy >= g.ny ? 1 : 0 );
-        const int i = xx - dx * g.nx, j = yy - dy * g.ny;
-        const int k = ( dy + 1 ) * 3 + dx + 1;
-        float s = xsum( k, i, j, c );
-        if ( j < g.gu ) s += xsum( k - 3, i, g.ny + j, c );
-        if ( j >= g.ny - g.gl ) s += xsum( k + 3, i, j - g.ny, c );
-        A[c * plane + row * XW + col] = s;
-    } );
-    for ( int p = 0; p < P; p++ ) {
-        __syncthreads();
-        const float ca = a.a[p], cb = a.b[p], cc = a.c[p];
-        float * const In = A;
-        float * const Out = Bf;
-        for_2d( 3 * g.ext_y, XW, [&]( int r, int x ) {
-            if ( x > p && x < XW - 1 - p ) {
-                const int k = r * XW + x;
-                Out[k] = In[k - 1] * ca + In[k] * cb + In[k + 1] * cc;
+        const int c1 = colt[2 * col], c2 = colt[2 * col + 1];
+        const long long r2 = rowt[2 * row + 1];
+        float s = 0.0f;
+        if ( c1 >= 0 ) {
+            const gptr<const float> p = dep + rowt[2 * row] + c;
+            s = p[c1];
+            if ( c2 >= 0 ) s += p[c2];
+            if ( r2 >= 0 ) {
+                const gptr<const float> p2 = dep + r2 + c;
+                float s2 = p2[c1];
+                if ( c2 >= 0 ) s2 += p2[c2];
+                s += s2;
             }
+        }
+        A[c * plane + row * XS + col] = s;
+    } );
+    // columns the filter moves: all but the guards at a non-periodic end
+    const int x_lo = left ? 0 : g.gl + P, x_hi = right ? XW : g.gl + P + g.nx;
+    int rs = XS, rplane = plane, shift = P;  // the result's row stride, plane and first column
+    if constexpr ( NP > 0 ) {
+        __syncthreads();
+        const int ES = E | 1, rows = 3 * g.ext_y, runs = ( E + CUR_RUN - 1 ) / CUR_RUN;
+        const bool edge = !left || !right;
+        for_2d( runs, rows, [&]( int run, int r ) {
+            const int col = run * CUR_RUN;  // output column of the run's first value, window column col + P
+            float v[CUR_RUN + 2 * NP];
+#pragma unroll
+            for ( int i = 0; i < CUR_RUN + 2 * NP; i++ ) v[i] = A[r * XS + min( col + i, XW - 1 )];
+            if ( edge ) filter_run<NP, true>( v, a, x_lo - col, x_hi - col );
+            else filter_run<NP, false>( v, a, 0, 0 );
+#pragma unroll
+            for ( int i = 0; i < CUR_RUN; i++ )
+                if ( col + i < E ) Bf[r * ES + col + i] = v[i];
         } );
-        A = Out;
-        Bf = In;
+        A = Bf;
+        rs = ES;
+        rplane = ES * g.ext_y;
+        shift = 0;
+    } else {
+        for ( int p = 0; p < P; p++ ) {
+            __syncthreads();
+            const float ca = a.a[p], cb = a.b[p], cc = a.c[p];
+            float * const In = A;
+            float * const Out = Bf;
+            for_2d( 3 * g.ext_y, XW, [&]( int r, int x ) {
+                const int k = r * XW + x;
+                if ( x < x_lo || x >= x_hi ) Out[k] = In[k];
+                else if ( x > p && x < XW - 1 - p ) Out[k] = In[k - 1] * ca + In[k] * cb + In[k + 1] * cc;
+            } );
+            A = Out;
+            Bf = In;
+        }
     }
     __syncthreads();
     const gptr<float> Jt = gbl( a.J ) + (size_t) t * g.vol * 3;
     float * const R = A;
     for_2d( g.ext_y, 3 * E, [&]( int row, int q ) {
         const int col = q / 3, c = q - 3 * col;
-        Jt[row * 3 * E + q] = R[c * plane + row * XW + col + P];
+        Jt[row * 3 * E + q] = R[c * rplane + row * rs + col + shift];
     } );
     // padding
     const int npad = 3 * ( g.vol - E * g.ext_y );
     if ( (int) threadIdx.x < npad ) {
         const size_t k = (size_t) 3 * E * g.ext_y + threadIdx.x;
-        Jt[k] = dep[s_nb[4] + k];
+        Jt[k] = dep[(size_t) t * g.vol * 3 + k];
     }
 }
 

@@ -446,8 +446,9 @@ void Current::set_bc( current::bc_type new_bc ) {
 
 bool Current::one_pass_ok( std::vector<float> & coef ) const {
     coef.clear();
-    const int2 p = J->get_periodic();
-    if ( !p.x || !p.y ) return false;
+    if ( bc.x.lower > current::bc::periodic || bc.x.upper > current::bc::periodic ||
+         bc.y.lower > current::bc::periodic || bc.y.upper > current::bc::periodic )
+        return false;  // walls change the current between the guard copy and the filter
     if ( filter->kind() == 1 || filter->kind() == 2 ) {
         const auto * f = dynamic_cast<const Filter::Binomial *>( filter );
         if ( !f || f->get_dir() != coord::x ) return false;
@@ -472,7 +473,8 @@ void Current::advance() {
             Jalt->name = J->name;
         }
         zpic_geom g = J->geom();
-        check( zpic_current_update( J->fbuf(), Jalt->fbuf(), &g, (int) coef.size() / 3, coef.data(), stream() ) );
+        const int2 p = J->get_periodic();
+        check( current_update( J->fbuf(), Jalt->fbuf(), &g, (int) coef.size() / 3, coef.data(), p.x, p.y, stream() ) );
         std::swap( J->d_buffer, Jalt->d_buffer );
         iter++;
         if ( moving_window.needs_move( iter * dt ) ) moving_window.advance();
@@ -850,13 +852,12 @@ void Species::advance_mov_window( EMF const & emf, Current & current ) { step( e
 
 // Fast mode with the order-free sort: the particle pass compacts stayers and
 // stages leaver records in the sort buffer (`tmp`), and the sort places them
-// from there.  Not on moving-window steps: their sort may have to take the
-// copy_sorted path, which reads the particles in place, and where it need not
-// (the injection cannot outgrow the buffer) the reference order measured
-// faster on the LWFA set-up (0.411 against 0.432 ms per step), whose tiles
-// hold few particles and all of whose particles move one cell on such steps.
+// from there.  Not on a step where the window moves and the injected
+// particles may outgrow the buffer: its sort may have to take the copy_sorted
+// path, which reads the particles in place.
 void Species::set_staging( zpic_sort & s, bool window ) const {
-    const bool staged = !deterministic && !window && zpic_get_sort_order() == 0;
+    const bool room = np_bound + max_injected() <= particles->max_part;
+    const bool staged = !deterministic && ( !window || room ) && zpic_get_sort_order() == 0;
     s.stage_ix = staged ? reinterpret_cast<int *>( tmp->ix ) : nullptr;
     s.stage_x = staged ? reinterpret_cast<float *>( tmp->x ) : nullptr;
     s.stage_u = staged ? reinterpret_cast<float *>( tmp->u ) : nullptr;
@@ -893,7 +894,7 @@ void Species::finish_step( bool shift ) {
         const uint2 gd = particles->dims;
         const int range[4] = { (int) gd.x - 1, (int) gd.x - 1, 0, (int) gd.y - 1 };
         np_inject( range, d_np_inj );
-        tile_sort( d_np_inj, (uint64_t) gd.y * ppc.x * ppc.y, !deterministic );
+        tile_sort( d_np_inj, max_injected(), !deterministic );
         inject( range );
         moving_window.advance();
     } else {

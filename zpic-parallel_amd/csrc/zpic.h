@@ -706,6 +706,8 @@ class Species {
     // energy sum.
     void particle_pass( EMF const & emf, Current & current, bool shift, bool set_j = false );
     void set_staging( zpic_sort & s, bool window = false ) const;
+    // most particles that a move of the window injects
+    uint64_t max_injected() const { return (uint64_t) particles->dims.y * ppc.x * ppc.y; }
     void finish_step( bool shift );
     // Whether this step shifts the particles (the window moves), for a step
     // of advance_mov_window (window) or advance (not window)
