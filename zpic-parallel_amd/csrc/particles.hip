@@ -1,13 +1,14 @@
 // Particle stages of the em2d step on gfx950: field interpolation + Boris
 // push, split-segment charge-conserving current deposit, and the tile sort.
 //
-// One workgroup per tile.  The tile's E and B (with guard cells) are staged in
-// LDS as six float planes.  Each wavefront accumulates its particles' current
-// in its own three J planes in LDS with plain read-add-writes, made
-// conflict-free by a per-round owner election (LDS float atomics run at about
-// one lane per clock on this part); the waves' planes are summed and flushed
-// once, with plain adds, into the tile's own region of the global J grid (each
-// tile owns its guard cells, so the flush needs no global atomics).
+// One workgroup per tile (or part of a tile).  The tile's E and B (with guard
+// cells) are staged in LDS as six float planes, and its current is summed in
+// LDS in 64-bit fixed point with integer atomics, shared by the workgroup's
+// waves: on this part LDS float atomics run at about three clocks per lane,
+// 64-bit integer ones at least twelve times as fast, and a sum of integers
+// does not depend on its order.  It is scaled and added once into the tile's
+// own region of the global J grid (each tile owns its guard cells, so that
+// needs no global atomics).
 //
 // Arithmetic is the reference's, operation for operation: no contraction
 // (built with -ffp-contract=off), fmaf exactly where the reference calls
@@ -245,16 +246,18 @@ __device__ inline void segment_current( const Seg & s, float qnx, float qny, flo
     v[7] = q * ( A1x * A1y + B1x * B1y + ( A1x * B1y - B1x * A1y ) / 2.0f );
 }
 
-// The same eight contributions with fused multiply-adds, for the fast mode
-// (whose J is compared to a tolerance: the deposit order differs anyway):
+// The same eight contributions with fused multiply-adds and without the
+// charge factors (qvz: half the velocity along z over c), for the fast mode
+// (whose J is compared to a tolerance: the deposit's sums differ anyway):
 // wy0 = (A0y + B0y) / 2 = 1/2 - (a.y + b.y) / 2, wy1 = 1/2 + (a.y + b.y) / 2,
 // and Jz = q (Ax (Ay + By / 2) + Bx (By - Ay / 2)), the reference's
-// Ax Ay + Bx By + (Ax By - Bx Ay) / 2 regrouped: 40 instead of 58 operations.
-__device__ inline void segment_current_fma( const Seg & s, float qnx, float qny, float v[8] ) {
+// Ax Ay + Bx By + (Ax By - Bx Ay) / 2 regrouped.  False if one of them is
+// not a number or large.
+__device__ inline bool segment_current_fma( const Seg & s, float v[8] ) {
     const float A0x = 0.5f - s.a.x, A1x = 0.5f + s.a.x, B0x = 0.5f - s.b.x, B1x = 0.5f + s.b.x;
     const float A0y = 0.5f - s.a.y, A1y = 0.5f + s.a.y, B0y = 0.5f - s.b.y, B1y = 0.5f + s.b.y;
-    const float jx = qnx * ( s.b.x - s.a.x );
-    const float jy = qny * ( s.b.y - s.a.y );
+    const float jx = s.b.x - s.a.x;
+    const float jy = s.b.y - s.a.y;
     const float mx = 0.5f * ( s.a.x + s.b.x ), my = 0.5f * ( s.a.y + s.b.y );
     v[0] = jx * ( 0.5f - my );
     v[5] = jx * ( 0.5f + my );
@@ -267,12 +270,14 @@ __device__ inline void segment_current_fma( const Seg & s, float qnx, float qny,
     v[4] = q * fmaf( A1x, p0, B1x * r0 );
     v[6] = q * fmaf( A0x, p1, B0x * r1 );
     v[7] = q * fmaf( A1x, p1, B1x * r1 );
+    // (ends inside the cell and |q| <= 1/2: 2.5; up to 3.5 no contribution
+    // reaches 8, and the conversion holds 32)
+    return fabsf( s.a.x ) + fabsf( s.b.x ) + fabsf( s.a.y ) + fabsf( s.b.y ) + fabsf( q ) < 3.5f;
 }
 
 // LDS (address space 3) element types: volatile accesses through generic
 // pointers would be lowered to flat instructions.
 typedef __attribute__( ( address_space( 3 ) ) ) float lds_f32;
-typedef __attribute__( ( address_space( 3 ) ) ) unsigned char lds_u8;
 
 // Read-add-write of the 8 contributions.  The accesses are volatile so that
 // they are issued in program order: another lane's contribution to the same
@@ -291,54 +296,55 @@ __device__ inline void add_current( volatile lds_f32 * Jx, volatile lds_f32 * Jy
     Jz[k + ys + 1] = Jz[k + ys + 1] + v[7];
 }
 
-// Read-add-write of the 8 contributions of lanes that own distinct cells, in
-// four batches by node offset (0, +1, +ys, +ys+1): inside a batch the lanes'
-// addresses are distinct, so each batch issues its reads together; a later
-// batch may touch what an earlier one wrote (Jx(k+ys) of one cell is Jx(k)
-// of the cell above) and, the accesses being volatile and LDS in order per
-// wave, sees those writes.
-__device__ inline void add_current_batched( volatile lds_f32 * Jx, volatile lds_f32 * Jy, volatile lds_f32 * Jz,
-                                            int k, int ys, const float v[8] ) {
-    {
-        const float a = Jx[k], b = Jy[k], c = Jz[k];
-        Jx[k] = a + v[0];
-        Jy[k] = b + v[1];
-        Jz[k] = c + v[2];
-    }
-    {
-        const float a = Jy[k + 1], b = Jz[k + 1];
-        Jy[k + 1] = a + v[3];
-        Jz[k + 1] = b + v[4];
-    }
-    {
-        const float a = Jx[k + ys], b = Jz[k + ys];
-        Jx[k + ys] = a + v[5];
-        Jz[k + ys] = b + v[6];
-    }
-    Jz[k + ys + 1] = Jz[k + ys + 1] + v[7];
+// The fast mode's current in LDS: 64-bit fixed point, 2^bits to the unit, for
+// contributions without their charge factors (a path's displacement in a
+// cell times its weights, at most 1; for z the velocity over c).  With `bits`
+// the np particles of a workgroup cannot overflow an element (FIX_HEADROOM
+// bits are left for a path's up to three segments and for weights of
+// positions a little outside their cell), and a contribution is off by at
+// most 2^-47 of the unit up to 2047 particles and 2^-43 at 16384: far less
+// than the rounding of its own FP32 arithmetic, and the sum adds nothing.
+typedef unsigned long long u64;
+typedef __attribute__( ( address_space( 3 ) ) ) u64 lds_u64;
+constexpr int FIX_HEADROOM = 5, FIX_MAX_BITS = 46;
+
+struct Fixed {
+    double magic;   // 1.5 * 2^(52 - bits): adding it leaves value * 2^bits in the low mantissa bits
+    unsigned hi;    // its upper word (the lower one is 0)
+    double unit;    // 2^-bits
+};
+__device__ inline Fixed fixed_point( int np ) {
+    const int bits = min( FIX_MAX_BITS, 62 - FIX_HEADROOM - ( 32 - __clz( np ) ) );
+    Fixed f;
+    f.hi = ( (unsigned) ( 1023 + 52 - bits ) << 20 ) | 0x80000u;
+    f.magic = __hiloint2double( (int) f.hi, 0 );
+    f.unit = __hiloint2double( ( 1023 - bits ) << 20, 0 );
+    return f;
+}
+__device__ inline void fixed_add( lds_u64 * p, float v, const Fixed & f ) {
+    u64 b = (u64) __double_as_longlong( (double) v + f.magic );
+    b -= (u64) f.hi << 32;
+    __hip_atomic_fetch_add( p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
 }
 
-// Fast-mode deposit of one segment per pending lane into the wave's private J
-// planes, without atomics: each round, every pending lane writes its lane id
-// into the tag byte of its cell and reads it back; the lane whose id survived
-// owns the cell for this round, so the owners of a round hold distinct cells
-// and their read-add-writes cannot collide.  Rounds repeat while lanes are
-// pending (as many rounds as the most repeated cell in the wave).
-__device__ inline void deposit_elected( bool pend, const Seg & s, float qnx, float qny, volatile lds_f32 * Jx,
-                                        volatile lds_f32 * Jy, volatile lds_f32 * Jz, volatile lds_u8 * tag, int ys,
-                                        unsigned lane ) {
-    // computed on every lane (SIMD lanes cost the same masked or not); used
-    // only by pending ones
+// Fast-mode deposit of one segment into J, element (node, component).
+// Returns false for a segment that is not a number or out of the fixed
+// point's range (a position far outside its cell), which is not deposited:
+// the tile's current is then not a number.
+__device__ inline bool deposit_fixed( const Seg & s, lds_u64 * J, int ys, const Fixed & f ) {
     float v[8];
-    segment_current_fma( s, qnx, qny, v );
-    const int k = s.c.x + __mul24( ys, s.c.y );
-    while ( __ballot( pend ) ) {
-        if ( pend ) tag[k] = (unsigned char) lane;
-        if ( pend && tag[k] == (unsigned char) lane ) {
-            add_current_batched( Jx, Jy, Jz, k, ys, v );
-            pend = false;
-        }
-    }
+    if ( !segment_current_fma( s, v ) ) return false;
+    lds_u64 * const p = J + 3 * ( s.c.x + __mul24( ys, s.c.y ) );
+    lds_u64 * const q = p + 3 * ys;
+    fixed_add( p, v[0], f );
+    fixed_add( p + 1, v[1], f );
+    fixed_add( p + 2, v[2], f );
+    fixed_add( p + 4, v[3], f );
+    fixed_add( p + 5, v[4], f );
+    fixed_add( q, v[5], f );
+    fixed_add( q + 2, v[6], f );
+    fixed_add( q + 5, v[7], f );
+    return true;
 }
 
 struct MoveArgs {
@@ -379,10 +385,10 @@ __device__ inline bool reflect_walls( int refl, int tx, int ty, int ntx, int nty
 // stages its leavers at the chunk's first positions.  seg[16 t + w] keeps
 // the count of each wave's leavers, seg[16 t + 15] the chunk.
 //
-// LDS: E and B planes (6*vol floats, PUSH), then W private J plane triples
-// (3*vol floats each, MOVE), then W tag byte arrays (vol bytes each, MOVE),
-// then W crossing queues (QCAP entries of QWORDS words, MOVE), then W
-// leaver buffers (LBCAP records of LBWORDS words, order-free sort, lbuf).
+// LDS: E and B planes (6*vol floats, PUSH), then J (MOVE: 3*vol 64-bit
+// elements, or 3*vol floats with DET), then W crossing queues (QCAP entries
+// of QWORDS words, MOVE), then W leaver buffers (LBCAP records of LBWORDS
+// words, order-free sort, lbuf).
 //
 // Fast mode: a particle that stays in its cell deposits its single segment
 // in the iteration that moves it; one that crosses a cell edge (about one in
@@ -407,12 +413,18 @@ constexpr int LBWORDS = 7;
 constexpr int SEG_CHUNK = 1, SEG_OLD_NP = 2, SEG_OLD_OFF = 3, SEG_COUNT = 4, SEG_FIRST = 5;
 constexpr int SEG16 = 13;
 
-// LDS of the particle pass: E and B planes (PUSH), W private J triples, W
-// tag arrays and W crossing queues (MOVE), W leaver buffers (lbuf).
+// LDS of the particle pass.
 __host__ __device__ inline size_t particles_lds_bytes( int vol, int W, bool push, bool move, bool lbuf = false ) {
-    return sizeof( float ) * (size_t) vol * ( ( push ? 6 : 0 ) + ( move ? 3 * W : 0 ) ) +
-           ( move ? ( ( (size_t) W * vol + 3 ) & ~(size_t) 3 ) + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 ) +
+    return sizeof( float ) * (size_t) vol * ( push ? 6 : 0 ) +
+           ( move ? sizeof( u64 ) * (size_t) vol * 3 + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 ) +
            ( move && lbuf ? sizeof( float ) * (size_t) W * LBCAP * LBWORDS : 0 );
+}
+// The rule that fits a pass's waves to the tile (zpic_fitted_threads_per_tile
+// states it): 64 KiB for the fields and a float J and a byte of each element
+// per wave.
+__host__ __device__ inline size_t fit_bytes( int vol, int W, bool push, bool move ) {
+    return sizeof( float ) * (size_t) vol * ( ( push ? 6 : 0 ) + ( move ? 3 * W : 0 ) ) +
+           ( move ? ( ( (size_t) W * vol + 3 ) & ~(size_t) 3 ) + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 );
 }
 
 // Arguments of one instance of the particle pass.
@@ -547,16 +559,15 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     float * Bx = Ez + vol;
     float * By = Bx + vol;
     float * Bz = By + vol;
-    float * Jall = PUSH ? Bz + vol : smem;        // W triples of planes
-    float * Jx = Jall + 3 * vol * w;              // this wave's planes
+    float * Jall = PUSH ? Bz + vol : smem;  // 64-bit elements (node, component); DET: three float planes
+    float * Jx = Jall;
     float * Jy = Jx + vol;
     float * Jz = Jy + vol;
-    unsigned char * tags = reinterpret_cast<unsigned char *>( Jall + 3 * vol * W ) + (size_t) vol * w;
-    float * const qbase = reinterpret_cast<float *>( reinterpret_cast<unsigned char *>( Jall + 3 * vol * W ) +
-                                                     ( ( (size_t) W * vol + 3 ) & ~(size_t) 3 ) );
+    float * const qbase = Jall + 6 * vol;
     float * queue = qbase + (size_t) w * QCAP * QWORDS;
     float * lbuf = qbase + (size_t) W * QCAP * QWORDS + (size_t) w * LBCAP * LBWORDS;  // if a.lbuf
     __shared__ int s_cnt[9];
+    __shared__ int s_bad;  // a segment that cannot be deposited
     __shared__ double s_en[FAST_BLOCK / WAVE];
     __shared__ int s_nl[FAST_BLOCK / WAVE];
     const int off = gbl( P.off )[t];
@@ -575,8 +586,9 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
         }
     }
     if constexpr ( MOVE ) {
-        for ( int k = tid; k < 3 * vol * W; k += nthr ) Jall[k] = 0.0f;
+        for ( int k = tid; k < 6 * vol; k += nthr ) Jall[k] = 0.0f;
         if ( tid < 9 ) s_cnt[tid] = 0;
+        if ( tid == 9 ) s_bad = 0;
     }
     __syncthreads();
 
@@ -603,7 +615,10 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     volatile lds_f32 * j0x = (volatile lds_f32 *) ( Jx + g.off );
     volatile lds_f32 * j0y = (volatile lds_f32 *) ( Jy + g.off );
     volatile lds_f32 * j0z = (volatile lds_f32 *) ( Jz + g.off );
-    volatile lds_u8 * tag0 = (volatile lds_u8 *) ( tags + g.off );
+    lds_u64 * const jfix = (lds_u64 *) reinterpret_cast<u64 *>( Jall );
+    lds_u64 * const jfix0 = jfix + 3 * g.off;
+    const Fixed fx = fixed_point( np );
+    bool ok = true;  // every segment so far was deposited
 
     double en = 0.0;
     int nl = 0;
@@ -641,9 +656,9 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
             int2 di;
             ns = split_path( c0, x0, x1, d, qvz, di, sg );
         }
-        deposit_elected( ns > 0, sg[0], m.qnx, m.qny, j0x, j0y, j0z, tag0, ys, lane );
-        if ( __ballot( ns > 1 ) ) deposit_elected( ns > 1, sg[1], m.qnx, m.qny, j0x, j0y, j0z, tag0, ys, lane );
-        if ( __ballot( ns > 2 ) ) deposit_elected( ns > 2, sg[2], m.qnx, m.qny, j0x, j0y, j0z, tag0, ys, lane );
+#pragma unroll
+        for ( int k = 0; k < 3; k++ )
+            if ( ns > k ) ok &= deposit_fixed( sg[k], jfix0, ys, fx );
     };
 
     // The particles of the next PREFETCH iterations are loaded while the
@@ -714,7 +729,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
             s0.c = c;
             s0.a = x;
             s0.b = make_float2( x.x + d.x, x.y + d.y );
-            s0.qvz = m.q * u.z * rg * 0.5f;
+            s0.qvz = u.z * rg * 0.5f;
             // deltai (species.cpp:342-343)
             const int2 di = make_int2( ( s0.b.x >= 0.5f ) - ( s0.b.x < -0.5f ), ( s0.b.y >= 0.5f ) - ( s0.b.y < -0.5f ) );
             const bool cross = act && ( di.x != 0 || di.y != 0 );
@@ -785,7 +800,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
             }
             nl += __popcll( mask );
             // paths inside one cell: their single segment now
-            deposit_elected( act && !cross, s0, m.qnx, m.qny, j0x, j0y, j0z, tag0, ys, lane );
+            if ( act && !cross ) ok &= deposit_fixed( s0, jfix0, ys, fx );
             // paths that cross: queued, split and deposited 64 at a time
             const unsigned long long cm = __ballot( cross );
             if ( cm ) {
@@ -863,6 +878,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     }
     if constexpr ( MOVE && !DET ) {
         if ( qn > 0 ) flush_queue( qn );
+        if ( !ok ) s_bad = 1;
         if ( lbon && lbn > 0 ) flush_leavers( lbn );
     }
 
@@ -882,13 +898,19 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
         // (species.cpp:1488-1492)
         const gptr<float> Jt = gbl( nparts > 1 ? a.parts.J + (size_t) y * 3 * vol
                                                : reinterpret_cast<float *>( J + (size_t) t * vol ) );
+        const float bad = ( !DET && s_bad ) ? __builtin_nanf( "" ) : 0.0f;
         for ( int k = tid; k < 3 * g.ext_x * g.ext_y; k += nthr ) {
             const int el = k / 3, c = k - 3 * el;
-            float s = Jall[c * vol + el];
-            for ( int v = 1; v < W; v++ ) s += Jall[3 * vol * v + c * vol + el];
+            float s;
+            if constexpr ( DET ) {
+                s = Jall[c * vol + el];
+            } else {
+                const double sum = (double) (long long) jfix[k] * fx.unit;
+                s = (float) ( sum * (double) ( c == 0 ? m.qnx : c == 1 ? m.qny : m.q ) ) + bad;  // + 0: never -0
+            }
             // jset (the first species of a step, fast mode): the region is
             // written instead of zeroed and added to; the same value, since
-            // s is never -0 (every plane element starts at +0)
+            // s is never -0
             if ( !DET && ( a.jset || nparts > 1 ) ) Jt[k] = s;
             else Jt[k] += s;
         }
@@ -2008,13 +2030,13 @@ int g_threads = 256;  // library-wide setting
 // time.
 int g_reference_order = 0;
 
-constexpr size_t LDS_LIMIT = 65536;  // dynamic LDS per workgroup
+constexpr size_t LDS_LIMIT = 65536;  // LDS of fit_bytes (the LDS itself takes up to 84 KiB for the largest tile)
 
 // Threads per tile the particle pass runs with for tiles of `vol` elements
 // when asked for `threads` (reduced until the LDS staging fits).
 int fitted_threads( int threads, int vol ) {
-    while ( threads > WAVE && particles_lds_bytes( vol, threads / WAVE, true, true ) > LDS_LIMIT ) threads -= WAVE;
-    return particles_lds_bytes( vol, threads / WAVE, true, true ) > LDS_LIMIT ? 0 : threads;
+    while ( threads > WAVE && fit_bytes( vol, threads / WAVE, true, true ) > LDS_LIMIT ) threads -= WAVE;
+    return fit_bytes( vol, threads / WAVE, true, true ) > LDS_LIMIT ? 0 : threads;
 }
 
 int check_threads( int threads ) {
@@ -2042,10 +2064,10 @@ int launch_particles( const zpic_particles * p, const zpic_geom * fld, const flo
     const int nt = fld->ntiles_x * fld->ntiles_y;
     // Large tiles: fewer wavefronts (each holds a private J copy) until LDS fits.
     int threads = det ? WAVE : g_threads;
-    while ( threads > WAVE && particles_lds_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT )
-        threads -= WAVE;
+    while ( threads > WAVE && fit_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT ) threads -= WAVE;
+    if ( fit_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT )
+        return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
     size_t lds = particles_lds_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE );
-    if ( lds > LDS_LIMIT ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
     PartArgs a{};
     a.P = view( p ); a.g = make_geo( fld );
     a.E = (const float3 *) E; a.B = (const float3 *) B; a.J = (float3 *) J;
@@ -2058,7 +2080,7 @@ int launch_particles( const zpic_particles * p, const zpic_geom * fld, const flo
         ZPIC_HIP_TRY( hipGetDevice( &dev ) );
         ZPIC_HIP_TRY( hipDeviceGetAttribute( &cu_lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev ) );
         const size_t stat = 256;  // the kernel's static LDS, rounded up
-        if ( with <= LDS_LIMIT && cu_lds / ( with + stat ) >= cu_lds / ( lds + stat ) ) {
+        if ( cu_lds / ( with + stat ) >= std::min( (size_t) 4, cu_lds / ( lds + stat ) ) ) {
             a.lbuf = 1;
             lds = with;
         }
@@ -2596,7 +2618,6 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
         weight[i] = 4LL * f.g.ntiles_x * f.g.ntiles_y * f.g.tile_vol;
         for ( int k = 0; k < nslots; k++ ) weight[i] += sp[k * n + i].p.max_part;
     }
-    if ( lds > LDS_LIMIT ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
     std::stable_sort( order.begin(), order.end(), [&]( int a, int b ) { return weight[a] > weight[b]; } );
     plan->block = block;
     plan->lds = lds;
