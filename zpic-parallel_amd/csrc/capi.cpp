@@ -401,11 +401,18 @@ long long zpic_species_charge( zpic_species * h, float * out ) {
         bnd<unsigned int> gc;
         gc.x = { 0, 1 };
         gc.y = { 0, 1 };
+        if ( !out ) {
+            // the size alone
+            const uint2 nt = h->sp->get_ntiles(), nx = h->sp->get_nx();
+            zpic_geom g{};
+            zpic::check( zpic_geom_init( &g, (int) nt.x, (int) nt.y, (int) nx.x, (int) nx.y, 0, 1 ) );
+            return (long long) g.tile_vol * ( (long long) nt.x * nt.y );
+        }
         grid<float> rho( h->sp->get_ntiles(), h->sp->get_nx(), gc );
         rho.zero();
         h->sp->deposit_charge( rho );
         rho.add_from_gc();
-        if ( out ) rho.download( out );
+        rho.download( out );
         return (long long) rho.buffer_size();
     } catch ( std::exception & e ) {
         return zpic::set_error( ZPIC_EINVAL, e.what() );

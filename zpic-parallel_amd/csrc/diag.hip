@@ -4,22 +4,27 @@
 // n = (d - min) * (size / (max - min)) - 0.5, k = int(n + 1) - 1, linear
 // weights (1 - w, w), the last bin of each axis never written.
 //
-// Fast mode: one workgroup per tile; the tile's contributions go to a
-// workgroup-private histogram in LDS when it fits (float LDS atomics), and
-// are added to the output with global float atomics.  Deterministic mode: one
-// wavefront walks the tiles and their particles in the reference's order and
-// adds them in that order, so the result is bit-identical to the reference's
-// (single-thread) deposit.
-#include "common.h"
+// Fast mode: a workgroup takes a few neighbouring tiles and sums their weights
+// in LDS in 64-bit fixed point, over the bins their particles can reach (a
+// tile's own cells along an axis of x or y), then adds those bins to the
+// output with global float atomics; where they do not fit, every term goes
+// there.  (9.4 million particles in 2304 tiles: x-ux on 128 x 96 bins 60 us,
+// uz 30 us; with a histogram of all bins in floats for each tile 233 and 101
+// us.)  Deterministic mode: one wavefront walks the tiles and their
+// particles in the reference's order and adds them in that order, so the
+// result is bit-identical to the reference's (single-thread) deposit.
+#include "fixed.h"
 
+#include <algorithm>
 #include <vector>
 
 namespace zpic {
 namespace {
 
 constexpr int WAVE = 64;
-constexpr int PHA_BLOCK = 256;
-constexpr int PHA_LDS_BINS = 12288;  // 48 KiB of float bins
+constexpr int PHA_BLOCK = 512;
+constexpr int PHA_LDS_BINS = 8192;  // 64 KiB
+constexpr int PHA_GROUPS = 1024;    // workgroups aimed at: each adds its bins to the output once
 
 struct PhaAxis {
     int quant;   // 0 x, 1 y, 2 ux, 3 uy, 4 uz
@@ -34,7 +39,8 @@ struct PhaArgs {
     const int2 * ix;
     const float2 * x;
     const float3 * u;
-    int ntx, nx, ny;
+    int ntx, nty, nx, ny;
+    int gx, gy;  // tiles of a workgroup along x and y
     PhaAxis a0, a1;  // a1.size == 0 for a 1-D phase space
     float norm;
 };
@@ -58,51 +64,94 @@ __device__ inline void pha_bin( const PhaAxis & a, float d, int & k, float & w )
 
 __device__ inline bool in_axis( int k, int size ) { return k >= 0 && k < size - 1; }
 
-// The (up to four) contributions of one particle, in the reference's order.
+// The (up to four) contributions of one particle, in the reference's order,
+// without the normalisation: add( k0, k1, weight ).
 template <class ADD>
 __device__ inline void pha_deposit( const PhaArgs & a, int shiftx, int shifty, int2 c, float2 x, float3 u, ADD add ) {
     int k0;
     float w0;
     pha_bin( a.a0, pha_value( a.a0.quant, shiftx, shifty, c, x, u ), k0, w0 );
     if ( a.a1.size == 0 ) {
-        if ( in_axis( k0, a.a0.size ) ) add( k0, ( 1 - w0 ) * a.norm );
-        if ( in_axis( k0 + 1, a.a0.size ) ) add( k0 + 1, w0 * a.norm );
+        if ( in_axis( k0, a.a0.size ) ) add( k0, 0, 1 - w0 );
+        if ( in_axis( k0 + 1, a.a0.size ) ) add( k0 + 1, 0, w0 );
         return;
     }
     int k1;
     float w1;
     pha_bin( a.a1, pha_value( a.a1.quant, shiftx, shifty, c, x, u ), k1, w1 );
-    const int s0 = a.a0.size;
-    if ( in_axis( k0, s0 ) && in_axis( k1, a.a1.size ) ) add( k1 * s0 + k0, ( 1 - w0 ) * ( 1 - w1 ) * a.norm );
-    if ( in_axis( k0 + 1, s0 ) && in_axis( k1, a.a1.size ) ) add( k1 * s0 + k0 + 1, w0 * ( 1 - w1 ) * a.norm );
-    if ( in_axis( k0, s0 ) && in_axis( k1 + 1, a.a1.size ) ) add( ( k1 + 1 ) * s0 + k0, ( 1 - w0 ) * w1 * a.norm );
-    if ( in_axis( k0 + 1, s0 ) && in_axis( k1 + 1, a.a1.size ) )
-        add( ( k1 + 1 ) * s0 + k0 + 1, w0 * w1 * a.norm );
+    const int s0 = a.a0.size, s1 = a.a1.size;
+    if ( in_axis( k0, s0 ) && in_axis( k1, s1 ) ) add( k0, k1, ( 1 - w0 ) * ( 1 - w1 ) );
+    if ( in_axis( k0 + 1, s0 ) && in_axis( k1, s1 ) ) add( k0 + 1, k1, w0 * ( 1 - w1 ) );
+    if ( in_axis( k0, s0 ) && in_axis( k1 + 1, s1 ) ) add( k0, k1 + 1, ( 1 - w0 ) * w1 );
+    if ( in_axis( k0 + 1, s0 ) && in_axis( k1 + 1, s1 ) ) add( k0 + 1, k1 + 1, w0 * w1 );
 }
 
-__global__ void __launch_bounds__( PHA_BLOCK ) k_phasespace( PhaArgs a, float * __restrict__ out, int bins ) {
-    extern __shared__ float hist[];
-    const int t = blockIdx.x;
-    const bool local = bins <= PHA_LDS_BINS;
+// Bins of an axis that the particles of cells [cell, cell + n) reach: [lo, hi).
+__device__ inline void pha_range( const PhaAxis & a, int cell, int n, int & lo, int & hi ) {
+    lo = 0;
+    hi = a.size;
+    if ( a.quant > 1 ) return;
+    float w;
+    pha_bin( a, (float) cell, lo, w );
+    pha_bin( a, (float) ( cell + n ), hi, w );
+    lo = min( max( lo, 0 ), a.size );
+    hi = max( lo, min( hi + 2, a.size ) );
+}
+
+__global__ void __launch_bounds__( PHA_BLOCK ) k_phasespace( PhaArgs a, float * __restrict__ out, int cap ) {
+    extern __shared__ __align__( 16 ) u64 hist_[];
+    lds_u64 * const hist = (lds_u64 *) hist_;
+    const int ngx = ( a.ntx + a.gx - 1 ) / a.gx;
+    const int tx0 = blockIdx.x % ngx * a.gx, ty0 = blockIdx.x / ngx * a.gy;
+    const int tx1 = min( a.ntx, tx0 + a.gx ), ty1 = min( a.nty, ty0 + a.gy );
+    const bool two = a.a1.size > 0;
+    int lo0, hi0, lo1 = 0, hi1 = 1;
+    pha_range( a.a0, a.a0.quant == 0 ? tx0 * a.nx : ty0 * a.ny, a.a0.quant == 0 ? ( tx1 - tx0 ) * a.nx : ( ty1 - ty0 ) * a.ny,
+               lo0, hi0 );
+    if ( two )  // (the second axis is never x)
+        pha_range( a.a1, ty0 * a.ny, ( ty1 - ty0 ) * a.ny, lo1, hi1 );
+    const int n0 = hi0 - lo0, bins = n0 * ( hi1 - lo1 );
+    const bool local = bins <= cap;  // cap: bins of LDS
+    if ( local )
+        for ( int k = threadIdx.x; k < bins; k += blockDim.x ) hist[k] = 0;
+    int total = 0;
+    for ( int ty = ty0; ty < ty1; ty++ )
+        for ( int tx = tx0; tx < tx1; tx++ ) total += a.np[ty * a.ntx + tx];
+    const Fixed fx = fixed_point( total );
+    __syncthreads();
+    const bool pos = a.a0.quant < 2 || ( two && a.a1.quant < 2 ), mom = a.a0.quant > 1 || ( two && a.a1.quant > 1 );
+    auto global_add = [&]( int k0, int k1, float v ) { atomicAdd( &out[k1 * a.a0.size + k0], v * a.norm ); };
+    for ( int ty = ty0; ty < ty1; ty++ )
+        for ( int tx = tx0; tx < tx1; tx++ ) {
+            const int t = ty * a.ntx + tx;
+            const int off = a.off[t], np = a.np[t];
+            for ( int i = threadIdx.x; i < np; i += blockDim.x ) {
+                int2 c = make_int2( 0, 0 );
+                float2 x = make_float2( 0.f, 0.f );
+                float3 u = make_float3( 0.f, 0.f, 0.f );
+                if ( pos ) {
+                    c = a.ix[off + i];
+                    x = a.x[off + i];
+                }
+                if ( mom ) u = a.u[off + i];
+                if ( local )
+                    pha_deposit( a, tx * a.nx, ty * a.ny, c, x, u, [&]( int k0, int k1, float v ) {
+                        // (out of reach: a position outside its cell, or not a number)
+                        if ( k0 >= lo0 && k0 < hi0 && k1 >= lo1 && k1 < hi1 && fabsf( v ) < 4.0f )
+                            fixed_add( hist + ( k1 - lo1 ) * n0 + k0 - lo0, v, fx );
+                        else
+                            global_add( k0, k1, v );
+                    } );
+                else
+                    pha_deposit( a, tx * a.nx, ty * a.ny, c, x, u, global_add );
+            }
+        }
     if ( local ) {
-        for ( int k = threadIdx.x; k < bins; k += blockDim.x ) hist[k] = 0.0f;
         __syncthreads();
-    }
-    const int shiftx = ( t % a.ntx ) * a.nx, shifty = ( t / a.ntx ) * a.ny;
-    const int off = a.off[t], np = a.np[t];
-    for ( int i = threadIdx.x; i < np; i += blockDim.x ) {
-        const int2 c = a.ix[off + i];
-        const float2 x = a.x[off + i];
-        const float3 u = a.u[off + i];
-        if ( local )
-            pha_deposit( a, shiftx, shifty, c, x, u, [&]( int k, float v ) { atomicAdd( &hist[k], v ); } );
-        else
-            pha_deposit( a, shiftx, shifty, c, x, u, [&]( int k, float v ) { atomicAdd( &out[k], v ); } );
-    }
-    if ( local ) {
-        __syncthreads();
-        for ( int k = threadIdx.x; k < bins; k += blockDim.x )
-            if ( hist[k] != 0.0f ) atomicAdd( &out[k], hist[k] );
+        for ( int k = threadIdx.x; k < bins; k += blockDim.x ) {
+            const u64 v = hist[k];
+            if ( v != 0 ) atomicAdd( &out[( lo1 + k / n0 ) * a.a0.size + lo0 + k % n0], fixed_value( v, fx, a.norm ) );
+        }
     }
 }
 
@@ -125,9 +174,9 @@ __global__ void __launch_bounds__( WAVE ) k_phasespace_det( PhaArgs a, float * _
             }
             for ( int l = 0; l < WAVE && i0 + l < np; l++ ) {
                 if ( lane == l )
-                    pha_deposit( a, shiftx, shifty, c, x, u, [&]( int k, float v ) {
-                        volatile float * o = out + k;
-                        *o = *o + v;
+                    pha_deposit( a, shiftx, shifty, c, x, u, [&]( int k0, int k1, float v ) {
+                        volatile float * o = out + k1 * a.a0.size + k0;
+                        *o = *o + v * a.norm;
                     } );
                 __builtin_amdgcn_wave_barrier();
             }
@@ -153,20 +202,34 @@ extern "C" int zpic_phasespace( const zpic_particles * p, int ntiles_x, int ntil
     PhaArgs a;
     a.np = p->np; a.off = p->offset; a.ix = (const int2 *) p->ix; a.x = (const float2 *) p->x;
     a.u = (const float3 *) p->u;
-    a.ntx = ntiles_x; a.nx = nx; a.ny = ny;
+    a.ntx = ntiles_x; a.nty = ntiles_y; a.nx = nx; a.ny = ny;
     a.a0 = PhaAxis{ quant0, min0, size0 / ( max0 - min0 ), size0 };
     a.a1 = two ? PhaAxis{ quant1, min1, size1 / ( max1 - min1 ), size1 } : PhaAxis{ 0, 0.f, 0.f, 0 };
     a.norm = norm;
     const long long bins = (long long) size0 * ( two ? size1 : 1 );
     if ( bins > ( 1ll << 30 ) ) return set_error( ZPIC_ERANGE, "phase-space grid too large" );
     hipStream_t st = as_stream( stream );
-    ZPIC_HIP_TRY( hipMemsetAsync( out, 0, sizeof( float ) * bins, st ) );
+    if ( int rc = zpic_fill( out, (size_t) bins, 0.0f, st ) ) return rc;
     const int nt = ntiles_x * ntiles_y;
     if ( deterministic ) {
         hipLaunchKernelGGL( k_phasespace_det, dim3( 1 ), dim3( WAVE ), 0, st, a, out, nt );
     } else {
-        const size_t lds = bins <= PHA_LDS_BINS ? sizeof( float ) * bins : 0;
-        hipLaunchKernelGGL( k_phasespace, dim3( nt ), dim3( PHA_BLOCK ), lds, st, a, out, (int) bins );
+        // tiles above one another share their bins of x, beside one another
+        // those of y
+        const bool over_y = quant0 == 0 && !( two && quant1 == 1 );
+        const int n = ( nt + PHA_GROUPS - 1 ) / PHA_GROUPS;
+        a.gx = over_y ? 1 : std::min( n, ntiles_x );
+        a.gy = over_y ? std::min( n, ntiles_y ) : 1;
+        const int groups = ( ( ntiles_x + a.gx - 1 ) / a.gx ) * ( ( ntiles_y + a.gy - 1 ) / a.gy );
+        // the most bins a workgroup's particles reach along each axis
+        auto reach = []( const PhaAxis & x, int cells ) -> long long {
+            if ( x.quant > 1 ) return x.size;
+            const float r = (float) cells * x.rdx + 4.0f;
+            return r < (float) x.size ? (long long) r : x.size;
+        };
+        const long long most = reach( a.a0, quant0 == 0 ? a.gx * nx : a.gy * ny ) * ( two ? reach( a.a1, a.gy * ny ) : 1 );
+        const int cap = (int) std::min( most, (long long) PHA_LDS_BINS );
+        hipLaunchKernelGGL( k_phasespace, dim3( groups ), dim3( PHA_BLOCK ), sizeof( u64 ) * cap, st, a, out, cap );
     }
     ZPIC_LAUNCH_CHECK( "k_phasespace" );
     return ZPIC_OK;

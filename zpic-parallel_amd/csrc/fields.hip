@@ -93,7 +93,7 @@ constexpr int CUR_BLOCK = 128;
 constexpr int CUR_TILES = 2;
 template <int NP>
 __global__ void __launch_bounds__( CUR_BLOCK_FEW ) k_current( CurArgs a ) {
-    extern __shared__ float sm[];
+    extern __shared__ __align__( 16 ) float sm[];
     for ( int t = blockIdx.x; t < a.g.ntx * a.g.nty; t += gridDim.x ) {
         if ( t != (int) blockIdx.x ) __syncthreads();  // LDS of the previous tile read out
         current_tile<NP>( a, t, sm );
@@ -101,52 +101,81 @@ __global__ void __launch_bounds__( CUR_BLOCK_FEW ) k_current( CurArgs a ) {
 }
 
 __global__ void __launch_bounds__( TILE_BLOCK ) k_yee( YeeArgs a, const YeeArgs * tab, const int2 * map ) {
-    extern __shared__ float sm[];
+    extern __shared__ __align__( 16 ) float sm[];
     const int t = select_instance( a, tab, map );
     yee_tile( a, t, sm );
 }
 
-// EMF::get_energy per tile (emf.cpp:680-705): one thread per (tile,
-// component), cells in the reference's order; the inner bound is nx.y as in
-// the reference loop.
-__global__ void k_energy_tiles( const float * __restrict__ E, const float * __restrict__ B, G g,
-                                double * __restrict__ out ) {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nt = g.ntx * g.nty;
-    if ( gid >= 6 * nt ) return;
-    const int t = gid / 6, comp = gid % 6;
-    const float * F = ( comp < 3 ) ? E : B;
-    const int c = comp % 3;
-    const float * base = F + ( (size_t) t * g.vol + g.off ) * 3;
-    double s = 0;
-    for ( int iy = 0; iy < g.ny; iy++ )
-        for ( int ix = 0; ix < g.ny; ix++ ) {
-            const float v = base[( iy * g.ext_x + ix ) * 3 + c];
-            s += v * v;
+// EMF::get_energy per tile (emf.cpp:680-705), cells in the reference's order;
+// the inner bound is nx.y as in the reference loop.  A wave stages a tile's
+// cells in LDS, ENERGY_CELLS at a time, and a lane per component of E and B
+// adds them (15 us for 2304 tiles; 106 us with a lane per tile and component,
+// each walking its own tile in global memory).
+constexpr int ENERGY_CELLS = 256;
+__global__ void __launch_bounds__( 64 ) k_energy_tiles( const float * __restrict__ E, const float * __restrict__ B, G g,
+                                                        double * __restrict__ out ) {
+    __shared__ float s[6][ENERGY_CELLS + 1];
+    const int t = blockIdx.x, lane = threadIdx.x;
+    const size_t base = ( (size_t) t * g.vol + g.off ) * 3;
+    const int n = g.ny * g.ny;
+    double sum = 0;
+    for ( int c0 = 0; c0 < n; c0 += ENERGY_CELLS ) {
+        const int m = min( ENERGY_CELLS, n - c0 );
+        __syncthreads();
+        for ( int e = lane; e < 3 * m; e += 64 ) {
+            const int cell = c0 + e / 3, c = e % 3;
+            const size_t k = base + ( cell / g.ny * g.ext_x + cell % g.ny ) * 3 + c;
+            s[c][e / 3] = E[k];
+            s[3 + c][e / 3] = B[k];
         }
-    out[6 * t + comp] = s;
+        __syncthreads();
+        if ( lane < 6 ) {
+#pragma unroll 8
+            for ( int k = 0; k < m; k++ ) {
+                const float v = s[lane][k];
+                sum += v * v;
+            }
+        }
+    }
+    if ( lane < 6 ) out[6 * t + lane] = sum;
 }
 
 // Sums tile values in tile order, out[c] = 0 + ((v0 + v1) + ...): the block
-// stages 1024 values at a time in LDS and thread c adds them in order.
+// stages SUM_BLOCK tiles' values at a time in LDS, the next ones on their
+// way, and thread c adds component c in order.  NC = values per tile (18 us
+// for six values of 2304 tiles; 526 us component after component).
 constexpr int SUM_BLOCK = 1024;
-__global__ void __launch_bounds__( SUM_BLOCK ) k_sum_tiles( const double * __restrict__ v, int n, int stride,
+template <int NC>
+__global__ void __launch_bounds__( SUM_BLOCK ) k_sum_tiles( const double * __restrict__ v, int n,
                                                             double * __restrict__ out ) {
-    __shared__ double buf[SUM_BLOCK];
-    for ( int c = 0; c < stride; c++ ) {
-        double acc = 0;
-        for ( int base = 0; base < n; base += SUM_BLOCK ) {
-            const int t = base + threadIdx.x;
-            buf[threadIdx.x] = t < n ? v[(size_t) t * stride + c] : 0.0;
-            __syncthreads();
-            if ( threadIdx.x == 0 ) {
-                const int m = min( SUM_BLOCK, n - base );
-                for ( int k = 0; k < m; k++ ) acc += buf[k];
-            }
-            __syncthreads();
+    __shared__ double buf[NC][SUM_BLOCK + 1];
+    double acc = 0, next[NC];
+    const int tid = threadIdx.x;
+    const size_t all = (size_t) n * NC;
+    auto load = [&]( int base ) {
+#pragma unroll
+        for ( int i = 0; i < NC; i++ ) {
+            const size_t k = (size_t) base * NC + i * SUM_BLOCK + tid;
+            next[i] = k < all ? v[k] : 0.0;
         }
-        if ( threadIdx.x == 0 ) out[c] = 0.0 + acc;
+    };
+    load( 0 );
+    for ( int base = 0; base < n; base += SUM_BLOCK ) {
+#pragma unroll
+        for ( int i = 0; i < NC; i++ ) {
+            const int e = i * SUM_BLOCK + tid;
+            buf[e % NC][e / NC] = next[i];
+        }
+        __syncthreads();
+        load( base + SUM_BLOCK );
+        if ( tid < NC ) {
+            const int m = min( SUM_BLOCK, n - base );
+#pragma unroll 16
+            for ( int k = 0; k < m; k++ ) acc += buf[tid][k];
+        }
+        __syncthreads();
     }
+    if ( tid < NC ) out[tid] = 0.0 + acc;
 }
 
 // Unordered parallel sum for the fast mode: per-thread runs (four partial
@@ -1084,9 +1113,9 @@ int field_energy_launch( const float * E, const float * B, const zpic_geom * gg,
                          hipStream_t st ) {
     const G g = make( gg );
     const int nt = g.ntx * g.nty;
-    hipLaunchKernelGGL( k_energy_tiles, dim3( ( 6 * nt + 255 ) / 256 ), dim3( 256 ), 0, st, E, B, g, tile_sums );
+    hipLaunchKernelGGL( k_energy_tiles, dim3( nt ), dim3( 64 ), 0, st, E, B, g, tile_sums );
     ZPIC_LAUNCH_CHECK( "k_energy_tiles" );
-    hipLaunchKernelGGL( k_sum_tiles, dim3( 1 ), dim3( SUM_BLOCK ), 0, st, tile_sums, nt, 6, out6 );
+    hipLaunchKernelGGL( k_sum_tiles<6>, dim3( 1 ), dim3( SUM_BLOCK ), 0, st, tile_sums, nt, out6 );
     ZPIC_LAUNCH_CHECK( "k_sum_tiles" );
     return ZPIC_OK;
 }
@@ -1150,7 +1179,7 @@ int zpic_field_energy_noalloc( const float * E, const float * B, const zpic_geom
 int zpic_sum_tiles( const double * v, int n, double * out, int deterministic, void * stream ) {
     if ( !v || !out || n < 0 ) return set_error( ZPIC_EINVAL, "invalid arguments" );
     if ( deterministic )
-        hipLaunchKernelGGL( k_sum_tiles, dim3( 1 ), dim3( SUM_BLOCK ), 0, as_stream( stream ), v, n, 1, out );
+        hipLaunchKernelGGL( k_sum_tiles<1>, dim3( 1 ), dim3( SUM_BLOCK ), 0, as_stream( stream ), v, n, out );
     else
         hipLaunchKernelGGL( k_sum_tiles_fast, dim3( 1 ), dim3( SUM_BLOCK ), 0, as_stream( stream ), v, n, out );
     ZPIC_LAUNCH_CHECK( "k_sum_tiles" );

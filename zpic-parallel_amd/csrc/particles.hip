@@ -19,6 +19,7 @@
 // tile and serialises the deposit and the energy sum over lanes in particle
 // order, which reproduces the reference's single-thread results exactly.
 #include "common.h"
+#include "fixed.h"
 #include "grid_ops.h"
 #include "parts.h"
 
@@ -294,37 +295,6 @@ __device__ inline void add_current( volatile lds_f32 * Jx, volatile lds_f32 * Jy
     Jx[k + ys] = Jx[k + ys] + v[5];
     Jz[k + ys] = Jz[k + ys] + v[6];
     Jz[k + ys + 1] = Jz[k + ys + 1] + v[7];
-}
-
-// The fast mode's current in LDS: 64-bit fixed point, 2^bits to the unit, for
-// contributions without their charge factors (a path's displacement in a
-// cell times its weights, at most 1; for z the velocity over c).  With `bits`
-// the np particles of a workgroup cannot overflow an element (FIX_HEADROOM
-// bits are left for a path's up to three segments and for weights of
-// positions a little outside their cell), and a contribution is off by at
-// most 2^-47 of the unit up to 2047 particles and 2^-43 at 16384: far less
-// than the rounding of its own FP32 arithmetic, and the sum adds nothing.
-typedef unsigned long long u64;
-typedef __attribute__( ( address_space( 3 ) ) ) u64 lds_u64;
-constexpr int FIX_HEADROOM = 5, FIX_MAX_BITS = 46;
-
-struct Fixed {
-    double magic;   // 1.5 * 2^(52 - bits): adding it leaves value * 2^bits in the low mantissa bits
-    unsigned hi;    // its upper word (the lower one is 0)
-    double unit;    // 2^-bits
-};
-__device__ inline Fixed fixed_point( int np ) {
-    const int bits = min( FIX_MAX_BITS, 62 - FIX_HEADROOM - ( 32 - __clz( np ) ) );
-    Fixed f;
-    f.hi = ( (unsigned) ( 1023 + 52 - bits ) << 20 ) | 0x80000u;
-    f.magic = __hiloint2double( (int) f.hi, 0 );
-    f.unit = __hiloint2double( ( 1023 - bits ) << 20, 0 );
-    return f;
-}
-__device__ inline void fixed_add( lds_u64 * p, float v, const Fixed & f ) {
-    u64 b = (u64) __double_as_longlong( (double) v + f.magic );
-    b -= (u64) f.hi << 32;
-    __hip_atomic_fetch_add( p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
 }
 
 // Fast-mode deposit of one segment into J, element (node, component).
@@ -905,8 +875,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
             if constexpr ( DET ) {
                 s = Jall[c * vol + el];
             } else {
-                const double sum = (double) (long long) jfix[k] * fx.unit;
-                s = (float) ( sum * (double) ( c == 0 ? m.qnx : c == 1 ? m.qny : m.q ) ) + bad;  // + 0: never -0
+                s = fixed_value( jfix[k], fx, c == 0 ? m.qnx : c == 1 ? m.qny : m.q ) + bad;  // + 0: never -0
             }
             // jset (the first species of a step, fast mode): the region is
             // written instead of zeroed and added to; the same value, since
@@ -949,7 +918,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
 
 template <bool PUSH, bool MOVE, bool DET>
 __global__ void __launch_bounds__( FAST_BLOCK ) k_particles( PartArgs a, const PartArgs * tab, const int2 * map ) {
-    extern __shared__ float smem[];
+    extern __shared__ __align__( 16 ) float smem[];
     const int t = select_instance( a, tab, map );
     particles_tile<PUSH, MOVE, DET>( a, t, smem );
 }
@@ -1932,46 +1901,60 @@ __global__ void __launch_bounds__( SORT_WAVES * WAVE ) k_sort_in_fast( SortArgs 
 
 // ---------------------------------------------------------------------------
 // dep_charge_kernel (species.cpp:2348-2395) into a scalar grid with guards.
+// Fast mode: the weights are summed in LDS in 64-bit fixed point and take
+// the charge at the end (float atomics there: 194 us for the 9.4 million
+// particles of 2304 tiles, against 40 us).
 template <bool DET>
 __global__ void __launch_bounds__( FAST_BLOCK ) k_charge( PartView P, Geo g, float * __restrict__ rho, float q ) {
-    extern __shared__ float smem[];
+    extern __shared__ __align__( 16 ) float smem[];
     const int t = blockIdx.x;
     const int vol = g.vol, ys = g.ext_x;
-    for ( int k = threadIdx.x; k < vol; k += blockDim.x ) smem[k] = 0.0f;
+    for ( int k = threadIdx.x; k < ( DET ? vol : 2 * vol ); k += blockDim.x ) smem[k] = 0.0f;
+    __shared__ int s_bad;
+    if ( threadIdx.x == 0 ) s_bad = 0;
     __syncthreads();
     float * c0 = smem + g.off;
+    lds_u64 * const fixed = (lds_u64 *) reinterpret_cast<u64 *>( smem );
+    lds_u64 * const f0 = fixed + g.off;
     const int off = P.off[t], np = P.np[t];
+    const Fixed fx = fixed_point( np );
     const int lane = threadIdx.x % WAVE;
     const int nthr = blockDim.x;
     for ( int i0 = ( threadIdx.x / WAVE ) * WAVE; i0 < np; i0 += nthr ) {
         const int i = i0 + lane;
         const bool act = i < np;
         int k = 0;
-        float w00 = 0, w10 = 0, w01 = 0, w11 = 0;
+        float s0x = 0, s1x = 0, s0y = 0, s1y = 0;
         if ( act ) {
             const int2 c = P.ix[off + i];
             const float2 x = P.x[off + i];
             k = c.y * ys + c.x;
-            const float s0x = 0.5f - x.x, s1x = 0.5f + x.x, s0y = 0.5f - x.y, s1y = 0.5f + x.y;
-            w00 = s0y * s0x * q; w10 = s0y * s1x * q; w01 = s1y * s0x * q; w11 = s1y * s1x * q;
+            s0x = 0.5f - x.x, s1x = 0.5f + x.x, s0y = 0.5f - x.y, s1y = 0.5f + x.y;
         }
         if constexpr ( DET ) {
+            const float w00 = s0y * s0x * q, w10 = s0y * s1x * q, w01 = s1y * s0x * q, w11 = s1y * s1x * q;
             for ( int l = 0; l < WAVE; l++ ) {
                 if ( lane == l && act ) {
                     c0[k] += w00; c0[k + 1] += w10; c0[k + ys] += w01; c0[k + ys + 1] += w11;
                 }
             }
         } else if ( act ) {
-            // diagnostic path: LDS float atomics are adequate here
-            __hip_atomic_fetch_add( &c0[k], w00, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
-            __hip_atomic_fetch_add( &c0[k + 1], w10, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
-            __hip_atomic_fetch_add( &c0[k + ys], w01, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
-            __hip_atomic_fetch_add( &c0[k + ys + 1], w11, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
+            if ( fabsf( s0x ) + fabsf( s0y ) < 5.0f ) {
+                fixed_add( f0 + k, s0y * s0x, fx );
+                fixed_add( f0 + k + 1, s0y * s1x, fx );
+                fixed_add( f0 + k + ys, s1y * s0x, fx );
+                fixed_add( f0 + k + ys + 1, s1y * s1x, fx );
+            } else {
+                s_bad = 1;  // a position far outside its cell, or not a number
+            }
         }
     }
     __syncthreads();
     float * dst = rho + (size_t) t * vol;
-    for ( int k = threadIdx.x; k < g.ext_x * g.ext_y; k += blockDim.x ) dst[k] += smem[k];
+    for ( int k = threadIdx.x; k < g.ext_x * g.ext_y; k += blockDim.x ) {
+        if constexpr ( DET ) dst[k] += smem[k];
+        else dst[k] += s_bad ? __builtin_nanf( "" ) : fixed_value( fixed[k], fx, q );
+    }
 }
 
 Geo make_geo( const zpic_geom * f ) {
@@ -2373,7 +2356,7 @@ constexpr int STEP_CHAIN = 8;
 
 template <int BLOCK>
 __global__ void __launch_bounds__( BLOCK, 4 ) k_batch_step( StepTables T ) {
-    extern __shared__ float smem[];
+    extern __shared__ __align__( 16 ) float smem[];
     __shared__ int s_item;
     const int home = blockIdx.x % STEP_QUEUES;
     int q = 0;  // queues exhausted so far, counted from the home queue
@@ -3294,8 +3277,8 @@ int zpic_deposit_charge( const zpic_particles * p, const zpic_geom * g, float * 
                          void * stream ) {
     if ( !p || !g || !rho ) return set_error( ZPIC_EINVAL, "null buffer" );
     const int nt = g->ntiles_x * g->ntiles_y;
-    const size_t lds = sizeof( float ) * g->tile_vol;
-    if ( lds > 65536 ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
+    const size_t lds = ( deterministic ? sizeof( float ) : sizeof( u64 ) ) * g->tile_vol;
+    if ( sizeof( float ) * g->tile_vol > 65536 ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
     hipStream_t st = as_stream( stream );
     if ( deterministic )
         hipLaunchKernelGGL( k_charge<true>, dim3( nt ), dim3( WAVE ), lds, st, view( p ), make_geo( g ), rho, q );
