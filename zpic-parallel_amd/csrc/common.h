@@ -40,6 +40,12 @@ inline hipStream_t as_stream( void * s ) { return s ? (hipStream_t) s : default_
 int current_update( const float * dep, float * J, const zpic_geom * g, int passes, const float * coef, int px, int py,
                     void * stream );
 
+// zpic_batch_fields_create for instances whose current's deposit is made in a
+// buffer of its own (dep[i], which need not be cleared: every element but the
+// padding is written) and updated from there in one launch; dep[i] = J: in
+// place, from a deposit that zpic_batch_zero_current need not clear either.
+int batch_fields_new( zpic_batch_fields ** out, const zpic_batch_fields_item * items, int n, const float * const * dep );
+
 }  // namespace zpic
 
 #define ZPIC_HIP_TRY( call )                                               \

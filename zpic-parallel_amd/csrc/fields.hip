@@ -106,6 +106,19 @@ __global__ void __launch_bounds__( TILE_BLOCK ) k_yee( YeeArgs a, const YeeArgs 
     yee_tile( a, t, sm );
 }
 
+template <int NP>
+__global__ void __launch_bounds__( CUR_BLOCK_FEW ) k_current_batch( const CurArgs * tab, const int2 * map ) {
+    extern __shared__ __align__( 16 ) float sm[];
+    const int2 r = gbl( map )[blockIdx.x];
+    current_tile<NP>( gbl( tab )[r.x], r.y, sm );
+}
+
+template <int NC>
+__global__ void __launch_bounds__( GC_BLOCK ) k_copy_gc_xy_batch( const GcArgs * tab, const int2 * map ) {
+    const int2 r = gbl( map )[blockIdx.x];
+    copy_gc_xy_tile<NC>( gbl( tab )[r.x], r.y );
+}
+
 // EMF::get_energy per tile (emf.cpp:680-705), cells in the reference's order;
 // the inner bound is nx.y as in the reference loop.  A wave stages a tile's
 // cells in LDS, ENERGY_CELLS at a time, and a lane per component of E and B
@@ -693,7 +706,7 @@ __global__ void k_fill_batch( const FillArgs * tab ) {
 // One batched launch: a device table of per-entry arguments and the
 // block -> (entry, tile) map.
 struct Group {
-    int kind;  // 0 add_gc_x, 1 add_gc_y, 2 copy_gc_x, 3 copy_gc_y, 4 kernel3, 5 yee
+    int kind;  // 0 add_gc_x, 1 add_gc_y, 2 copy_gc_x, 3 copy_gc_y, 4 kernel3, 5 yee, 6 copy_gc, 7 + p current update of p passes
     void * tab;
     int2 * map;
     int nblocks;
@@ -727,6 +740,14 @@ int run_group( const Group & grp, hipStream_t st ) {
     case 2: hipLaunchKernelGGL( k_copy_gc_x<3>, nb, dim3( GC_BLOCK ), 0, st, GcArgs{}, (const GcArgs *) grp.tab, grp.map ); break;
     case 3: hipLaunchKernelGGL( k_copy_gc_y<3>, nb, dim3( GC_BLOCK ), 0, st, GcArgs{}, (const GcArgs *) grp.tab, grp.map ); break;
     case 4: hipLaunchKernelGGL( k_kernel3, nb, dim3( TILE_BLOCK ), grp.lds, st, K3Args{}, (const K3Args *) grp.tab, grp.map ); break;
+    case 6: hipLaunchKernelGGL( k_copy_gc_xy_batch<3>, nb, dim3( GC_BLOCK ), 0, st, (const GcArgs *) grp.tab, grp.map ); break;
+    case 7: hipLaunchKernelGGL( k_current_batch<0>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
+    case 8: hipLaunchKernelGGL( k_current_batch<1>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
+    case 9: hipLaunchKernelGGL( k_current_batch<2>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
+    case 10: hipLaunchKernelGGL( k_current_batch<3>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
+    case 11: hipLaunchKernelGGL( k_current_batch<4>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
+    case 12: hipLaunchKernelGGL( k_current_batch<5>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
+    case 13: hipLaunchKernelGGL( k_current_batch<-1>, nb, dim3( CUR_BLOCK_FEW ), grp.lds, st, (const CurArgs *) grp.tab, grp.map ); break;
     case 5: hipLaunchKernelGGL( k_yee, nb, dim3( TILE_BLOCK ), grp.lds, st, YeeArgs{}, (const YeeArgs *) grp.tab, grp.map ); break;
     }
     ZPIC_LAUNCH_CHECK( "batched grid kernel" );
@@ -748,7 +769,8 @@ struct BatchFieldPlan {
     }
 };
 
-int batch_fields_create( BatchFieldPlan ** out, const zpic_batch_fields_item * items, int n ) {
+int batch_fields_create( BatchFieldPlan ** out, const zpic_batch_fields_item * items, int n,
+                         const float * const * dep = nullptr ) {
     if ( !out || !items || n < 1 ) return set_error( ZPIC_EINVAL, "empty batch" );
     auto plan = std::make_unique<BatchFieldPlan>();
     plan->n = n;
@@ -796,9 +818,50 @@ int batch_fields_create( BatchFieldPlan ** out, const zpic_batch_fields_item * i
     ZPIC_HIP_TRY( hipMalloc( (void **) &plan->d_fill, sizeof( FillArgs ) * n ) );
     ZPIC_HIP_TRY( hipMemcpy( plan->d_fill, fills.data(), sizeof( FillArgs ) * n, hipMemcpyHostToDevice ) );
 
-    for ( int kind = 0; kind < 4; kind++ ) {
+    // instances updated from a deposit buffer of their own, by passes
+    for ( int np = 0; np <= CUR_REG_PASSES + 1; np++ ) {
+        std::vector<CurArgs> cur;
+        std::vector<int> nt;
+        size_t lds = 0;
+        for ( int i = 0; i < n; i++ ) {
+            const int P = (int) passes[i].size();
+            if ( !dep || dep[i] == items[i].J || std::min( P, CUR_REG_PASSES + 1 ) != np ) continue;
+            CurArgs a{};
+            a.dep = dep[i];
+            a.J = items[i].J;
+            a.g = jgc[i].g;
+            a.px = jgc[i].px;
+            a.py = jgc[i].py;
+            a.passes = P;
+            for ( int p = 0; p < P; p++ ) {
+                a.a[p] = passes[i][p].a;
+                a.b[p] = passes[i][p].b;
+                a.c[p] = passes[i][p].c;
+            }
+            cur.push_back( a );
+            nt.push_back( tiles[i] );
+            lds = std::max( lds, current_lds_bytes( a.g, P ) );
+        }
+        if ( cur.empty() ) continue;
         Group grp;
-        if ( int rc = make_group( grp, kind, jgc, tiles, 0 ) ) return rc;
+        if ( int rc = make_group( grp, 7 + np, cur, nt, lds ) ) return rc;
+        plan->current.push_back( grp );
+    }
+    // the others in place: guard add, guard copy, filter passes
+    std::vector<GcArgs> in_place;
+    std::vector<int> in_place_tiles;
+    for ( int i = 0; i < n; i++ ) {
+        if ( dep && dep[i] != items[i].J ) {
+            passes[i].clear();
+            continue;
+        }
+        in_place.push_back( jgc[i] );
+        in_place_tiles.push_back( tiles[i] );
+    }
+    for ( int kind : { 0, 1, 6 } ) {
+        if ( in_place.empty() ) break;
+        Group grp;
+        if ( int rc = make_group( grp, kind, in_place, in_place_tiles, 0 ) ) return rc;
         plan->current.push_back( grp );
     }
     for ( size_t p = 0; p < max_passes; p++ ) {
@@ -823,13 +886,11 @@ int batch_fields_create( BatchFieldPlan ** out, const zpic_batch_fields_item * i
         }
     }
     {
-        Group gy, gx, gyy;
+        Group gy, gc;
         if ( int rc = make_group( gy, 5, yees, tiles, sizeof( float ) * 6 * max_vol ) ) return rc;
-        if ( int rc = make_group( gx, 2, ebgc, tiles2, 0 ) ) return rc;
-        if ( int rc = make_group( gyy, 3, ebgc, tiles2, 0 ) ) return rc;
         plan->yee.push_back( gy );
-        plan->yee.push_back( gx );
-        plan->yee.push_back( gyy );
+        if ( int rc = make_group( gc, 6, ebgc, tiles2, 0 ) ) return rc;
+        plan->yee.push_back( gc );
     }
     *out = plan.release();
     return ZPIC_OK;
@@ -1288,12 +1349,21 @@ int zpic_div_corr_x( float * E, float * B, const zpic_geom * gg, float dx, float
 extern "C" {
 
 int zpic_batch_fields_create( zpic_batch_fields ** out, const zpic_batch_fields_item * items, int n ) {
+    return zpic::batch_fields_new( out, items, n, nullptr );
+}
+
+}  // extern "C"
+
+int zpic::batch_fields_new( zpic_batch_fields ** out, const zpic_batch_fields_item * items, int n,
+                            const float * const * dep ) {
     if ( !out ) return set_error( ZPIC_EINVAL, "null output" );
     BatchFieldPlan * plan = nullptr;
-    if ( int rc = batch_fields_create( &plan, items, n ) ) return rc;
+    if ( int rc = batch_fields_create( &plan, items, n, dep ) ) return rc;
     *out = new zpic_batch_fields{ plan };
     return ZPIC_OK;
 }
+
+extern "C" {
 
 int zpic_batch_zero_current( zpic_batch_fields * b, void * stream ) {
     if ( !b || !b->plan ) return set_error( ZPIC_EINVAL, "null batch" );

@@ -215,15 +215,16 @@ void ParticleSort::grow( uint32_t max_part ) {
     buf.idx = nullptr;
     buf.idx = device_alloc<int>( max_part );
     idx_size = max_part;
-    if ( parts.on ) parts.size = part_size( max_part );
+    if ( parts.on ) parts.size = part_size( max_part, parts.cap - ntiles );
     listed = false;
 }
 
 void ParticleSort::init_parts( uint32_t max_part, int tile_vol ) {
     parts.on = part_rule( ntiles );
     if ( !parts.on ) return;
-    parts.size = part_size( max_part );
-    parts.cap = ntiles + PART_TARGET;
+    const int extra = part_extra( max_part );
+    parts.size = part_size( max_part, extra );
+    parts.cap = ntiles + extra;
     parts.seg = device_alloc<int>( (size_t) PART_SEG * ntiles );
     parts.item = device_alloc<int>( 2 * (size_t) parts.cap );
     parts.total = device_alloc<int>( 1 );
@@ -462,16 +463,41 @@ bool Current::one_pass_ok( std::vector<float> & coef ) const {
     return passes <= 16 && J->nx.x >= gw + passes && J->nx.y >= gw && lds <= 65536;
 }
 
+float * Current::second_buffer() {
+    if ( !Jalt ) {
+        Jalt = new vec3grid<float3>( J->get_ntiles(), J->nx, J->gc );
+        Jalt->name = J->name;
+        Jalt->zero();
+    }
+    return Jalt->fbuf();
+}
+
+float * Current::deposit_buffer() {
+    std::vector<float> coef;
+    return one_pass_ok( coef ) ? second_buffer() : J->fbuf();
+}
+
+void Current::advance_from( const float * dep ) {
+    if ( dep == J->fbuf() ) {
+        advance();
+        return;
+    }
+    std::vector<float> coef;
+    if ( !one_pass_ok( coef ) ) throw std::runtime_error( "(*error*) the current's filter changed during a step" );
+    zpic_geom g = J->geom();
+    const int2 p = J->get_periodic();
+    check( current_update( dep, J->fbuf(), &g, (int) coef.size() / 3, coef.data(), p.x, p.y, stream() ) );
+    iter++;
+    if ( moving_window.needs_move( iter * dt ) ) moving_window.advance();
+}
+
 // Current::advance (current.cpp:227-246)
 void Current::advance() {
     std::vector<float> coef;
     if ( one_pass_ok( coef ) ) {
         // guard add, guard copy and the x filter in one launch into the
         // second buffer, which then becomes J's
-        if ( !Jalt ) {
-            Jalt = new vec3grid<float3>( J->get_ntiles(), J->nx, J->gc );
-            Jalt->name = J->name;
-        }
+        second_buffer();
         zpic_geom g = J->geom();
         const int2 p = J->get_periodic();
         check( current_update( J->fbuf(), Jalt->fbuf(), &g, (int) coef.size() / 3, coef.data(), p.x, p.y, stream() ) );
@@ -863,6 +889,11 @@ void Species::set_staging( zpic_sort & s, bool window ) const {
     s.stage_u = staged ? reinterpret_cast<float *>( tmp->u ) : nullptr;
 }
 
+bool Species::side_by_side() const {
+    const int2 p = particles->periodic;
+    return sort->parts.on && !deterministic && zpic_get_sort_order() == 0 && p.x && p.y && reflect_mask() == 0;
+}
+
 void Species::list_parts() {
     if ( !sort->parts.on || sort->listed ) return;
     check( part_list( particles->np, sort->ntiles, sort->parts, stream() ) );
@@ -1019,6 +1050,7 @@ Simulation::Simulation( uint2 const ntiles_, uint2 const nx_, float2 const box_,
 }
 
 Simulation::~Simulation() {
+    zpic_batch_particles_free( side );
     for ( auto & v : ev )
         for ( auto e : v ) (void) hipEventDestroy( e );
     for ( hipEvent_t e : dep )
@@ -1059,8 +1091,15 @@ void Simulation::set_moving_window() {
 // Stage timing records events in one of TSLOTS slots and reads a slot's
 // elapsed times only when the slot comes round again (or in get_timing()),
 // so that timing adds no host wait per step.
+//
+// Where every species' tiles are taken in parts (small grids), the species
+// run side by side instead, each stage one launch for all of them: at that
+// size a step is a chain of launches of a few microseconds each, and a
+// 128x128 Weibel step of two species took 146 us with a chain per species,
+// 107 us side by side.
 void Simulation::step( bool window ) {
     const size_t nsp = species.size();
+    if ( !window && step_side_by_side() ) return;
     const bool overlap = window && nsp > 0;
     const size_t nev = 2 * nsp + 4;
     const int slot = (int) ( t_ring % TSLOTS );
@@ -1115,6 +1154,66 @@ void Simulation::step( bool window ) {
         t_ring++;
     }
     iter++;
+}
+
+bool Simulation::step_side_by_side() {
+    if ( species.empty() ) return false;
+    for ( auto * s : species )
+        if ( !s->side_by_side() ) return false;
+    float * const dep = current.deposit_buffer();
+    std::vector<const void *> key{ dep, emf.E->fbuf(), emf.B->fbuf(), nullptr };
+    key[3] = reinterpret_cast<const void *>( (uintptr_t) zpic_get_threads_per_tile() );
+    for ( auto * s : species ) s->buffers( key );
+    if ( !side || key != side_key ) {
+        zpic_batch_particles_free( side );
+        side = nullptr;
+        std::vector<zpic_batch_species> items;
+        std::vector<PartScratch> parts;
+        for ( auto * s : species ) {
+            items.push_back( s->batch_item( emf, current ) );
+            items.back().J = dep;
+            parts.push_back( s->part_scratch() );
+        }
+        // tables of the last build may still be read by kernels on the way
+        zpic::hip_check( hipStreamSynchronize( stream() ), "hipStreamSynchronize" );
+        check( batch_particles_new( &side, items.data(), (int) items.size(), zpic_get_threads_per_tile(), parts.data(),
+                                    (int) items.size() ) );
+        side_key = key;
+    }
+    const size_t nsp = species.size(), nev = 2 * nsp + 4;
+    const int slot = (int) ( t_ring % TSLOTS );
+    std::vector<hipEvent_t> & E = ev[slot];
+    auto rec = [&]( size_t i ) {
+        if ( timing ) hip_check( hipEventRecord( E[i], stream() ), "hipEventRecord" );
+    };
+    if ( timing ) {
+        if ( ev_pending[slot] ) accumulate( slot );
+        while ( E.size() < nev ) {
+            hipEvent_t e;
+            hip_check( hipEventCreate( &e ), "hipEventCreate" );
+            E.push_back( e );
+        }
+    }
+    for ( auto * s : species ) s->list_parts();
+    rec( 0 );
+    check( batch_particles_pass( side, stream() ) );
+    rec( 1 );
+    check( batch_particles_sort( side, stream() ) );
+    for ( size_t i = 2; i <= 2 * nsp; i++ ) rec( i );
+    for ( auto * s : species ) s->note_side_by_side();
+    current.advance_from( dep );
+    rec( 2 * nsp + 1 );
+    emf.advance( current );
+    rec( 2 * nsp + 2 );
+    rec( 2 * nsp + 3 );
+    if ( timing ) {
+        ev_pending[slot] = true;
+        ev_overlap[slot] = false;
+        ev_nsp[slot] = nsp;
+        t_ring++;
+    }
+    iter++;
+    return true;
 }
 
 // Stage times of the step recorded in `slot` (waits for its last event):
@@ -1307,7 +1406,31 @@ void Batch::build() {
         bound = buffers();
         return;
     }
-    for ( size_t k = 0; k < nsp; k++ ) {
+    // all instances' tiles in parts: the species side by side, each instance's
+    // current from its deposit buffer
+    bool all = true;
+    for ( auto * s : sims )
+        for ( auto * sp : s->species ) all = all && sp->side_by_side();
+    std::vector<const float *> dep;
+    side_by_side = all;
+    if ( all ) {
+        std::vector<zpic_batch_species> items;
+        std::vector<PartScratch> parts;
+        for ( size_t i = 0; i < sims.size(); i++ ) {
+            Simulation * s = sims[i];
+            dep.push_back( s->current.deposit_buffer() );
+            for ( auto * sp : s->species ) {
+                items.push_back( sp->batch_item( s->emf, s->current ) );
+                items.back().J = const_cast<float *>( dep.back() );
+                items.back().threads = sim_threads[i];
+                parts.push_back( sp->part_scratch() );
+            }
+        }
+        zpic_batch_particles * plan = nullptr;
+        check( batch_particles_new( &plan, items.data(), (int) items.size(), threads, parts.data(), (int) nsp ) );
+        slots.push_back( plan );
+    }
+    for ( size_t k = 0; k < nsp && !all; k++ ) {
         std::vector<zpic_batch_species> items;
         std::vector<PartScratch> parts;
         for ( size_t i = 0; i < sims.size(); i++ ) {
@@ -1322,7 +1445,7 @@ void Batch::build() {
     }
     std::vector<zpic_batch_fields_item> fitems;
     for ( auto * s : sims ) fitems.push_back( s->batch_fields() );
-    check( zpic_batch_fields_create( &fields, fitems.data(), (int) fitems.size() ) );
+    check( batch_fields_new( &fields, fitems.data(), (int) fitems.size(), all ? dep.data() : nullptr ) );
     bound = buffers();
 }
 
@@ -1333,7 +1456,7 @@ void Batch::step_kernels() {
         check( zpic_batch_step_advance( persistent_step, stream() ) );
         return;
     }
-    check( zpic_batch_zero_current( fields, stream() ) );
+    if ( !side_by_side ) check( zpic_batch_zero_current( fields, stream() ) );
     for ( auto * plan : slots ) check( zpic_batch_particles_advance( plan, stream() ) );
     check( zpic_batch_current_advance( fields, stream() ) );
     check( zpic_batch_yee( fields, stream() ) );

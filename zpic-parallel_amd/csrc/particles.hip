@@ -24,6 +24,7 @@
 #include "parts.h"
 
 #include <algorithm>
+#include <cstring>
 #include <memory>
 #include <vector>
 
@@ -412,6 +413,7 @@ struct PartArgs {
     int lbuf;   // order-free sort: leavers buffered in LDS (LDS sized for it)
     int jset;   // fast mode: the tile's J region is written, not added to
     PartScratch parts;  // parts.on (order-free sort): workgroup y takes part y of the list
+    int apart;  // tiles of one part too leave their J to the merge (species that run side by side)
 };
 
 struct PartG {
@@ -866,8 +868,9 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     if constexpr ( MOVE ) {
         // flush: J(tile) += sum of the waves' J (LDS), guard cells included
         // (species.cpp:1488-1492)
-        const gptr<float> Jt = gbl( nparts > 1 ? a.parts.J + (size_t) y * 3 * vol
-                                               : reinterpret_cast<float *>( J + (size_t) t * vol ) );
+        const bool apart = nparts > 1 || a.apart;
+        const gptr<float> Jt = gbl( apart ? a.parts.J + (size_t) y * 3 * vol
+                                          : reinterpret_cast<float *>( J + (size_t) t * vol ) );
         const float bad = ( !DET && s_bad ) ? __builtin_nanf( "" ) : 0.0f;
         for ( int k = tid; k < 3 * g.ext_x * g.ext_y; k += nthr ) {
             const int el = k / 3, c = k - 3 * el;
@@ -880,7 +883,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
             // jset (the first species of a step, fast mode): the region is
             // written instead of zeroed and added to; the same value, since
             // s is never -0
-            if ( !DET && ( a.jset || nparts > 1 ) ) Jt[k] = s;
+            if ( !DET && ( a.jset || apart ) ) Jt[k] = s;
             else Jt[k] += s;
         }
         if ( tid == 0 ) {
@@ -923,6 +926,24 @@ __global__ void __launch_bounds__( FAST_BLOCK ) k_particles( PartArgs a, const P
     particles_tile<PUSH, MOVE, DET>( a, t, smem );
 }
 
+// The direction counts and energies of a tile's parts into the tile's own.
+__device__ inline void part_merge_counts( const PartArgs & a, const int t ) {
+    const gptr<const int> end = gbl( (const int *) a.S.seg ) + PART_SEG * ( t + 1 );
+    const int nparts = end[-SEG_COUNT] & 255, first = end[-SEG_FIRST];
+    if ( nparts < 2 ) return;
+    if ( threadIdx.x < 9 ) {
+        const gptr<const int> m = gbl( (const int *) a.parts.npt ) + 9 * first + threadIdx.x;
+        int s = 0;
+        for ( int p = 0; p < nparts; p++ ) s += m[9 * p];
+        gbl( a.S.npt )[9 * t + threadIdx.x] = s;
+    } else if ( threadIdx.x == 64 ) {
+        const gptr<const double> e = gbl( (const double *) a.parts.energy ) + first;
+        double s = 0.0;
+        for ( int p = 0; p < nparts; p++ ) s += e[p];
+        gbl( a.tile_energy )[t] = s;
+    }
+}
+
 // A tile taken in parts: their J regions, direction counts and energies into
 // the tile's own, in part order (a tile of one part wrote its own).  Slice
 // `slice` of `slices` workgroups of the tile.
@@ -945,24 +966,43 @@ __device__ inline void part_merge_tile( const PartArgs & a, const int t, const i
         }
         Jt[k] = s + sum;
     }
-    if ( slice != 0 ) return;
-    if ( threadIdx.x < 9 ) {
-        const gptr<const int> m = gbl( (const int *) a.parts.npt ) + 9 * first + threadIdx.x;
-        int s = 0;
-        for ( int p = 0; p < nparts; p++ ) s += m[9 * p];
-        gbl( a.S.npt )[9 * t + threadIdx.x] = s;
-    } else if ( threadIdx.x == 64 ) {
-        const gptr<const double> e = gbl( (const double *) a.parts.energy ) + first;
-        double s = 0.0;
-        for ( int p = 0; p < nparts; p++ ) s += e[p];
-        gbl( a.tile_energy )[t] = s;
-    }
+    if ( slice == 0 ) part_merge_counts( a, t );
 }
-
 constexpr int MERGE_BLOCK = 256;
 __global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge( PartArgs a, const PartArgs * tab, const int2 * map ) {
     const int t = select_instance( a, tab, map );
     if ( a.parts.on ) part_merge_tile( a, t, blockIdx.y, gridDim.y );
+}
+
+// The same for the `group` species of an instance that ran side by side:
+// their J regions, species after species, are the tile's J (map: workgroup ->
+// (instance, tile); entries instance * group ...).
+__global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge_group( const PartArgs * tab, const int2 * map, int group ) {
+    const int2 r = gbl( map )[blockIdx.x];
+    const int t = r.y;
+    const PartArgs * const e = tab + r.x * group;
+    const int vol3 = 3 * e[0].g.vol, n = 3 * e[0].g.ext_x * e[0].g.ext_y;
+    const gptr<float> Jt = gbl( reinterpret_cast<float *>( e[0].J ) ) + (size_t) t * vol3;
+    for ( int k = blockIdx.y * blockDim.x + threadIdx.x; k < n; k += gridDim.y * blockDim.x ) {
+        float total = 0.0f;
+        for ( int g = 0; g < group; g++ ) {
+            const gptr<const int> end = gbl( (const int *) e[g].S.seg ) + PART_SEG * ( t + 1 );
+            const int nparts = end[-SEG_COUNT] & 255;
+            const gptr<const float> src = gbl( (const float *) e[g].parts.J ) + (size_t) end[-SEG_FIRST] * vol3 + k;
+            float sum = 0.0f;
+            for ( int p = 0; p < nparts; p += MERGE_LOADS ) {
+                float v[MERGE_LOADS];
+#pragma unroll
+                for ( int i = 0; i < MERGE_LOADS; i++ ) v[i] = p + i < nparts ? src[(size_t) ( p + i ) * vol3] : 0.0f;
+#pragma unroll
+                for ( int i = 0; i < MERGE_LOADS; i++ ) sum += v[i];
+            }
+            total = g == 0 ? sum : total + sum;
+        }
+        Jt[k] = total;
+    }
+    if ( blockIdx.y == 0 )
+        for ( int g = 0; g < group; g++ ) part_merge_counts( gbl( tab )[r.x * group + g], t );
 }
 // workgroups per tile: a tile's elements over several where the tiles are few
 int merge_slices( int ntiles ) { return ntiles <= 256 ? 4 : 1; }
@@ -2028,6 +2068,18 @@ int check_threads( int threads ) {
     return ZPIC_OK;
 }
 
+// Whether the leaver buffers cost no workgroup per CU, or leave four, with
+// which the pass already runs at its memory rate (three buffers more or less
+// measured the same).
+bool lbuf_fits( size_t without, size_t with ) {
+    int dev = 0, cu_lds = 0;
+    if ( hipGetDevice( &dev ) != hipSuccess ||
+         hipDeviceGetAttribute( &cu_lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev ) != hipSuccess )
+        return false;
+    const size_t stat = 256;  // the kernel's static LDS, rounded up
+    return cu_lds / ( with + stat ) >= std::min( (size_t) 4, cu_lds / ( without + stat ) );
+}
+
 // Tiles in parts need the order-free sort (its segment table).
 bool parts_on( const SortView & S, const PartScratch * parts ) { return parts && parts->on && S.stage_ix; }
 void use_parts( PartArgs & a, const PartScratch * parts ) {
@@ -2057,13 +2109,8 @@ int launch_particles( const zpic_particles * p, const zpic_geom * fld, const flo
     a.alpha = alpha; a.m = m; a.tile_energy = tile_energy; a.S = view( s );
     a.jset = MOVE && !det && jset;
     if ( MOVE && !det && s->stage_ix ) {
-        // the leaver buffers, where they cost no workgroup per CU
         const size_t with = particles_lds_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE, true );
-        int dev = 0, cu_lds = 0;
-        ZPIC_HIP_TRY( hipGetDevice( &dev ) );
-        ZPIC_HIP_TRY( hipDeviceGetAttribute( &cu_lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev ) );
-        const size_t stat = 256;  // the kernel's static LDS, rounded up
-        if ( cu_lds / ( with + stat ) >= std::min( (size_t) 4, cu_lds / ( lds + stat ) ) ) {
+        if ( lbuf_fits( lds, with ) ) {
             a.lbuf = 1;
             lds = with;
         }
@@ -2117,32 +2164,39 @@ struct BatchParticlePlan {
     int threads = FAST_BLOCK;  // workgroup size: the largest of the entries' fitted threads
     size_t lds = 0;            // the largest of the entries' LDS needs
     bool staged = false;       // every entry uses the order-free sort
+    char * tables = nullptr;   // the allocation of the tables below
     PartArgs * d_part = nullptr;
     SortArgs * d_sort = nullptr;
     int2 * d_map = nullptr;    // block -> (entry, tile)
     int2 * d_items = nullptr;  // particle pass: block -> (entry, part of a tile)
     int nitems = 0;
+    int group = 0;             // species that run side by side (0: one plan per species)
+    int2 * d_inst = nullptr;   // group > 0: block -> (instance, tile)
+    int ninst = 0;             // its length
     EnergyArgs * d_energy = nullptr;  // [nentries]
     std::vector<PartArgs> h_part;
 };
 
 void batch_particles_destroy( BatchParticlePlan * plan ) {
     if ( !plan ) return;
-    (void) hipFree( plan->d_part ); (void) hipFree( plan->d_sort ); (void) hipFree( plan->d_map );
-    (void) hipFree( plan->d_items ); (void) hipFree( plan->d_energy );
+    (void) hipFree( plan->tables );
     delete plan;
 }
 
 int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species * items, int n, int threads,
-                            const PartScratch * parts ) {
+                            const PartScratch * parts, int group ) {
     if ( !out || !items || n < 1 ) return set_error( ZPIC_EINVAL, "empty batch" );
+    if ( group < 0 || ( group > 0 && ( !parts || n % group ) ) ) return set_error( ZPIC_EINVAL, "invalid species group" );
     if ( int rc = check_threads( threads ) ) return rc;
     auto * plan = new BatchParticlePlan();
     plan->threads = WAVE;
     plan->nentries = n;
     std::vector<SortArgs> sorts( n );
     std::vector<EnergyArgs> energies( n );
-    std::vector<int2> map, pmap;
+    std::vector<int2> map, pmap, inst;
+    plan->group = group;
+    bool lbuf = true;
+    size_t lds_with = 0;
     for ( int e = 0; e < n; e++ ) {
         const zpic_batch_species & it = items[e];
         if ( int rc = check_geom( &it.fld ) ) { delete plan; return rc; }
@@ -2154,6 +2208,11 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
         zpic_sort s = it.s;
         a.S = view( &s );
         use_parts( a, parts ? parts + e : nullptr );
+        a.apart = group > 0;
+        if ( group > 0 && !a.parts.on ) {
+            delete plan;
+            return set_error( ZPIC_EINVAL, "species side by side need their tiles in parts" );
+        }
         // each entry runs with the threads that fit its own tiles, as its own
         // single-instance pass does
         if ( it.threads && check_threads( it.threads ) ) { delete plan; return ZPIC_EINVAL; }
@@ -2161,7 +2220,11 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
         if ( th == 0 ) { delete plan; return set_error( ZPIC_ERANGE, "tile too large for LDS staging" ); }
         a.waves = th / WAVE;
         plan->threads = std::max( plan->threads, th );
-        plan->lds = std::max( plan->lds, particles_lds_bytes( it.fld.tile_vol, a.waves, true, true ) );
+        const size_t lds = particles_lds_bytes( it.fld.tile_vol, a.waves, true, true );
+        const size_t with = particles_lds_bytes( it.fld.tile_vol, a.waves, true, true, true );
+        lbuf = lbuf && it.s.stage_ix && lbuf_fits( lds, with );
+        plan->lds = std::max( plan->lds, lds );
+        lds_with = std::max( lds_with, with );
         plan->h_part.push_back( a );
         zpic_particles p = it.p, t = it.tmp;
         sorts[e] = sort_args( &p, &t, &s, it.fld.ntiles_x, it.fld.ntiles_y, it.fld.nx, it.fld.ny, it.periodic_x,
@@ -2169,12 +2232,17 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
         const int nt = it.fld.ntiles_x * it.fld.ntiles_y;
         energies[e] = EnergyArgs{ it.tile_energy, nt, it.energy_out };
         for ( int t2 = 0; t2 < nt; t2++ ) map.push_back( make_int2( e, t2 ) );
+        if ( group > 0 && e % group == 0 )
+            for ( int t2 = 0; t2 < nt; t2++ ) inst.push_back( make_int2( e / group, t2 ) );
         for ( int y = 0; y < ( a.parts.on ? a.parts.cap : nt ); y++ ) pmap.push_back( make_int2( e, y ) );
         plan->max_tiles = std::max( plan->max_tiles, nt );
         plan->max_vol = std::max( plan->max_vol, it.fld.tile_vol );
     }
     plan->nblocks = (int) map.size();
     plan->nitems = (int) pmap.size();
+    plan->ninst = (int) inst.size();
+    if ( lbuf ) plan->lds = lds_with;
+    for ( PartArgs & a : plan->h_part ) a.lbuf = lbuf;
     {
         int nst = 0;
         for ( int e = 0; e < n; e++ ) nst += items[e].s.stage_ix != nullptr;
@@ -2184,20 +2252,35 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
         }
         plan->staged = nst == n;
     }
-    hipError_t e1 = hipMalloc( (void **) &plan->d_part, sizeof( PartArgs ) * n );
-    hipError_t e2 = hipMalloc( (void **) &plan->d_sort, sizeof( SortArgs ) * n );
-    hipError_t e3 = hipMalloc( (void **) &plan->d_map, sizeof( int2 ) * map.size() );
-    hipError_t e4 = hipMalloc( (void **) &plan->d_energy, sizeof( EnergyArgs ) * n );
-    hipError_t e5 = hipMalloc( (void **) &plan->d_items, sizeof( int2 ) * pmap.size() );
-    if ( e1 || e2 || e3 || e4 || e5 ) {
-        batch_particles_destroy( plan );
+    // all tables in one allocation, copied at once
+    std::vector<char> host;
+    auto place = [&]( const void * src, size_t bytes ) {
+        const size_t at = host.size();
+        host.resize( at + ( ( bytes + 255 ) & ~(size_t) 255 ) );
+        std::memcpy( host.data() + at, src, bytes );
+        return at;
+    };
+    const size_t o1 = place( plan->h_part.data(), sizeof( PartArgs ) * n );
+    const size_t o2 = place( sorts.data(), sizeof( SortArgs ) * n );
+    const size_t o3 = place( map.data(), sizeof( int2 ) * map.size() );
+    const size_t o4 = place( energies.data(), sizeof( EnergyArgs ) * n );
+    const size_t o5 = place( pmap.data(), sizeof( int2 ) * pmap.size() );
+    const size_t o6 = inst.empty() ? 0 : place( inst.data(), sizeof( int2 ) * inst.size() );
+    if ( hipMalloc( (void **) &plan->tables, host.size() ) != hipSuccess ) {
+        delete plan;
         return set_error( ZPIC_EHIP, "hipMalloc failed for batch tables" );
     }
-    ZPIC_HIP_TRY( hipMemcpy( plan->d_part, plan->h_part.data(), sizeof( PartArgs ) * n, hipMemcpyHostToDevice ) );
-    ZPIC_HIP_TRY( hipMemcpy( plan->d_sort, sorts.data(), sizeof( SortArgs ) * n, hipMemcpyHostToDevice ) );
-    ZPIC_HIP_TRY( hipMemcpy( plan->d_map, map.data(), sizeof( int2 ) * map.size(), hipMemcpyHostToDevice ) );
-    ZPIC_HIP_TRY( hipMemcpy( plan->d_items, pmap.data(), sizeof( int2 ) * pmap.size(), hipMemcpyHostToDevice ) );
-    ZPIC_HIP_TRY( hipMemcpy( plan->d_energy, energies.data(), sizeof( EnergyArgs ) * n, hipMemcpyHostToDevice ) );
+    const hipError_t err = hipMemcpy( plan->tables, host.data(), host.size(), hipMemcpyHostToDevice );
+    if ( err != hipSuccess ) {
+        batch_particles_destroy( plan );
+        return hip_error( err, "batch tables" );
+    }
+    plan->d_part = (PartArgs *) ( plan->tables + o1 );
+    plan->d_sort = (SortArgs *) ( plan->tables + o2 );
+    plan->d_map = (int2 *) ( plan->tables + o3 );
+    plan->d_energy = (EnergyArgs *) ( plan->tables + o4 );
+    plan->d_items = (int2 *) ( plan->tables + o5 );
+    plan->d_inst = inst.empty() ? nullptr : (int2 *) ( plan->tables + o6 );
     *out = plan;
     return ZPIC_OK;
 }
@@ -2229,17 +2312,26 @@ int batch_particles_place( BatchParticlePlan * plan, hipStream_t st ) {
     return ZPIC_OK;
 }
 
-int batch_particles_step( BatchParticlePlan * plan, void * stream ) {
+int batch_particles_pass( BatchParticlePlan * plan, void * stream ) {
     hipStream_t st = as_stream( stream );
     PartArgs dummy{};
     hipLaunchKernelGGL( ( k_particles<true, true, false> ), dim3( plan->nitems ), dim3( plan->threads ), plan->lds, st,
                         dummy, (const PartArgs *) plan->d_part, (const int2 *) plan->d_items );
     ZPIC_LAUNCH_CHECK( "k_particles (batch)" );
-    if ( plan->nitems > plan->nblocks ) {
+    if ( plan->group > 0 ) {
+        hipLaunchKernelGGL( k_part_merge_group, dim3( plan->ninst, merge_slices( plan->ninst ) ), dim3( MERGE_BLOCK ), 0, st,
+                            (const PartArgs *) plan->d_part, (const int2 *) plan->d_inst, plan->group );
+        ZPIC_LAUNCH_CHECK( "k_part_merge_group" );
+    } else if ( plan->nitems > plan->nblocks ) {
         hipLaunchKernelGGL( k_part_merge, dim3( plan->nblocks, merge_slices( plan->nblocks ) ), dim3( MERGE_BLOCK ), 0, st, dummy,
                             (const PartArgs *) plan->d_part, (const int2 *) plan->d_map );
         ZPIC_LAUNCH_CHECK( "k_part_merge (batch)" );
     }
+    return ZPIC_OK;
+}
+
+int batch_particles_sort( BatchParticlePlan * plan, void * stream ) {
+    hipStream_t st = as_stream( stream );
     SortArgs sd{};
     if ( plan->max_tiles <= SCAN_BLOCK ) {
         hipLaunchKernelGGL( k_sort_plan, dim3( plan->nentries ), dim3( SCAN_BLOCK ), 0, st, sd,
@@ -3199,16 +3291,16 @@ struct zpic_batch_particles {
 
 int zpic_batch_particles_create( zpic_batch_particles ** out, const zpic_batch_species * items, int n,
                                  int threads_per_tile ) {
-    return zpic::batch_particles_new( out, items, n, threads_per_tile, nullptr );
+    return zpic::batch_particles_new( out, items, n, threads_per_tile, nullptr, 0 );
 }
 
 }  // extern "C"
 
 int zpic::batch_particles_new( zpic_batch_particles ** out, const zpic_batch_species * items, int n,
-                               int threads_per_tile, const PartScratch * parts ) {
+                               int threads_per_tile, const PartScratch * parts, int group ) {
     if ( !out ) return set_error( ZPIC_EINVAL, "null output" );
     BatchParticlePlan * plan = nullptr;
-    if ( int rc = batch_particles_create( &plan, items, n, threads_per_tile, parts ) ) return rc;
+    if ( int rc = batch_particles_create( &plan, items, n, threads_per_tile, parts, group ) ) return rc;
     *out = new zpic_batch_particles{ plan };
     return ZPIC_OK;
 }
@@ -3217,8 +3309,16 @@ extern "C" {
 
 int zpic_batch_particles_advance( zpic_batch_particles * b, void * stream ) {
     if ( !b || !b->plan ) return set_error( ZPIC_EINVAL, "null batch" );
-    return batch_particles_step( b->plan, stream );
+    if ( int rc = batch_particles_pass( b->plan, stream ) ) return rc;
+    return batch_particles_sort( b->plan, stream );
 }
+
+}  // extern "C"
+
+int zpic::batch_particles_pass( zpic_batch_particles * b, void * stream ) { return batch_particles_pass( b->plan, stream ); }
+int zpic::batch_particles_sort( zpic_batch_particles * b, void * stream ) { return batch_particles_sort( b->plan, stream ); }
+
+extern "C" {
 
 void zpic_batch_particles_free( zpic_batch_particles * b ) {
     if ( !b ) return;

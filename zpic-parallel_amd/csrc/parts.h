@@ -22,13 +22,13 @@ namespace zpic {
 constexpr int PART_SEG = 64;      // ints per tile of the segment table
 constexpr int PART_MAX_SEG = 59;  // wave segments of one tile
 constexpr int PART_MAX = 14;
-constexpr int PART_TARGET = 1024;  // parts beyond one per tile, at most
-constexpr unsigned PART_MIN = 1024;
+constexpr unsigned PART_TARGET = 1024;  // parts beyond one per tile, at most
+constexpr unsigned PART_MIN = 1024;     // particles of a part, at least
 
 struct PartScratch {
     int on = 0;    // 0: tiles are not cut, the rest is unused
     int size = 0;  // particles of a part
-    int cap = 0;   // most parts of all tiles: ntiles + PART_TARGET
+    int cap = 0;   // most parts of all tiles: ntiles + part_extra
     int * seg = nullptr;    // [PART_SEG * ntiles] segment tables
     int * item = nullptr;   // [2 * cap] the parts: tile, part | parts of the tile << 8
     int * total = nullptr;  // [1] their number
@@ -41,13 +41,14 @@ struct PartScratch {
 // crowded tile bounds the pass: up to 1024 tiles, one workgroup each on the
 // device at once.
 inline bool part_rule( int ntiles ) { return ntiles <= 1024; }
-// Particles of a part for a buffer of max_part: no more than PART_TARGET parts
-// beyond one per tile, and no fewer than PART_MIN particles, which take a
+// Parts beyond one per tile for a buffer of max_part particles, and the
+// particles of a part that keep to them: no fewer than PART_MIN, which take a
 // workgroup about as long as its staging and its J region.  (512 and 2048
 // parts measured within 3 % on these runs, 4096 of at least 256 particles up
 // to 15 % slower on a 512x512 grid.)
-inline int part_size( unsigned max_part ) {
-    return (int) std::max( PART_MIN, ( max_part / PART_TARGET + 64 ) & ~63u );
+inline int part_extra( unsigned max_part ) { return (int) std::min( PART_TARGET, max_part / PART_MIN + 1 ); }
+inline int part_size( unsigned max_part, int extra ) {
+    return (int) std::max( PART_MIN, ( max_part / (unsigned) extra + 64 ) & ~63u );
 }
 
 // The list of parts for the tiles' particle counts np[ntiles].
@@ -64,8 +65,14 @@ int tile_sort_count( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, in
                      const double * tile_energy, double * energy, void * stream );
 int tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int ntiles_x, int ntiles_y, int nx, int ny,
                     int periodic_x, int periodic_y, int mode, const PartScratch * parts, void * stream );
+// group > 0: the n items are the species of n / group instances, `group` of
+// each side by side, all in parts, and go through each stage together; J is
+// written, not added to.
 int batch_particles_new( zpic_batch_particles ** out, const zpic_batch_species * items, int n, int threads_per_tile,
-                         const PartScratch * parts );
+                         const PartScratch * parts, int group = 0 );
+// zpic_batch_particles_advance in its two halves.
+int batch_particles_pass( zpic_batch_particles * plan, void * stream );
+int batch_particles_sort( zpic_batch_particles * plan, void * stream );
 int batch_step_new( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
                     const zpic_batch_fields_item * fields, int n, int threads_per_tile, const PartScratch * parts );
 

@@ -553,6 +553,7 @@ class Current {
     vec3grid<float3> * Jalt;
     // whether advance() may run as one pass, and the filter's x passes
     bool one_pass_ok( std::vector<float> & coef ) const;
+    float * second_buffer();
 
   public:
     vec3grid<float3> * J;
@@ -571,6 +572,11 @@ class Current {
         filter = new_filter.clone();
     }
     void advance();
+    // For a caller that writes the whole deposit itself: the buffer to write it
+    // to (J's own where advance() does not run as one pass), and advance() from
+    // there, which leaves J where it is.
+    float * deposit_buffer();
+    void advance_from( const float * dep );
     void zero();
     // Current::set_moving_window (current.h:123-136): 0, or -1 after the first step
     int set_moving_window();
@@ -758,6 +764,13 @@ class Species {
     // Arguments of this species for a batched advance with the given fields
     zpic_batch_species batch_item( EMF const & emf, Current & current ) const;
     zpic::PartScratch part_scratch() const { return sort->parts; }
+    // Whether a step's particle pass may run beside other species' (tiles in
+    // parts, order-free sort, no walls), and what such a step leaves behind.
+    bool side_by_side() const;
+    void note_side_by_side() {
+        sort->in_parts = true;
+        note_step();
+    }
     // The list of parts, where the particle counts changed by other means than
     // a sort that wrote it.
     void list_parts();
@@ -790,6 +803,11 @@ class Simulation {
     double t_acc[5];
     long long t_steps;
     void accumulate( int slot );
+    // particle passes of all species side by side: the launch tables and the
+    // buffers they were built on
+    zpic_batch_particles * side = nullptr;
+    std::vector<const void *> side_key;
+    bool step_side_by_side();
 
   public:
     const uint2 ntiles;
@@ -852,6 +870,7 @@ class Batch {
     int threads;
     bool use_graph;
     bool persistent;
+    bool side_by_side = false;  // one plan for all species
     hipGraph_t graph;
     hipGraphExec_t exec;
     std::vector<const void *> bound;  // device buffers the tables were built on
