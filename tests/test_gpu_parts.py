@@ -25,8 +25,10 @@ def crowded(ntiles, nx, counts, seed):
     ((3, 2), (8, 8), 256, [0, 1, 1023, 1024, 1025, 2048]),
     ((3, 2), (8, 8), 64, [2049, 0, 14 * 1024, 64, 16000, 3]),
     ((2, 2), (32, 32), 512, [30000, 1, 0, 1100]),
-    ((33, 32), (8, 8), 256, [3] * 1055 + [5000]),   # more tiles than the cut is used for
+    ((33, 32), (8, 8), 256, [3] * 1055 + [5000]),   # more than one tile per thread of the scan
     ((32, 32), (8, 8), 256, [1] * 1000 + [0] * 23 + [9000]),
+    ((64, 64), (4, 4), 256, [2] * 4090 + [0] * 5 + [3000]),
+    ((241, 17), (4, 5), 256, [1] * 4096 + [3000]),  # more tiles than the cut is used for
 ])
 def test_crowded_tiles(ntiles, nx, threads, counts):
     import pyzpic as zp

@@ -1229,17 +1229,18 @@ __device__ inline void batch_energy_body( const EnergyArgs & a ) {
     __syncthreads();  // s_wsum may be reused by the next body in the workgroup
 }
 
-// New counts, offsets and the push energy of an instance of at most
-// SCAN_BLOCK tiles, a thread per tile: three launches' work in one.  (With
-// more tiles the nine counts each tile gathers are too many for one
-// workgroup.)
+// New counts, offsets and the push energy of an instance of at most PLAN_TILES
+// tiles, K tiles per thread: three launches' work in one.  (With more tiles
+// the nine counts each tile gathers are too many for one workgroup.)
+constexpr int PLAN_TILES = 4 * SCAN_BLOCK;
+template <int K>
 __global__ void __launch_bounds__( SCAN_BLOCK ) k_sort_plan( SortArgs a, const SortArgs * tab, EnergyArgs e,
                                                              const EnergyArgs * etab ) {
     if ( tab ) {
         a = gbl( tab )[blockIdx.x];
         e = gbl( etab )[blockIdx.x];
     }
-    sort_count_body<SCAN_BLOCK, false, 1, true>( a );
+    sort_count_body<SCAN_BLOCK, false, K, true>( a );
     if ( e.tile ) batch_energy_body( e );
 }
 
@@ -2333,9 +2334,10 @@ int batch_particles_pass( BatchParticlePlan * plan, void * stream ) {
 int batch_particles_sort( BatchParticlePlan * plan, void * stream ) {
     hipStream_t st = as_stream( stream );
     SortArgs sd{};
-    if ( plan->max_tiles <= SCAN_BLOCK ) {
-        hipLaunchKernelGGL( k_sort_plan, dim3( plan->nentries ), dim3( SCAN_BLOCK ), 0, st, sd,
-                            (const SortArgs *) plan->d_sort, EnergyArgs{}, (const EnergyArgs *) plan->d_energy );
+    if ( plan->max_tiles <= PLAN_TILES ) {
+        hipLaunchKernelGGL( plan->max_tiles <= SCAN_BLOCK ? k_sort_plan<1> : k_sort_plan<4>, dim3( plan->nentries ),
+                            dim3( SCAN_BLOCK ), 0, st, sd, (const SortArgs *) plan->d_sort, EnergyArgs{},
+                            (const EnergyArgs *) plan->d_energy );
         ZPIC_LAUNCH_CHECK( "k_sort_plan (batch)" );
         return batch_particles_place( plan, st );
     }
@@ -3179,9 +3181,9 @@ int zpic::tile_sort_count( zpic_particles * p, zpic_particles * tmp, zpic_sort *
     a.extra = extra;
     const SortArgs * tab = nullptr;
     hipStream_t st = as_stream( stream );
-    if ( nt <= SCAN_BLOCK ) {
+    if ( nt <= PLAN_TILES ) {
         const EnergyArgs e{ tile_energy, nt, energy }, * etab = nullptr;
-        hipLaunchKernelGGL( k_sort_plan, dim3( 1 ), dim3( SCAN_BLOCK ), 0, st, a, tab, e, etab );
+        hipLaunchKernelGGL( nt <= SCAN_BLOCK ? k_sort_plan<1> : k_sort_plan<4>, dim3( 1 ), dim3( SCAN_BLOCK ), 0, st, a, tab, e, etab );
         ZPIC_LAUNCH_CHECK( "k_sort_plan" );
         return ZPIC_OK;
     }

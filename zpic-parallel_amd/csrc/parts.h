@@ -37,10 +37,14 @@ struct PartScratch {
     float * J = nullptr;        // [3 * tile_vol * cap]
 };
 
-// Worth its two launches (the merge, about 5 us, and the list) where one
-// crowded tile bounds the pass: up to 1024 tiles, one workgroup each on the
-// device at once.
-inline bool part_rule( int ntiles ) { return ntiles <= 1024; }
+// Up to 4096 tiles, whose counts one workgroup still scans in one launch and
+// where a crowded tile or a chain of launches per species shows: a step of
+// 1056x720 cells in 1485 tiles 263 -> 213 us, of 768x640 in 1920 tiles at 64
+// particles per cell 1502 -> 1195, of 1024x1024 in 4096 tiles at 16 783 -> 716,
+// at one 232 -> 202 us.  Beyond, the passes fill the device by themselves and
+// the J regions of the parts would be written and read for every tile.
+inline bool part_rule( int ntiles ) { return ntiles <= 4096; }
+
 // Parts beyond one per tile for a buffer of max_part particles, and the
 // particles of a part that keep to them: no fewer than PART_MIN, which take a
 // workgroup about as long as its staging and its J region.  (512 and 2048
