@@ -247,3 +247,23 @@ def test_batch_after_single_steps_matches_single_instances(zp, persistent):
             s.close()
     finally:
         zp.set_threads_per_tile(old)
+
+
+@pytest.mark.parametrize("shape", [
+    dict(ntiles=(3, 3), nx=(16, 16), ppc=(2, 2), filter=("binomial", 0, 5)),     # the most passes held in registers
+    dict(ntiles=(3, 2), nx=(16, 16), ppc=(2, 2), filter=("compensated", 0, 5)),  # one more
+    dict(ntiles=(65, 64), nx=(8, 8), ppc=(1, 1), filter=("binomial", 0, 2)),     # more tiles than are cut
+    dict(ntiles=(2, 2), nx=(4, 4), ppc=(4, 4), filter=("binomial", 0, 4)),       # narrower than the one-stage update takes
+])
+def test_persistent_current_from_deposit(zp, shape):
+    """The persistent step's current, formed from the deposit buffer in one
+    stage where the tiles and the filter allow."""
+    sims = [make(zp, shape) for _ in range(2)]
+    batch = zp.Batch(sims[:1], threads_per_tile=256, graph=False, persistent=True)
+    sims[1].advance(5)
+    batch.advance(5)
+    batch.status()
+    assert_same(state(sims[0]), state(sims[1]), str(shape))
+    batch.close()
+    for s in sims:
+        s.close()

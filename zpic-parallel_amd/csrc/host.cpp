@@ -1400,9 +1400,13 @@ void Batch::build() {
                 parts.push_back( s->species[k]->part_scratch() );
             }
         std::vector<zpic_batch_fields_item> fitems;
-        for ( auto * s : sims ) fitems.push_back( s->batch_fields() );
+        std::vector<const float *> dep;
+        for ( auto * s : sims ) {
+            fitems.push_back( s->batch_fields() );
+            dep.push_back( s->current.deposit_buffer() );
+        }
         check( batch_step_new( &persistent_step, items.data(), (int) nsp, fitems.data(), (int) fitems.size(), threads,
-                               parts.data() ) );
+                               parts.data(), dep.data() ) );
         bound = buffers();
         return;
     }

@@ -974,21 +974,20 @@ __global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge( PartArgs a, const
     if ( a.parts.on ) part_merge_tile( a, t, blockIdx.y, gridDim.y );
 }
 
-// The same for the `group` species of an instance that ran side by side:
-// their J regions, species after species, are the tile's J (map: workgroup ->
-// (instance, tile); entries instance * group ...).
-__global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge_group( const PartArgs * tab, const int2 * map, int group ) {
-    const int2 r = gbl( map )[blockIdx.x];
-    const int t = r.y;
-    const PartArgs * const e = tab + r.x * group;
+// The same for the `group` species of an instance that ran side by side
+// (entries e[0], e[stride], ...): their J regions, species after species, are
+// the tile's J.
+__device__ inline void part_merge_group( const PartArgs * const e, const int stride, const int group, const int t,
+                                         const int slice, const int slices ) {
     const int vol3 = 3 * e[0].g.vol, n = 3 * e[0].g.ext_x * e[0].g.ext_y;
     const gptr<float> Jt = gbl( reinterpret_cast<float *>( e[0].J ) ) + (size_t) t * vol3;
-    for ( int k = blockIdx.y * blockDim.x + threadIdx.x; k < n; k += gridDim.y * blockDim.x ) {
+    for ( int k = slice * blockDim.x + threadIdx.x; k < n; k += slices * blockDim.x ) {
         float total = 0.0f;
         for ( int g = 0; g < group; g++ ) {
-            const gptr<const int> end = gbl( (const int *) e[g].S.seg ) + PART_SEG * ( t + 1 );
+            const PartArgs & a = e[g * stride];
+            const gptr<const int> end = gbl( (const int *) a.S.seg ) + PART_SEG * ( t + 1 );
             const int nparts = end[-SEG_COUNT] & 255;
-            const gptr<const float> src = gbl( (const float *) e[g].parts.J ) + (size_t) end[-SEG_FIRST] * vol3 + k;
+            const gptr<const float> src = gbl( (const float *) a.parts.J ) + (size_t) end[-SEG_FIRST] * vol3 + k;
             float sum = 0.0f;
             for ( int p = 0; p < nparts; p += MERGE_LOADS ) {
                 float v[MERGE_LOADS];
@@ -1001,8 +1000,13 @@ __global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge_group( const PartA
         }
         Jt[k] = total;
     }
-    if ( blockIdx.y == 0 )
-        for ( int g = 0; g < group; g++ ) part_merge_counts( gbl( tab )[r.x * group + g], t );
+    if ( slice == 0 )
+        for ( int g = 0; g < group; g++ ) part_merge_counts( gbl( e )[g * stride], t );
+}
+// map: workgroup -> (instance, tile); entries instance * group ...
+__global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge_group( const PartArgs * tab, const int2 * map, int group ) {
+    const int2 r = gbl( map )[blockIdx.x];
+    part_merge_group( tab + r.x * group, 1, group, r.y, blockIdx.y, gridDim.y );
 }
 // workgroups per tile: a tile's elements over several where the tiles are few
 int merge_slices( int ntiles ) { return ntiles <= 256 ? 4 : 1; }
@@ -2372,6 +2376,8 @@ enum StepKind : int {
     SK_ZERO = 0,  // Current::zero of tiles [t0, t1)
     SK_PART,      // particle pass of items [t0, t1) (tiles, or parts of them), one after the other
     SK_MERGE,     // J regions and counts of tiles taken in parts (tiles [t0, t1))
+    SK_MERGE_ALL, // the same of all species of an instance that ran side by side
+    SK_CURRENT,   // Current::advance from the instance's deposit buffer (tiles [t0, t1))
     SK_NEWNP,     // new per-tile counts of tiles [t0, t1)
     SK_COUNT,     // offsets scan, nmove and push energy of the species
     SK_SHIFT,     // order-free sort: stayers outside the new range staged (tiles [t0, t1))
@@ -2406,6 +2412,8 @@ struct StepTables {
     const PartArgs * part;
     const SortArgs * sort;
     const EnergyArgs * energy;
+    int n, nslots;  // instances, species of each: entry slot * n + instance of part, sort and energy
+    const grid_ops::CurArgs * cur;
     const grid_ops::GcArgs * gc;
     const grid_ops::K3Args * k3;
     const grid_ops::YeeArgs * yee;
@@ -2528,6 +2536,25 @@ __global__ void __launch_bounds__( BLOCK, 4 ) k_batch_step( StepTables T ) {
         case SK_MERGE: {
             const PartArgs a = uniform_load( T.part + it.arg );
             for ( int t = it.t0; t < it.t1; t++ ) part_merge_tile( a, t, 0, 1 );
+            break;
+        }
+        case SK_MERGE_ALL:
+            for ( int t = it.t0; t < it.t1; t++ ) part_merge_group( T.part + it.arg, T.n, T.nslots, t, 0, 1 );
+            break;
+        case SK_CURRENT: {
+            const grid_ops::CurArgs & a = T.cur[it.arg];
+            for ( int t = it.t0; t < it.t1; t++ ) {
+                if ( t > it.t0 ) __syncthreads();
+                switch ( a.passes ) {
+                case 0: grid_ops::current_tile<0>( a, t, smem ); break;
+                case 1: grid_ops::current_tile<1>( a, t, smem ); break;
+                case 2: grid_ops::current_tile<2>( a, t, smem ); break;
+                case 3: grid_ops::current_tile<3>( a, t, smem ); break;
+                case 4: grid_ops::current_tile<4>( a, t, smem ); break;
+                case 5: grid_ops::current_tile<5>( a, t, smem ); break;
+                default: grid_ops::current_tile<-1>( a, t, smem ); break;
+                }
+            }
             break;
         }
         case SK_NEWNP: {
@@ -2653,7 +2680,7 @@ std::vector<FilterPass> filter_passes( const zpic_batch_fields_item & it ) {
 }
 
 int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int nslots, const zpic_batch_fields_item * fl,
-                       int n, int threads, const PartScratch * parts ) {
+                       int n, int threads, const PartScratch * parts, const float * const * dep ) {
     if ( !out || !sp || !fl || n < 1 || nslots < 1 ) return set_error( ZPIC_EINVAL, "empty batch" );
     if ( int rc = check_threads( threads ) ) return rc;
     auto plan = std::make_unique<BatchStepPlan>();
@@ -2703,6 +2730,13 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     std::vector<PartArgs> part( (size_t) nslots * n );
     std::vector<SortArgs> sort( (size_t) nslots * n );
     std::vector<EnergyArgs> ener( (size_t) nslots * n );
+    std::vector<grid_ops::CurArgs> cur( n );
+    // instances that deposit into dep[i], the current formed from it in one
+    // stage (2 + 2 * (filter passes) stages fewer; not where that stage would
+    // need more LDS than the particle pass takes), and of these the ones whose
+    // species run side by side, tiles in parts, their J regions merged into
+    // dep[i] (2 * species - 1 stages fewer)
+    std::vector<char> direct( n, 0 ), apart( n, 0 );
     std::vector<grid_ops::GcArgs> gc( 3 * (size_t) n );
     std::vector<grid_ops::YeeArgs> yee( n );
     std::vector<grid_ops::K3Args> k3;
@@ -2718,6 +2752,27 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
         yee[i] = grid_ops::YeeArgs{ f.E, f.B, f.J, g, f.dt_dx, f.dt_dy, f.dt };
         passes[i] = filter_passes( f );
         max_passes = std::max( max_passes, passes[i].size() );
+        if ( dep && dep[i] && dep[i] != f.J && passes[i].size() <= (size_t) grid_ops::CUR_MAX_PASSES &&
+             grid_ops::current_lds_bytes( g, (int) passes[i].size() ) <=
+                 particles_lds_bytes( f.g.tile_vol, waves[i], true, true ) ) {
+            direct[i] = apart[i] = 1;
+            for ( int k = 0; k < nslots; k++ ) {  // the tiles of every species in parts (as use_parts decides)
+                zpic_sort so = sp[k * n + i].s;
+                apart[i] = apart[i] && parts_on( view( &so ), parts ? parts + k * n + i : nullptr );
+            }
+            gc[3 * i].buf = const_cast<float *>( dep[i] );  // zeroed instead of J
+            grid_ops::CurArgs & a = cur[i];
+            a.dep = dep[i];
+            a.J = f.J;
+            a.g = g;
+            a.px = a.py = 1;
+            a.passes = (int) passes[i].size();
+            for ( int p = 0; p < a.passes; p++ ) {
+                a.a[p] = passes[i][p].a;
+                a.b[p] = passes[i][p].b;
+                a.c[p] = passes[i][p].c;
+            }
+        }
         for ( const FilterPass & p : passes[i] ) {
             k3_of[i].push_back( (int) k3.size() );
             k3.push_back( grid_ops::K3Args{ f.J, g, p.dir, p.a, p.b, p.c } );
@@ -2735,6 +2790,8 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
             a.S = view( &s );
             use_parts( a, parts ? parts + k * n + i : nullptr );
             a.waves = waves[i];
+            a.apart = apart[i];
+            if ( direct[i] ) a.J = (float3 *) dep[i];
             part[k * n + i] = a;
             zpic_particles p = it.p, t = it.tmp;
             sort[k * n + i] = sort_args( &p, &t, &s, it.fld.ntiles_x, it.fld.ntiles_y, it.fld.nx, it.fld.ny, 1, 1,
@@ -2763,6 +2820,7 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     stages.push_back( { SK_ADD_X, 0 } );
     stages.push_back( { SK_ADD_Y, 0 } );
     stages.push_back( { SK_COPY_XY, 0 } );
+    stages.push_back( { SK_CURRENT, 0 } );
     for ( size_t p = 0; p < max_passes; p++ ) {
         stages.push_back( { SK_K3, (int) p } );
         stages.push_back( { SK_COPY_X, (int) p } );  // x or y guard copy by the pass's direction
@@ -2771,8 +2829,6 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     stages.push_back( { SK_COPY_XY, 1 } );
     const int ns = (int) stages.size();
 
-    // tiles per item of the light stages
-    constexpr int ZERO_TILES = 32, NEWNP_TILES = 1024, GC_TILES = 16;
     constexpr int CELL_GRAIN = 4096;
     // tiles per item of the per-tile stages: small tiles are grouped so that
     // an item moves at least ~65536 particles (particle pass, sort) or covers
@@ -2786,6 +2842,12 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     long long all = 0;
     for ( int k = 0; k < nslots * n; k++ ) all += sp[k].p.max_part;
     const long long PART_GRAIN = std::max( 4096LL, std::min( 65536LL, all / 4096 ) );
+    // tiles per item of the light stages; the guard copies and merges, chains
+    // of dependent loads, shrink with the batch too (16 -> 4 on a 12-instance
+    // scan of 59 M particles: 1.94 -> 1.71 ms per step; 64 instances, 513 M:
+    // 8.92 at 16, 9.23 at 4)
+    constexpr int ZERO_TILES = 32, NEWNP_TILES = 1024;
+    const int GC_TILES = (int) std::max( 4LL, std::min( 16LL, PART_GRAIN / 4096 ) );
     std::vector<int> part_group( n ), cell_group( n );
     for ( int i = 0; i < n; i++ ) {
         const int cells = fl[i].g.nx * fl[i].g.ny;
@@ -2808,7 +2870,7 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
             const int i = order[oi];
             const zpic_batch_fields_item & f = fl[i];
             const int nt = f.g.ntiles_x * f.g.ntiles_y;
-            const int ctr = si * n + i;
+            int ctr = si * n + i;
             auto push = [&]( int kind, int arg, int t0, int t1, int dep0 ) {
                 StepItem it{};
                 it.kind = kind; it.arg = arg; it.t0 = t0; it.t1 = t1; it.done = ctr;
@@ -2820,21 +2882,34 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
             int dep = -1;
             switch ( st.kind ) {
             case SK_ZERO:
+                if ( apart[i] ) break;  // the merge writes every element
                 for ( int t = 0; t < nt; t += ZERO_TILES ) push( SK_ZERO, 3 * i, t, std::min( nt, t + ZERO_TILES ), -1 );
                 last[i] = si;
                 break;
             case SK_PART:
-                dep = last[i] * n + i;
+                dep = last[i] >= 0 ? last[i] * n + i : -1;
+                if ( apart[i] ) {  // one counter for all species, none waits
+                    dep = -1;
+                    if ( st.slot > 0 ) ctr = last[i] * n + i;
+                }
             {
                 // a tile in parts: each item takes the particles of part_group tiles
                 const PartScratch & pt = part[st.slot * n + i].parts;
                 const int ny = pt.on ? pt.cap : nt;
                 const int step = pt.on ? std::max( part_group[i], (int) ( PART_GRAIN / pt.size ) ) : part_group[i];
                 for ( int y = 0; y < ny; y += step ) push( SK_PART, st.slot * n + i, y, std::min( ny, y + step ), dep );
-                last[i] = part_stage[st.slot * n + i] = si;
+                if ( !apart[i] || st.slot == 0 ) last[i] = part_stage[st.slot * n + i] = si;
                 break;
             }
             case SK_MERGE:
+                if ( apart[i] ) {
+                    if ( st.slot < nslots - 1 ) break;
+                    dep = last[i] * n + i;
+                    for ( int t = 0; t < nt; t += GC_TILES ) push( SK_MERGE_ALL, i, t, std::min( nt, t + GC_TILES ), dep );
+                    last[i] = si;
+                    for ( int k = 0; k < nslots; k++ ) part_stage[k * n + i] = si;
+                    break;
+                }
                 if ( !part[st.slot * n + i].parts.on ) break;
                 dep = last[i] * n + i;
                 for ( int t = 0; t < nt; t += GC_TILES ) push( SK_MERGE, st.slot * n + i, t, std::min( nt, t + GC_TILES ), dep );
@@ -2862,6 +2937,7 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
             case SK_ADD_Y:
             case SK_COPY_XY:
             case SK_YEE: {
+                if ( direct[i] && st.kind != SK_YEE && st.slot == 0 ) break;  // SK_CURRENT does these
                 dep = last[i] * n + i;
                 const int arg = st.kind == SK_YEE ? i : 3 * i + st.slot;
                 if ( st.kind == SK_COPY_XY && st.slot == 1 ) {
@@ -2878,9 +2954,15 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
                 last[i] = si;
                 break;
             }
+            case SK_CURRENT:
+                if ( !direct[i] ) break;
+                dep = last[i] * n + i;
+                for ( int t = 0; t < nt; t += cell_group[i] ) push( SK_CURRENT, i, t, std::min( nt, t + cell_group[i] ), dep );
+                last[i] = si;
+                break;
             case SK_K3:
             case SK_COPY_X: {
-                if ( (size_t) st.slot >= passes[i].size() ) break;  // no such pass: the chain skips it
+                if ( direct[i] || (size_t) st.slot >= passes[i].size() ) break;  // no such pass: the chain skips it
                 dep = last[i] * n + i;
                 if ( st.kind == SK_K3 ) {
                     for ( int t = 0; t < nt; t += cell_group[i] )
@@ -2924,17 +3006,20 @@ int batch_step_create( BatchStepPlan ** out, const zpic_batch_species * sp, int 
     PartArgs * d_part = nullptr;
     SortArgs * d_sort = nullptr;
     EnergyArgs * d_ener = nullptr;
+    grid_ops::CurArgs * d_cur = nullptr;
     grid_ops::GcArgs * d_gc = nullptr;
     grid_ops::K3Args * d_k3 = nullptr;
     grid_ops::YeeArgs * d_yee = nullptr;
     if ( int rc = plan->upload( &d_part, part ) ) return rc;
     if ( int rc = plan->upload( &d_sort, sort ) ) return rc;
     if ( int rc = plan->upload( &d_ener, ener ) ) return rc;
+    if ( int rc = plan->upload( &d_cur, cur ) ) return rc;
     if ( int rc = plan->upload( &d_gc, gc ) ) return rc;
     if ( int rc = plan->upload( &d_k3, k3 ) ) return rc;
     if ( int rc = plan->upload( &d_yee, yee ) ) return rc;
     plan->T.part = d_part; plan->T.sort = d_sort; plan->T.energy = d_ener;
-    plan->T.gc = d_gc; plan->T.k3 = d_k3; plan->T.yee = d_yee;
+    plan->T.n = n; plan->T.nslots = nslots;
+    plan->T.cur = d_cur; plan->T.gc = d_gc; plan->T.k3 = d_k3; plan->T.yee = d_yee;
 
     // the dynamic LDS beside the kernel's static LDS must fit one workgroup
     int dev = 0, cus = 0, per_cu = 0, max_lds = 0;
@@ -3334,17 +3419,17 @@ struct zpic_batch_step {
 
 int zpic_batch_step_create( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
                             const zpic_batch_fields_item * fields, int n, int threads_per_tile ) {
-    return zpic::batch_step_new( out, species, nslots, fields, n, threads_per_tile, nullptr );
+    return zpic::batch_step_new( out, species, nslots, fields, n, threads_per_tile, nullptr, nullptr );
 }
 
 }  // extern "C"
 
 int zpic::batch_step_new( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
                           const zpic_batch_fields_item * fields, int n, int threads_per_tile,
-                          const PartScratch * parts ) {
+                          const PartScratch * parts, const float * const * dep ) {
     if ( !out ) return set_error( ZPIC_EINVAL, "null output" );
     BatchStepPlan * plan = nullptr;
-    if ( int rc = batch_step_create( &plan, species, nslots, fields, n, threads_per_tile, parts ) ) return rc;
+    if ( int rc = batch_step_create( &plan, species, nslots, fields, n, threads_per_tile, parts, dep ) ) return rc;
     *out = new zpic_batch_step{ plan };
     return ZPIC_OK;
 }

@@ -77,7 +77,11 @@ int batch_particles_new( zpic_batch_particles ** out, const zpic_batch_species *
 // zpic_batch_particles_advance in its two halves.
 int batch_particles_pass( zpic_batch_particles * plan, void * stream );
 int batch_particles_sort( zpic_batch_particles * plan, void * stream );
+// dep: deposit buffers of the instances, the current formed from them in one
+// stage, and with all tiles in parts the species side by side (null, or an
+// entry null or the instance's J: deposited into J, stage by stage).
 int batch_step_new( zpic_batch_step ** out, const zpic_batch_species * species, int nslots,
-                    const zpic_batch_fields_item * fields, int n, int threads_per_tile, const PartScratch * parts );
+                    const zpic_batch_fields_item * fields, int n, int threads_per_tile, const PartScratch * parts,
+                    const float * const * dep );
 
 }  // namespace zpic
