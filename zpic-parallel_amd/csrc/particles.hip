@@ -354,7 +354,10 @@ __device__ inline bool reflect_walls( int refl, int tx, int ty, int ntx, int nty
 // to the tile's list (idx[offset + w*chunk ...]) are in increasing order;
 // with the order-free sort it compacts its stayers to the chunk's front and
 // stages its leavers at the chunk's first positions.  seg[16 t + w] keeps
-// the count of each wave's leavers, seg[16 t + 15] the chunk.
+// the count of each wave's leavers, seg[16 t + 15] the chunk; with tiles in
+// parts the table has PART_SEG entries a tile: the waves of part after part,
+// and at its end the chunk, the old count and offset, the number of parts and
+// segments and the first part.
 //
 // LDS: E and B planes (6*vol floats, PUSH), then J (MOVE: 3*vol 64-bit
 // elements, or 3*vol floats with DET), then W crossing queues (QCAP entries
@@ -2048,7 +2051,7 @@ int check_geom( const zpic_geom * g ) {
 // Threads per tile of the fast particle pass (a multiple of 64, at most
 // FAST_BLOCK); the deterministic mode always uses one wavefront.  Default 256:
 // on the 2048^2 Weibel step the particle pass took 7.08 ms with 4 waves per
-// tile against 7.36 ms with 8 (fewer private J planes to clear and reduce).
+// tile against 7.36 ms with 8 (measured with a J copy per wave).
 int g_threads = 256;  // library-wide setting
 // Fast-mode tile sort: 0 (default) = order-free (leavers staged by the
 // particle pass, k_sort_shift + k_sort_in_fast), 1 = the reference's
@@ -2102,7 +2105,7 @@ int launch_particles( const zpic_particles * p, const zpic_geom * fld, const flo
     if ( !p || ( PUSH && ( !E || !B || !tile_energy ) ) || ( MOVE && ( !J || !s ) ) )
         return set_error( ZPIC_EINVAL, "null buffer" );
     const int nt = fld->ntiles_x * fld->ntiles_y;
-    // Large tiles: fewer wavefronts (each holds a private J copy) until LDS fits.
+    // Large tiles: fewer wavefronts (fit_bytes).
     int threads = det ? WAVE : g_threads;
     while ( threads > WAVE && fit_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT ) threads -= WAVE;
     if ( fit_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT )

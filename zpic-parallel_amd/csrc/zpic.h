@@ -546,10 +546,11 @@ class Current {
     double dt;
     current::bc_type bc;
     int iter;
-    // Second buffer of the one-pass update (zpic_current_update): on periodic
-    // grids with no filter or a filter along x, advance() forms the new
+    // Second buffer of the one-pass update (current_update): without walls
+    // and with no filter or a filter along x, advance() forms the new
     // current from J's deposit into this grid's buffer in one launch, then
-    // J and this grid exchange buffers (allocated on first use).
+    // J and this grid exchange buffers; a step whose species run side by side
+    // deposits here and forms J from it (allocated on first use).
     vec3grid<float3> * Jalt;
     // whether advance() may run as one pass, and the filter's x passes
     bool one_pass_ok( std::vector<float> & coef ) const;
