@@ -1,7 +1,7 @@
-// Sums in LDS in 64-bit fixed point, by integer atomics: on gfx950 a wave's
-// ds_add_f32 takes about 194 cycles of its compute unit, whatever the
-// addresses, its ds_add_u64 at most 16 (ds_add_f64 23), and a sum of integers
-// does not depend on its order.
+// Sums of weights (terms of about 1) in LDS in 64-bit fixed point, by integer
+// atomics: on gfx950 a wave's ds_add_f32 takes about 194 cycles of its compute
+// unit, whatever the addresses, its ds_add_u64 at most 16 (ds_add_f64 23), and
+// a sum of integers does not depend on its order.
 #pragma once
 
 #include "common.h"
@@ -15,13 +15,12 @@ typedef __attribute__( ( address_space( 3 ) ) ) u64 lds_u64;
 typedef u64 lds_u64;
 #endif
 
-// 2^bits to the unit, for terms of at most about 1 (the common factors of a
-// sum are applied to its end).  With `bits` the terms of n particles cannot
-// overflow an element (FIX_HEADROOM bits are left for a path's up to three
-// segments and for weights of positions a little outside their cell), and a
-// term is off by at most 2^-47 of the unit up to 2047 particles and 2^-43 at
-// 16384: far less than the rounding of its own FP32 arithmetic, and the sum
-// adds nothing.  fixed_add holds terms below 32.
+// 2^bits to the unit (the common factors of a sum are applied to its end).
+// With `bits` the weights of n particles cannot overflow an element
+// (FIX_HEADROOM bits are left for those of positions outside their cell), and
+// a term is off by at most 2^-47 up to 2047 particles and 2^-43 at 16384.  The
+// quantum is absolute: terms far below 1 lose bits (lds_sum.h holds those).
+// fixed_add holds terms below 32.
 constexpr int FIX_HEADROOM = 5, FIX_MAX_BITS = 46;
 
 struct Fixed {

@@ -3,12 +3,9 @@
 //
 // One workgroup per tile (or part of a tile).  The tile's E and B (with guard
 // cells) are staged in LDS as six float planes, and its current is summed in
-// LDS in 64-bit fixed point with integer atomics, shared by the workgroup's
-// waves: on this part LDS float atomics run at about three clocks per lane,
-// 64-bit integer ones at least twelve times as fast, and a sum of integers
-// does not depend on its order.  It is scaled and added once into the tile's
-// own region of the global J grid (each tile owns its guard cells, so that
-// needs no global atomics).
+// LDS in doubles (lds_sum.h), shared by the workgroup's waves.  It takes its
+// charge factors and is added once into the tile's own region of the global J
+// grid (each tile owns its guard cells, so that needs no global atomics).
 //
 // Arithmetic is the reference's, operation for operation: no contraction
 // (built with -ffp-contract=off), fmaf exactly where the reference calls
@@ -21,6 +18,7 @@
 #include "common.h"
 #include "fixed.h"
 #include "grid_ops.h"
+#include "lds_sum.h"
 #include "parts.h"
 
 #include <algorithm>
@@ -253,9 +251,8 @@ __device__ inline void segment_current( const Seg & s, float qnx, float qny, flo
 // (whose J is compared to a tolerance: the deposit's sums differ anyway):
 // wy0 = (A0y + B0y) / 2 = 1/2 - (a.y + b.y) / 2, wy1 = 1/2 + (a.y + b.y) / 2,
 // and Jz = q (Ax (Ay + By / 2) + Bx (By - Ay / 2)), the reference's
-// Ax Ay + Bx By + (Ax By - Bx Ay) / 2 regrouped.  False if one of them is
-// not a number or large.
-__device__ inline bool segment_current_fma( const Seg & s, float v[8] ) {
+// Ax Ay + Bx By + (Ax By - Bx Ay) / 2 regrouped.
+__device__ inline void segment_current_fma( const Seg & s, float v[8] ) {
     const float A0x = 0.5f - s.a.x, A1x = 0.5f + s.a.x, B0x = 0.5f - s.b.x, B1x = 0.5f + s.b.x;
     const float A0y = 0.5f - s.a.y, A1y = 0.5f + s.a.y, B0y = 0.5f - s.b.y, B1y = 0.5f + s.b.y;
     const float jx = s.b.x - s.a.x;
@@ -272,9 +269,6 @@ __device__ inline bool segment_current_fma( const Seg & s, float v[8] ) {
     v[4] = q * fmaf( A1x, p0, B1x * r0 );
     v[6] = q * fmaf( A0x, p1, B0x * r1 );
     v[7] = q * fmaf( A1x, p1, B1x * r1 );
-    // (ends inside the cell and |q| <= 1/2: 2.5; up to 3.5 no contribution
-    // reaches 8, and the conversion holds 32)
-    return fabsf( s.a.x ) + fabsf( s.b.x ) + fabsf( s.a.y ) + fabsf( s.b.y ) + fabsf( q ) < 3.5f;
 }
 
 // LDS (address space 3) element types: volatile accesses through generic
@@ -299,23 +293,19 @@ __device__ inline void add_current( volatile lds_f32 * Jx, volatile lds_f32 * Jy
 }
 
 // Fast-mode deposit of one segment into J, element (node, component).
-// Returns false for a segment that is not a number or out of the fixed
-// point's range (a position far outside its cell), which is not deposited:
-// the tile's current is then not a number.
-__device__ inline bool deposit_fixed( const Seg & s, lds_u64 * J, int ys, const Fixed & f ) {
+__device__ inline void deposit_segment( const Seg & s, lds_f64 * J, int ys ) {
     float v[8];
-    if ( !segment_current_fma( s, v ) ) return false;
-    lds_u64 * const p = J + 3 * ( s.c.x + __mul24( ys, s.c.y ) );
-    lds_u64 * const q = p + 3 * ys;
-    fixed_add( p, v[0], f );
-    fixed_add( p + 1, v[1], f );
-    fixed_add( p + 2, v[2], f );
-    fixed_add( p + 4, v[3], f );
-    fixed_add( p + 5, v[4], f );
-    fixed_add( q, v[5], f );
-    fixed_add( q + 2, v[6], f );
-    fixed_add( q + 5, v[7], f );
-    return true;
+    segment_current_fma( s, v );
+    lds_f64 * const p = J + 3 * ( s.c.x + __mul24( ys, s.c.y ) );
+    lds_f64 * const q = p + 3 * ys;
+    lds_add( p, v[0] );
+    lds_add( p + 1, v[1] );
+    lds_add( p + 2, v[2] );
+    lds_add( p + 4, v[3] );
+    lds_add( p + 5, v[4] );
+    lds_add( q, v[5] );
+    lds_add( q + 2, v[6] );
+    lds_add( q + 5, v[7] );
 }
 
 struct MoveArgs {
@@ -359,8 +349,8 @@ __device__ inline bool reflect_walls( int refl, int tx, int ty, int ntx, int nty
 // and at its end the chunk, the old count and offset, the number of parts and
 // segments and the first part.
 //
-// LDS: E and B planes (6*vol floats, PUSH), then J (MOVE: 3*vol 64-bit
-// elements, or 3*vol floats with DET), then W crossing queues (QCAP entries
+// LDS: E and B planes (6*vol floats, PUSH), then J (MOVE: 3*vol doubles, or
+// 3*vol floats with DET), then W crossing queues (QCAP entries
 // of QWORDS words, MOVE), then W leaver buffers (LBCAP records of LBWORDS
 // words, order-free sort, lbuf).
 //
@@ -390,7 +380,7 @@ constexpr int SEG16 = 13;
 // LDS of the particle pass.
 __host__ __device__ inline size_t particles_lds_bytes( int vol, int W, bool push, bool move, bool lbuf = false ) {
     return sizeof( float ) * (size_t) vol * ( push ? 6 : 0 ) +
-           ( move ? sizeof( u64 ) * (size_t) vol * 3 + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 ) +
+           ( move ? sizeof( double ) * (size_t) vol * 3 + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 ) +
            ( move && lbuf ? sizeof( float ) * (size_t) W * LBCAP * LBWORDS : 0 );
 }
 // The rule that fits a pass's waves to the tile (zpic_fitted_threads_per_tile
@@ -534,7 +524,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     float * Bx = Ez + vol;
     float * By = Bx + vol;
     float * Bz = By + vol;
-    float * Jall = PUSH ? Bz + vol : smem;  // 64-bit elements (node, component); DET: three float planes
+    float * Jall = PUSH ? Bz + vol : smem;  // doubles (node, component); DET: three float planes
     float * Jx = Jall;
     float * Jy = Jx + vol;
     float * Jz = Jy + vol;
@@ -542,7 +532,6 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     float * queue = qbase + (size_t) w * QCAP * QWORDS;
     float * lbuf = qbase + (size_t) W * QCAP * QWORDS + (size_t) w * LBCAP * LBWORDS;  // if a.lbuf
     __shared__ int s_cnt[9];
-    __shared__ int s_bad;  // a segment that cannot be deposited
     __shared__ double s_en[FAST_BLOCK / WAVE];
     __shared__ int s_nl[FAST_BLOCK / WAVE];
     const int off = gbl( P.off )[t];
@@ -563,7 +552,6 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     if constexpr ( MOVE ) {
         for ( int k = tid; k < 6 * vol; k += nthr ) Jall[k] = 0.0f;
         if ( tid < 9 ) s_cnt[tid] = 0;
-        if ( tid == 9 ) s_bad = 0;
     }
     __syncthreads();
 
@@ -590,10 +578,8 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     volatile lds_f32 * j0x = (volatile lds_f32 *) ( Jx + g.off );
     volatile lds_f32 * j0y = (volatile lds_f32 *) ( Jy + g.off );
     volatile lds_f32 * j0z = (volatile lds_f32 *) ( Jz + g.off );
-    lds_u64 * const jfix = (lds_u64 *) reinterpret_cast<u64 *>( Jall );
-    lds_u64 * const jfix0 = jfix + 3 * g.off;
-    const Fixed fx = fixed_point( np );
-    bool ok = true;  // every segment so far was deposited
+    lds_f64 * const jsum = (lds_f64 *) reinterpret_cast<double *>( Jall );
+    lds_f64 * const jsum0 = jsum + 3 * g.off;
 
     double en = 0.0;
     int nl = 0;
@@ -633,7 +619,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
         }
 #pragma unroll
         for ( int k = 0; k < 3; k++ )
-            if ( ns > k ) ok &= deposit_fixed( sg[k], jfix0, ys, fx );
+            if ( ns > k ) deposit_segment( sg[k], jsum0, ys );
     };
 
     // The particles of the next PREFETCH iterations are loaded while the
@@ -775,7 +761,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
             }
             nl += __popcll( mask );
             // paths inside one cell: their single segment now
-            if ( act && !cross ) ok &= deposit_fixed( s0, jfix0, ys, fx );
+            if ( act && !cross ) deposit_segment( s0, jsum0, ys );
             // paths that cross: queued, split and deposited 64 at a time
             const unsigned long long cm = __ballot( cross );
             if ( cm ) {
@@ -853,7 +839,6 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     }
     if constexpr ( MOVE && !DET ) {
         if ( qn > 0 ) flush_queue( qn );
-        if ( !ok ) s_bad = 1;
         if ( lbon && lbn > 0 ) flush_leavers( lbn );
     }
 
@@ -869,19 +854,18 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     __syncthreads();
 
     if constexpr ( MOVE ) {
-        // flush: J(tile) += sum of the waves' J (LDS), guard cells included
+        // flush: J(tile) += the J of the LDS, guard cells included
         // (species.cpp:1488-1492)
         const bool apart = nparts > 1 || a.apart;
         const gptr<float> Jt = gbl( apart ? a.parts.J + (size_t) y * 3 * vol
                                           : reinterpret_cast<float *>( J + (size_t) t * vol ) );
-        const float bad = ( !DET && s_bad ) ? __builtin_nanf( "" ) : 0.0f;
         for ( int k = tid; k < 3 * g.ext_x * g.ext_y; k += nthr ) {
             const int el = k / 3, c = k - 3 * el;
             float s;
             if constexpr ( DET ) {
                 s = Jall[c * vol + el];
             } else {
-                s = fixed_value( jfix[k], fx, c == 0 ? m.qnx : c == 1 ? m.qny : m.q ) + bad;  // + 0: never -0
+                s = (float) ( jsum[k] * ( c == 0 ? m.qnx : c == 1 ? m.qny : m.q ) ) + 0.0f;  // + 0: never -0
             }
             // jset (the first species of a step, fast mode): the region is
             // written instead of zeroed and added to; the same value, since
