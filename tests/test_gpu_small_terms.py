@@ -92,3 +92,33 @@ def test_ill_particles(what, count):
         # (paths cut outside their cell: terms of some tens, each to 2^-24)
         ok = ~np.isnan(ref)
         assert np.abs(fast - ref)[ok].max() <= 1e-5 * np.abs(ref[ok]).max()
+
+
+@pytest.mark.parametrize("count", [3, 5000])
+@pytest.mark.parametrize("where", [(np.nan, 0.1), (0.2, -7.0), (3e4, 2e4)])
+def test_charge_of_ill_positions(where, count):
+    """The charge of a position that is no number, or outside its cell: the
+    same elements as in the deterministic mode, nothing lost beside them."""
+    import pyzpic as zp
+    ntiles, nx = (3, 2), (8, 8)
+    rng = np.random.default_rng(8)
+    np_ = np.array([5, 0, 2000, 40, count, 1], np.int32)
+    n = int(np_.sum())
+    ix = rng.integers(0, 8, (n, 2)).astype(np.int32)
+    x = (rng.random((n, 2)) - 0.5).astype(np.float32)
+    bad = int(np_[:4].sum()) + count // 2
+    ix[bad], x[bad] = (3, 5), where
+    out = []
+    for det in (False, True):
+        sim = simulation(zp, ntiles, nx, det)
+        sim.species[0].set_particles(np_, ix, x, np.zeros((n, 3), np.float32))
+        out.append(sim.species[0].charge())
+        sim.close()
+    fast, ref = out
+    assert np.array_equal(np.isnan(fast), np.isnan(ref))
+    assert np.isnan(ref).any() == bool(np.isnan(where[0])) and not np.isnan(ref).all()
+    # (each element to 1e-5 of its own, the particles of an element being a
+    # few hundred terms of one sign; those of the bad cell to 1e-5 of its terms)
+    ok = ~np.isnan(ref)
+    size = np.abs(ref[ok])
+    assert (np.abs(fast - ref)[ok] <= 1e-5 * np.where(size > 100, size.max(), size + 1e-3)).all()

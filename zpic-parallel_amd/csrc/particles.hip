@@ -16,7 +16,6 @@
 // tile and serialises the deposit and the energy sum over lanes in particle
 // order, which reproduces the reference's single-thread results exactly.
 #include "common.h"
-#include "fixed.h"
 #include "grid_ops.h"
 #include "lds_sum.h"
 #include "parts.h"
@@ -1933,23 +1932,21 @@ __global__ void __launch_bounds__( SORT_WAVES * WAVE ) k_sort_in_fast( SortArgs 
 
 // ---------------------------------------------------------------------------
 // dep_charge_kernel (species.cpp:2348-2395) into a scalar grid with guards.
-// Fast mode: the weights are summed in LDS in 64-bit fixed point and take
-// the charge at the end (float atomics there: 194 us for the 9.4 million
-// particles of 2304 tiles, against 40 us).
+// Fast mode: the weights are summed in LDS in doubles and take the charge at
+// the end (9.4 million particles of 2304 tiles: 34 us; by integers in fixed
+// point 30, but a position far outside its cell, or no number, made the whole
+// tile's charge NaN; by float atomics 194).
 template <bool DET>
 __global__ void __launch_bounds__( FAST_BLOCK ) k_charge( PartView P, Geo g, float * __restrict__ rho, float q ) {
     extern __shared__ __align__( 16 ) float smem[];
     const int t = blockIdx.x;
     const int vol = g.vol, ys = g.ext_x;
     for ( int k = threadIdx.x; k < ( DET ? vol : 2 * vol ); k += blockDim.x ) smem[k] = 0.0f;
-    __shared__ int s_bad;
-    if ( threadIdx.x == 0 ) s_bad = 0;
     __syncthreads();
     float * c0 = smem + g.off;
-    lds_u64 * const fixed = (lds_u64 *) reinterpret_cast<u64 *>( smem );
-    lds_u64 * const f0 = fixed + g.off;
+    lds_f64 * const sum = (lds_f64 *) reinterpret_cast<double *>( smem );
+    lds_f64 * const f0 = sum + g.off;
     const int off = P.off[t], np = P.np[t];
-    const Fixed fx = fixed_point( np );
     const int lane = threadIdx.x % WAVE;
     const int nthr = blockDim.x;
     for ( int i0 = ( threadIdx.x / WAVE ) * WAVE; i0 < np; i0 += nthr ) {
@@ -1971,21 +1968,17 @@ __global__ void __launch_bounds__( FAST_BLOCK ) k_charge( PartView P, Geo g, flo
                 }
             }
         } else if ( act ) {
-            if ( fabsf( s0x ) + fabsf( s0y ) < 5.0f ) {
-                fixed_add( f0 + k, s0y * s0x, fx );
-                fixed_add( f0 + k + 1, s0y * s1x, fx );
-                fixed_add( f0 + k + ys, s1y * s0x, fx );
-                fixed_add( f0 + k + ys + 1, s1y * s1x, fx );
-            } else {
-                s_bad = 1;  // a position far outside its cell, or not a number
-            }
+            lds_add( f0 + k, s0y * s0x );
+            lds_add( f0 + k + 1, s0y * s1x );
+            lds_add( f0 + k + ys, s1y * s0x );
+            lds_add( f0 + k + ys + 1, s1y * s1x );
         }
     }
     __syncthreads();
     float * dst = rho + (size_t) t * vol;
     for ( int k = threadIdx.x; k < g.ext_x * g.ext_y; k += blockDim.x ) {
         if constexpr ( DET ) dst[k] += smem[k];
-        else dst[k] += s_bad ? __builtin_nanf( "" ) : fixed_value( fixed[k], fx, q );
+        else dst[k] += (float) ( sum[k] * q );
     }
 }
 
@@ -3451,7 +3444,7 @@ int zpic_deposit_charge( const zpic_particles * p, const zpic_geom * g, float * 
                          void * stream ) {
     if ( !p || !g || !rho ) return set_error( ZPIC_EINVAL, "null buffer" );
     const int nt = g->ntiles_x * g->ntiles_y;
-    const size_t lds = ( deterministic ? sizeof( float ) : sizeof( u64 ) ) * g->tile_vol;
+    const size_t lds = ( deterministic ? sizeof( float ) : sizeof( double ) ) * g->tile_vol;
     if ( sizeof( float ) * g->tile_vol > 65536 ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
     hipStream_t st = as_stream( stream );
     if ( deterministic )
