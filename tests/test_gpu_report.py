@@ -50,7 +50,9 @@ def close(a, b):
     (0, (-0.3, 40.0), 128, 2, (-0.4, 0.4), 96),
     (1, (0.0, 6.0), 50, 4, (-1.0, 1.0), 33),
     (0, (0.0, 8.0), 90, 1, (0.0, 8.0), 110),
-    (2, (-0.3, 0.3), 128, 4, (-0.9, 0.9), 96),        # more bins than fit
+    (2, (-0.3, 0.3), 128, 4, (-0.9, 0.9), 96),        # the most bins that fit
+    (2, (-0.3, 0.3), 128, 4, (-0.9, 0.9), 97),        # more
+    (2, (-0.3, 0.3), 91, 3, (-0.3, 0.3), 91),
     (2, (-0.3, 0.3), 3, 3, (-0.9, 0.9), 4),
 ])
 def test_phasespace(pair, axes):

