@@ -267,3 +267,30 @@ def test_persistent_current_from_deposit(zp, shape):
     batch.close()
     for s in sims:
         s.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_without_species(zp, graph):
+    """Instances of fields alone (a pulse in vacuum), eager and replayed."""
+    rng = np.random.default_rng(3)
+    start = {}
+
+    def vacuum(ntiles, nx):
+        sim = zp.Simulation(ntiles, nx, tuple(np.float32(a * b * 0.1) for a, b in zip(ntiles, nx)), 0.07)
+        for f in "EB":
+            start.setdefault((ntiles, f), rng.normal(0, 1, sim.field(f).shape).astype(np.float32))
+            sim.set_field(f, start[ntiles, f])
+        return sim
+
+    grids = [((3, 2), (16, 16)), ((1, 4), (8, 24))]
+    sims, refs = ([vacuum(*g) for g in grids] for _ in range(2))
+    batch = zp.Batch(sims, graph=graph)
+    for step in range(3):
+        batch.advance()
+        for sim, ref in zip(sims, refs):
+            ref.advance()
+            for f in "EBJ":
+                assert np.array_equal(sim.field(f).view(np.uint32), ref.field(f).view(np.uint32)), (step, f)
+    batch.close()
+    for sim in sims + refs:
+        sim.close()

@@ -1415,8 +1415,8 @@ void Batch::build() {
         return;
     }
     // all instances' tiles in parts: the species side by side, each instance's
-    // current from its deposit buffer
-    bool all = true;
+    // current from its deposit buffer (instances without species: fields alone)
+    bool all = nsp > 0;
     for ( auto * s : sims )
         for ( auto * sp : s->species ) all = all && sp->side_by_side();
     std::vector<const float *> dep;
