@@ -294,3 +294,22 @@ def test_batch_without_species(zp, graph):
     batch.close()
     for sim in sims + refs:
         sim.close()
+
+
+@pytest.mark.parametrize("persistent", [False, True])
+def test_batch_of_large_tiles(zp, persistent):
+    """Tiles of which one workgroup's LDS leaves room for no second one on a
+    compute unit, beside small ones, equal their single runs."""
+    shapes = [dict(ntiles=(2, 1), nx=(38, 38), ppc=(2, 3), filter=None),
+              dict(ntiles=(3, 2), nx=(16, 16), ppc=(3, 3), filter=("binomial", 0, 2)),
+              dict(ntiles=(1, 2), nx=(36, 37), ppc=(2, 2), filter=None)]
+    sims, refs = ([make(zp, sh) for sh in shapes] for _ in range(2))
+    batch = zp.Batch(sims, threads_per_tile=zp.get_threads_per_tile(), persistent=persistent)
+    batch.advance(4)
+    batch.status()
+    for k, (s, r) in enumerate(zip(sims, refs)):
+        r.advance(4)
+        assert_same(state(s), state(r), f"instance {k}")
+    batch.close()
+    for s in sims + refs:
+        s.close()

@@ -28,6 +28,9 @@ def crowded(ntiles, nx, counts, seed):
     ((33, 32), (8, 8), 256, [3] * 1055 + [5000]),   # more than one tile per thread of the scan
     ((32, 32), (8, 8), 256, [1] * 1000 + [0] * 23 + [9000]),
     ((64, 64), (4, 4), 256, [2] * 4090 + [0] * 5 + [3000]),
+    ((2, 2), (36, 36), 256, [20000, 3, 0, 1025]),   # the largest tiles: two workgroups of the pass per CU
+    ((2, 2), (38, 38), 512, [20000, 3, 0, 1025]),   # and one
+    ((1, 1), (38, 38), 64, [5000]),
     ((241, 17), (4, 5), 256, [1] * 4096 + [3000]),  # more tiles than the cut is used for
 ])
 def test_crowded_tiles(ntiles, nx, threads, counts):

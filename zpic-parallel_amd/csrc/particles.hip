@@ -349,7 +349,7 @@ __device__ inline bool reflect_walls( int refl, int tx, int ty, int ntx, int nty
 // segments and the first part.
 //
 // LDS: E and B planes (6*vol floats, PUSH), then J (MOVE: 3*vol doubles, or
-// 3*vol floats with DET), then W crossing queues (QCAP entries
+// 3*vol floats and no more with DET), then W crossing queues (QCAP entries
 // of QWORDS words, MOVE), then W leaver buffers (LBCAP records of LBWORDS
 // words, order-free sort, lbuf).
 //
@@ -377,14 +377,16 @@ constexpr int SEG_CHUNK = 1, SEG_OLD_NP = 2, SEG_OLD_OFF = 3, SEG_COUNT = 4, SEG
 constexpr int SEG16 = 13;
 
 // LDS of the particle pass.
-__host__ __device__ inline size_t particles_lds_bytes( int vol, int W, bool push, bool move, bool lbuf = false ) {
-    return sizeof( float ) * (size_t) vol * ( push ? 6 : 0 ) +
+__host__ __device__ inline size_t particles_lds_bytes( int vol, int W, bool push, bool move, bool lbuf = false,
+                                                       bool det = false ) {
+    const size_t fields = sizeof( float ) * (size_t) vol * ( push ? 6 : 0 );
+    if ( det ) return fields + sizeof( float ) * (size_t) vol * ( move ? 3 : 0 );
+    return fields +
            ( move ? sizeof( double ) * (size_t) vol * 3 + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 ) +
            ( move && lbuf ? sizeof( float ) * (size_t) W * LBCAP * LBWORDS : 0 );
 }
-// The rule that fits a pass's waves to the tile (zpic_fitted_threads_per_tile
-// states it): 64 KiB for the fields and a float J and a byte of each element
-// per wave.
+// The rule that fits a pass's waves to the tile (fitted_threads): 64 KiB for
+// the fields and a float J and a byte of each element per wave.
 __host__ __device__ inline size_t fit_bytes( int vol, int W, bool push, bool move ) {
     return sizeof( float ) * (size_t) vol * ( ( push ? 6 : 0 ) + ( move ? 3 * W : 0 ) ) +
            ( move ? ( ( (size_t) W * vol + 3 ) & ~(size_t) 3 ) + sizeof( float ) * (size_t) W * QCAP * QWORDS : 0 );
@@ -549,7 +551,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
         }
     }
     if constexpr ( MOVE ) {
-        for ( int k = tid; k < 6 * vol; k += nthr ) Jall[k] = 0.0f;
+        for ( int k = tid; k < ( DET ? 3 : 6 ) * vol; k += nthr ) Jall[k] = 0.0f;
         if ( tid < 9 ) s_cnt[tid] = 0;
     }
     __syncthreads();
@@ -2038,13 +2040,23 @@ int g_threads = 256;  // library-wide setting
 // time.
 int g_reference_order = 0;
 
-constexpr size_t LDS_LIMIT = 65536;  // LDS of fit_bytes (the LDS itself takes up to 84 KiB for the largest tile)
+constexpr size_t LDS_LIMIT = 65536;  // LDS of fit_bytes (the LDS itself takes up to 83 KiB for the largest tile)
+constexpr size_t CU_LDS = 163840;
+constexpr size_t STATIC_LDS = 256;  // the kernel's static LDS, rounded up
 
 // Threads per tile the particle pass runs with for tiles of `vol` elements
-// when asked for `threads` (reduced until the LDS staging fits).
-int fitted_threads( int threads, int vol ) {
-    while ( threads > WAVE && fit_bytes( vol, threads / WAVE, true, true ) > LDS_LIMIT ) threads -= WAVE;
-    return fit_bytes( vol, threads / WAVE, true, true ) > LDS_LIMIT ? 0 : threads;
+// when asked for `threads` (reduced until fit_bytes allows it; 0: the tile is
+// too large).  Where J in doubles leaves room for one workgroup per CU (about
+// 1660 elements with the fields, 38 x 38 cells), that one takes up to four
+// waves: 70 x 70 such tiles at 2 x 16 particles per cell take 6.1 ms a step so,
+// 19.4 with the single wave of the rule, 15.0 with float sums in 64 KiB.
+int fitted_threads( int threads, int vol, bool push = true, bool move = true ) {
+    int fit = threads;
+    while ( fit > WAVE && fit_bytes( vol, fit / WAVE, push, move ) > LDS_LIMIT ) fit -= WAVE;
+    if ( fit_bytes( vol, fit / WAVE, push, move ) > LDS_LIMIT ) return 0;
+    if ( 2 * ( particles_lds_bytes( vol, fit / WAVE, push, move ) + STATIC_LDS ) > CU_LDS )
+        fit = std::max( fit, std::min( threads, 4 * WAVE ) );
+    return fit;
 }
 
 int check_threads( int threads ) {
@@ -2057,12 +2069,7 @@ int check_threads( int threads ) {
 // which the pass already runs at its memory rate (three buffers more or less
 // measured the same).
 bool lbuf_fits( size_t without, size_t with ) {
-    int dev = 0, cu_lds = 0;
-    if ( hipGetDevice( &dev ) != hipSuccess ||
-         hipDeviceGetAttribute( &cu_lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev ) != hipSuccess )
-        return false;
-    const size_t stat = 256;  // the kernel's static LDS, rounded up
-    return cu_lds / ( with + stat ) >= std::min( (size_t) 4, cu_lds / ( without + stat ) );
+    return CU_LDS / ( with + STATIC_LDS ) >= std::min( (size_t) 4, CU_LDS / ( without + STATIC_LDS ) );
 }
 
 // Tiles in parts need the order-free sort (its segment table).
@@ -2082,12 +2089,9 @@ int launch_particles( const zpic_particles * p, const zpic_geom * fld, const flo
     if ( !p || ( PUSH && ( !E || !B || !tile_energy ) ) || ( MOVE && ( !J || !s ) ) )
         return set_error( ZPIC_EINVAL, "null buffer" );
     const int nt = fld->ntiles_x * fld->ntiles_y;
-    // Large tiles: fewer wavefronts (fit_bytes).
-    int threads = det ? WAVE : g_threads;
-    while ( threads > WAVE && fit_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT ) threads -= WAVE;
-    if ( fit_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE ) > LDS_LIMIT )
-        return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
-    size_t lds = particles_lds_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE );
+    const int threads = fitted_threads( det ? WAVE : g_threads, fld->tile_vol, PUSH, MOVE );
+    if ( threads == 0 ) return set_error( ZPIC_ERANGE, "tile too large for LDS staging" );
+    size_t lds = particles_lds_bytes( fld->tile_vol, threads / WAVE, PUSH, MOVE, false, det );
     PartArgs a{};
     a.P = view( p ); a.g = make_geo( fld );
     a.E = (const float3 *) E; a.B = (const float3 *) B; a.J = (float3 *) J;
