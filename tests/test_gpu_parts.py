@@ -65,3 +65,27 @@ def test_crowded_tiles(ntiles, nx, threads, counts):
         zp.set_threads_per_tile(old)
         for sim in sims:
             sim.close()
+
+
+def test_species_of_different_sizes():
+    """Species side by side whose lists of parts differ in length, one of them
+    empty."""
+    import pyzpic as zp
+    sims = []
+    for det in (False, True):
+        sim = zp.Simulation((5, 4), (8, 8), (np.float32(4.0), np.float32(3.2)), 0.07, deterministic=det)
+        for k, ppc in enumerate([(1, 1), (20, 20), (2, 1)]):
+            sim.add_species(zp.Species(f"s{k}", (-1.0, 1.0, 4.0)[k], ppc))
+        sims.append(sim)
+    for sim in sims:
+        for k, counts in enumerate([[3] * 19 + [700], [1200] * 20, [0] * 20]):
+            sim.species[k].set_particles(*crowded((5, 4), (8, 8), counts, 11 + k))
+        sim.advance()
+    fast, det = sims
+    for k in range(3):
+        assert same_tile_multisets(fast.species[k].particles(), det.species[k].particles()), k
+    for f in "JEB":
+        a, b = fast.field(f).astype(np.float64), det.field(f).astype(np.float64)
+        assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b), f
+    for sim in sims:
+        sim.close()

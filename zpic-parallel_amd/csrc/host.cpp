@@ -225,17 +225,19 @@ void ParticleSort::init_parts( uint32_t max_part, int tile_vol ) {
     const int extra = part_extra( max_part );
     parts.size = part_size( max_part, extra );
     parts.cap = ntiles + extra;
-    parts.seg = device_alloc<int>( (size_t) PART_SEG * ntiles );
-    parts.item = device_alloc<int>( 2 * (size_t) parts.cap );
-    parts.total = device_alloc<int>( 1 );
-    parts.npt = device_alloc<int>( 9 * (size_t) parts.cap );
-    parts.energy = device_alloc<double>( parts.cap );
-    parts.J = device_alloc<float>( 3 * (size_t) parts.cap * tile_vol );
+    // one allocation: J regions, energies, segment table, items, counts, their number
+    const size_t nJ = 3 * (size_t) parts.cap * tile_vol, nseg = (size_t) PART_SEG * ntiles, cap = parts.cap;
+    char * p = device_alloc<char>( 4 * nJ + 8 * cap + 4 * ( nseg + 2 * cap + 9 * cap + 1 ) );
+    parts.J = reinterpret_cast<float *>( p );
+    parts.energy = reinterpret_cast<double *>( parts.J + nJ );  // (tile_vol is a multiple of 4)
+    parts.seg = reinterpret_cast<int *>( parts.energy + cap );
+    parts.item = parts.seg + nseg;
+    parts.npt = parts.item + 2 * cap;
+    parts.total = parts.npt + 9 * cap;
 }
 
 ParticleSort::~ParticleSort() {
-    device_free( parts.J ); device_free( parts.energy ); device_free( parts.npt );
-    device_free( parts.total ); device_free( parts.item ); device_free( parts.seg );
+    device_free( parts.J );
     device_free( buf.nmove );
     device_free( buf.total ); device_free( buf.tmp_np ); device_free( buf.seg );
     device_free( buf.new_np ); device_free( buf.npt ); device_free( buf.idx );
@@ -1164,22 +1166,20 @@ bool Simulation::step_side_by_side() {
     if ( species.empty() ) return false;
     for ( auto * s : species )
         if ( !s->side_by_side() ) return false;
-    float * const dep = current.deposit_buffer();
-    std::vector<const void *> key{ dep, emf.E->fbuf(), emf.B->fbuf(), nullptr };
-    key[3] = reinterpret_cast<const void *>( (uintptr_t) zpic_get_threads_per_tile() );
+    std::vector<const void *> key{ emf.E->fbuf(), emf.B->fbuf(), nullptr };
+    key[2] = reinterpret_cast<const void *>( (uintptr_t) zpic_get_threads_per_tile() );
     for ( auto * s : species ) s->buffers( key );
     if ( !side || key != side_key ) {
+        // kernels on the way may still read the tables of the last build
+        if ( side ) zpic::hip_check( hipStreamSynchronize( stream() ), "hipStreamSynchronize" );
         zpic_batch_particles_free( side );
         side = nullptr;
         std::vector<zpic_batch_species> items;
         std::vector<PartScratch> parts;
         for ( auto * s : species ) {
             items.push_back( s->batch_item( emf, current ) );
-            items.back().J = dep;
             parts.push_back( s->part_scratch() );
         }
-        // tables of the last build may still be read by kernels on the way
-        zpic::hip_check( hipStreamSynchronize( stream() ), "hipStreamSynchronize" );
         check( batch_particles_new( &side, items.data(), (int) items.size(), zpic_get_threads_per_tile(), parts.data(),
                                     (int) items.size() ) );
         side_key = key;
@@ -1201,6 +1201,9 @@ bool Simulation::step_side_by_side() {
     for ( auto * s : species ) s->list_parts();
     rec( 0 );
     check( batch_particles_pass( side, stream() ) );
+    // (on the first step the buffer is allocated while the pass runs)
+    float * const dep = current.deposit_buffer();
+    check( batch_particles_merge( side, dep, stream() ) );
     rec( 1 );
     check( batch_particles_sort( side, stream() ) );
     for ( size_t i = 2; i <= 2 * nsp; i++ ) rec( i );

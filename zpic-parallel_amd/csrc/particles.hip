@@ -463,7 +463,8 @@ struct TileArray {
 
 // Single-instance launches pass map == nullptr and use `a` with tile =
 // blockIdx.x; batched launches pass a table of per-instance arguments and a
-// map from block to (instance, tile).
+// map from block to (instance, tile); the species of one instance side by side
+// a table, entry blockIdx.y, and no map.
 template <class A>
 __device__ inline int select_instance( A & a, const A * tab, const int2 * map ) {
     if ( map ) {
@@ -471,6 +472,7 @@ __device__ inline int select_instance( A & a, const A * tab, const int2 * map ) 
         a = gbl( tab )[r.x];
         return r.y;
     }
+    if ( tab ) a = gbl( tab )[blockIdx.y];
     return blockIdx.x;
 }
 
@@ -482,6 +484,7 @@ __device__ inline int select_item( A & a, const A * tab, const int2 * map, int g
         a = gbl( tab )[r.x];
         return r.y;
     }
+    if ( tab ) a = gbl( tab )[blockIdx.y];
     return g;
 }
 
@@ -495,6 +498,7 @@ __device__ inline void particles_tile( const PartArgs & a, const int y, float * 
     const bool in_parts = MOVE && !DET && a.parts.on;
     int t = y, part = 0, nparts = 1;
     if ( in_parts ) {
+        if ( y >= a.parts.cap ) return;  // (another species' list is longer)
         const gptr<const int> item = gbl( (const int *) a.parts.item ) + 2 * y;
         const int total = gbl( a.parts.total )[0];
         t = item[0];
@@ -964,11 +968,11 @@ __global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge( PartArgs a, const
 
 // The same for the `group` species of an instance that ran side by side
 // (entries e[0], e[stride], ...): their J regions, species after species, are
-// the tile's J.
+// the tile's region of J.
 __device__ inline void part_merge_group( const PartArgs * const e, const int stride, const int group, const int t,
-                                         const int slice, const int slices ) {
+                                         const int slice, const int slices, float3 * const J ) {
     const int vol3 = 3 * e[0].g.vol, n = 3 * e[0].g.ext_x * e[0].g.ext_y;
-    const gptr<float> Jt = gbl( reinterpret_cast<float *>( e[0].J ) ) + (size_t) t * vol3;
+    const gptr<float> Jt = gbl( reinterpret_cast<float *>( J ) ) + (size_t) t * vol3;
     for ( int k = slice * blockDim.x + threadIdx.x; k < n; k += slices * blockDim.x ) {
         float total = 0.0f;
         for ( int g = 0; g < group; g++ ) {
@@ -991,10 +995,13 @@ __device__ inline void part_merge_group( const PartArgs * const e, const int str
     if ( slice == 0 )
         for ( int g = 0; g < group; g++ ) part_merge_counts( gbl( e )[g * stride], t );
 }
-// map: workgroup -> (instance, tile); entries instance * group ...
-__global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge_group( const PartArgs * tab, const int2 * map, int group ) {
-    const int2 r = gbl( map )[blockIdx.x];
-    part_merge_group( tab + r.x * group, 1, group, r.y, blockIdx.y, gridDim.y );
+// map: workgroup -> (instance, tile), null: one instance, whose current goes to
+// J; entries instance * group ...
+__global__ void __launch_bounds__( MERGE_BLOCK ) k_part_merge_group( const PartArgs * tab, const int2 * map, int group,
+                                                                     float3 * J ) {
+    int2 r = make_int2( 0, blockIdx.x );
+    if ( map ) r = gbl( map )[blockIdx.x];
+    part_merge_group( tab + r.x * group, 1, group, r.y, blockIdx.y, gridDim.y, map ? tab[r.x * group].J : J );
 }
 // workgroups per tile: a tile's elements over several where the tiles are few
 int merge_slices( int ntiles ) { return ntiles <= 256 ? 4 : 1; }
@@ -2162,6 +2169,11 @@ struct BatchParticlePlan {
     int group = 0;             // species that run side by side (0: one plan per species)
     int2 * d_inst = nullptr;   // group > 0: block -> (instance, tile)
     int ninst = 0;             // its length
+    // one instance's species side by side: no maps (with one entry per tile and
+    // part they made the first step of 64x64 tiles 190 us longer), the grids'
+    // y is the species
+    bool single = false;
+    int max_cap = 0;           // longest list of parts
     EnergyArgs * d_energy = nullptr;  // [nentries]
     std::vector<PartArgs> h_part;
 };
@@ -2184,6 +2196,7 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
     std::vector<EnergyArgs> energies( n );
     std::vector<int2> map, pmap, inst;
     plan->group = group;
+    plan->single = group == n;
     bool lbuf = true;
     size_t lds_with = 0;
     for ( int e = 0; e < n; e++ ) {
@@ -2220,16 +2233,25 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
                               it.periodic_y, parts ? parts + e : nullptr );
         const int nt = it.fld.ntiles_x * it.fld.ntiles_y;
         energies[e] = EnergyArgs{ it.tile_energy, nt, it.energy_out };
+        plan->max_tiles = std::max( plan->max_tiles, nt );
+        plan->max_vol = std::max( plan->max_vol, it.fld.tile_vol );
+        plan->max_cap = std::max( plan->max_cap, a.parts.cap );
+        if ( plan->single ) {
+            if ( nt != plan->max_tiles ) { delete plan; return set_error( ZPIC_EINVAL, "species of one instance differ in their tiles" ); }
+            plan->nblocks += nt;
+            plan->ninst = nt;
+            continue;
+        }
         for ( int t2 = 0; t2 < nt; t2++ ) map.push_back( make_int2( e, t2 ) );
         if ( group > 0 && e % group == 0 )
             for ( int t2 = 0; t2 < nt; t2++ ) inst.push_back( make_int2( e / group, t2 ) );
         for ( int y = 0; y < ( a.parts.on ? a.parts.cap : nt ); y++ ) pmap.push_back( make_int2( e, y ) );
-        plan->max_tiles = std::max( plan->max_tiles, nt );
-        plan->max_vol = std::max( plan->max_vol, it.fld.tile_vol );
     }
-    plan->nblocks = (int) map.size();
-    plan->nitems = (int) pmap.size();
-    plan->ninst = (int) inst.size();
+    if ( !plan->single ) {
+        plan->nblocks = (int) map.size();
+        plan->nitems = (int) pmap.size();
+        plan->ninst = (int) inst.size();
+    }
     if ( lbuf ) plan->lds = lds_with;
     for ( PartArgs & a : plan->h_part ) a.lbuf = lbuf;
     {
@@ -2266,9 +2288,9 @@ int batch_particles_create( BatchParticlePlan ** out, const zpic_batch_species *
     }
     plan->d_part = (PartArgs *) ( plan->tables + o1 );
     plan->d_sort = (SortArgs *) ( plan->tables + o2 );
-    plan->d_map = (int2 *) ( plan->tables + o3 );
+    plan->d_map = map.empty() ? nullptr : (int2 *) ( plan->tables + o3 );
     plan->d_energy = (EnergyArgs *) ( plan->tables + o4 );
-    plan->d_items = (int2 *) ( plan->tables + o5 );
+    plan->d_items = pmap.empty() ? nullptr : (int2 *) ( plan->tables + o5 );
     plan->d_inst = inst.empty() ? nullptr : (int2 *) ( plan->tables + o6 );
     *out = plan;
     return ZPIC_OK;
@@ -2282,13 +2304,13 @@ __global__ void __launch_bounds__( 256 ) k_batch_energy( const EnergyArgs * tab 
 int batch_particles_place( BatchParticlePlan * plan, hipStream_t st ) {
     const SortArgs sd{};
     if ( plan->staged ) {
-        const int slices = sort_slices( plan->nblocks );
-        const dim3 grid( ( plan->nblocks * slices + SORT_WAVES - 1 ) / SORT_WAVES );
+        const int slices = sort_slices( plan->nblocks ), n = plan->single ? plan->max_tiles : plan->nblocks;
+        const dim3 grid( ( n * slices + SORT_WAVES - 1 ) / SORT_WAVES, plan->single ? plan->nentries : 1 );
         hipLaunchKernelGGL( k_sort_shift, grid, dim3( SORT_WAVES * WAVE ), 0, st, sd, (const SortArgs *) plan->d_sort,
-                            (const int2 *) plan->d_map, plan->nblocks, slices );
+                            (const int2 *) plan->d_map, n, slices );
         ZPIC_LAUNCH_CHECK( "k_sort_shift (batch)" );
         hipLaunchKernelGGL( k_sort_in_fast, grid, dim3( SORT_WAVES * WAVE ), 0, st, sd, (const SortArgs *) plan->d_sort,
-                            (const int2 *) plan->d_map, plan->nblocks, slices );
+                            (const int2 *) plan->d_map, n, slices );
         ZPIC_LAUNCH_CHECK( "k_sort_in_fast (batch)" );
     } else {
         hipLaunchKernelGGL( k_sort_out<false>, dim3( plan->nblocks ), dim3( SORT_BLOCK ), 0, st, sd,
@@ -2301,19 +2323,26 @@ int batch_particles_place( BatchParticlePlan * plan, hipStream_t st ) {
     return ZPIC_OK;
 }
 
+// The particle pass, and what its parts leave to the merge (J: of a plan for
+// one instance, whose tables do not hold it).
 int batch_particles_pass( BatchParticlePlan * plan, void * stream ) {
     hipStream_t st = as_stream( stream );
-    PartArgs dummy{};
-    hipLaunchKernelGGL( ( k_particles<true, true, false> ), dim3( plan->nitems ), dim3( plan->threads ), plan->lds, st,
-                        dummy, (const PartArgs *) plan->d_part, (const int2 *) plan->d_items );
+    hipLaunchKernelGGL( ( k_particles<true, true, false> ), plan->single ? dim3( plan->max_cap, plan->nentries ) : dim3( plan->nitems ),
+                        dim3( plan->threads ), plan->lds, st, PartArgs{}, (const PartArgs *) plan->d_part,
+                        (const int2 *) plan->d_items );
     ZPIC_LAUNCH_CHECK( "k_particles (batch)" );
+    return ZPIC_OK;
+}
+
+int batch_particles_merge( BatchParticlePlan * plan, float * J, void * stream ) {
+    hipStream_t st = as_stream( stream );
     if ( plan->group > 0 ) {
         hipLaunchKernelGGL( k_part_merge_group, dim3( plan->ninst, merge_slices( plan->ninst ) ), dim3( MERGE_BLOCK ), 0, st,
-                            (const PartArgs *) plan->d_part, (const int2 *) plan->d_inst, plan->group );
+                            (const PartArgs *) plan->d_part, (const int2 *) plan->d_inst, plan->group, (float3 *) J );
         ZPIC_LAUNCH_CHECK( "k_part_merge_group" );
     } else if ( plan->nitems > plan->nblocks ) {
-        hipLaunchKernelGGL( k_part_merge, dim3( plan->nblocks, merge_slices( plan->nblocks ) ), dim3( MERGE_BLOCK ), 0, st, dummy,
-                            (const PartArgs *) plan->d_part, (const int2 *) plan->d_map );
+        hipLaunchKernelGGL( k_part_merge, dim3( plan->nblocks, merge_slices( plan->nblocks ) ), dim3( MERGE_BLOCK ), 0, st,
+                            PartArgs{}, (const PartArgs *) plan->d_part, (const int2 *) plan->d_map );
         ZPIC_LAUNCH_CHECK( "k_part_merge (batch)" );
     }
     return ZPIC_OK;
@@ -2523,7 +2552,7 @@ __global__ void __launch_bounds__( BLOCK, 4 ) k_batch_step( StepTables T ) {
             break;
         }
         case SK_MERGE_ALL:
-            for ( int t = it.t0; t < it.t1; t++ ) part_merge_group( T.part + it.arg, T.n, T.nslots, t, 0, 1 );
+            for ( int t = it.t0; t < it.t1; t++ ) part_merge_group( T.part + it.arg, T.n, T.nslots, t, 0, 1, T.part[it.arg].J );
             break;
         case SK_CURRENT: {
             const grid_ops::CurArgs & a = T.cur[it.arg];
@@ -3381,12 +3410,16 @@ extern "C" {
 int zpic_batch_particles_advance( zpic_batch_particles * b, void * stream ) {
     if ( !b || !b->plan ) return set_error( ZPIC_EINVAL, "null batch" );
     if ( int rc = batch_particles_pass( b->plan, stream ) ) return rc;
+    if ( int rc = batch_particles_merge( b->plan, reinterpret_cast<float *>( b->plan->h_part[0].J ), stream ) ) return rc;
     return batch_particles_sort( b->plan, stream );
 }
 
 }  // extern "C"
 
 int zpic::batch_particles_pass( zpic_batch_particles * b, void * stream ) { return batch_particles_pass( b->plan, stream ); }
+int zpic::batch_particles_merge( zpic_batch_particles * b, float * J, void * stream ) {
+    return batch_particles_merge( b->plan, J, stream );
+}
 int zpic::batch_particles_sort( zpic_batch_particles * b, void * stream ) { return batch_particles_sort( b->plan, stream ); }
 
 extern "C" {

@@ -71,11 +71,12 @@ int tile_sort_copy( zpic_particles * p, zpic_particles * tmp, zpic_sort * s, int
                     int periodic_x, int periodic_y, int mode, const PartScratch * parts, void * stream );
 // group > 0: the n items are the species of n / group instances, `group` of
 // each side by side, all in parts, and go through each stage together; J is
-// written, not added to.
+// written, not added to.  With n = group (one instance) J is given to the merge.
 int batch_particles_new( zpic_batch_particles ** out, const zpic_batch_species * items, int n, int threads_per_tile,
                          const PartScratch * parts, int group = 0 );
-// zpic_batch_particles_advance in its two halves.
+// zpic_batch_particles_advance in its three parts.
 int batch_particles_pass( zpic_batch_particles * plan, void * stream );
+int batch_particles_merge( zpic_batch_particles * plan, float * J, void * stream );
 int batch_particles_sort( zpic_batch_particles * plan, void * stream );
 // dep: deposit buffers of the instances, the current formed from them in one
 // stage, and with all tiles in parts the species side by side (null, or an
