@@ -24,6 +24,8 @@ def crowded(ntiles, nx, counts, seed):
     ((1, 1), (16, 16), 256, [5000]),
     ((3, 2), (8, 8), 256, [0, 1, 1023, 1024, 1025, 2048]),
     ((3, 2), (8, 8), 64, [2049, 0, 14 * 1024, 64, 16000, 3]),
+    ((3, 2), (8, 8), 256, [2047, 2048, 2049, 4096, 4097, 1]),
+    ((3, 2), (8, 8), 64, [14 * 2048, 14 * 2048 + 1, 0, 40000, 13 * 2048, 6143]),
     ((2, 2), (32, 32), 512, [30000, 1, 0, 1100]),
     ((33, 32), (8, 8), 256, [3] * 1055 + [5000]),   # more than one tile per thread of the scan
     ((32, 32), (8, 8), 256, [1] * 1000 + [0] * 23 + [9000]),

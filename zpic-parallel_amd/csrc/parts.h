@@ -6,11 +6,11 @@
 // where the tiles alone do not fill the device, or one crowded tile would
 // hold up the rest (part_rule): with one workgroup per tile, a 128x128 Weibel
 // run (64 tiles, 2 x 1M particles) took 1.18 ms a step over its first
-// thousand steps, as filaments gather up to three times the mean in a tile,
-// and takes 0.20 ms; a 64x64 box of 8x8 tiles and as many particles 1.92 and
-// 0.20 ms.  The list of parts follows the tiles'
-// particle counts: the sort writes it for the next pass, and part_list()
-// where the counts came about in another way.
+// thousand steps, as filaments gather up to three times the mean in a tile;
+// cut, and with the species side by side, it takes 0.10 to 0.11 ms, a 64x64
+// box of 8x8 tiles and as many particles 0.09 for 1.92.  The list of parts
+// follows the tiles' particle counts: the sort writes it for the next pass,
+// and part_list() where the counts came about in another way.
 #pragma once
 
 #include <algorithm>
@@ -23,7 +23,7 @@ constexpr int PART_SEG = 64;      // ints per tile of the segment table
 constexpr int PART_MAX_SEG = 59;  // wave segments of one tile
 constexpr int PART_MAX = 14;
 constexpr unsigned PART_TARGET = 1024;  // parts beyond one per tile, at most
-constexpr unsigned PART_MIN = 1024;     // particles of a part, at least
+constexpr unsigned PART_MIN = 2048;     // particles of a part, at least
 
 struct PartScratch {
     int on = 0;    // 0: tiles are not cut, the rest is unused
@@ -46,10 +46,14 @@ struct PartScratch {
 inline bool part_rule( int ntiles ) { return ntiles <= 4096; }
 
 // Parts beyond one per tile for a buffer of max_part particles, and the
-// particles of a part that keep to them: no fewer than PART_MIN, which take a
-// workgroup about as long as its staging and its J region.  (512 and 2048
-// parts measured within 3 % on these runs, 4096 of at least 256 particles up
-// to 15 % slower on a 512x512 grid.)
+// particles of a part that keep to them, no fewer than PART_MIN: a part also
+// stages its tile's fields and writes and merges a J region, which costs time
+// where the device is full anyway.  Microseconds a step at PART_MIN 1024, 2048
+// and 4096: 64 tiles of 2 x 16384 particles 104, 99 and 98, of one such species
+// 78, 77 and 81, 16 tiles of 16384 63, 64 and 71; 64 quiet instances in one
+// persistent launch 8970, 8700 and 8600 (8560 without parts, evolved 9600, 9350
+// and 9300).  PART_TARGET 512 instead of 1024: an evolved 512x512 run in 1024
+// tiles 805 for 675; 2048: 16384 particles in each of 1024 tiles 302 for 290.
 inline int part_extra( unsigned max_part ) { return (int) std::min( PART_TARGET, max_part / PART_MIN + 1 ); }
 inline int part_size( unsigned max_part, int extra ) {
     return (int) std::max( PART_MIN, ( max_part / (unsigned) extra + 64 ) & ~63u );
