@@ -24,10 +24,16 @@ namespace {
 constexpr int WAVE = 64;
 constexpr int PHA_BLOCK = 512;
 // 96 KiB, one workgroup per CU.  9.4 million particles on 110 x 110 bins of two
-// momenta take 135 us so, 7473 by global atomics alone (8192 bins, 64 KiB), 262
+// momenta take 129 us so, 7473 by global atomics alone (8192 bins, 64 KiB), 262
 // with float atomics on 48 KiB.
 constexpr int PHA_LDS_BINS = 12288;
-constexpr int PHA_GROUPS = 1024;    // workgroups aimed at: each adds its bins to the output once
+// Workgroups aimed at, each of which clears its bins and adds them to the output
+// once: as many as run at the same time, four per CU, fewer where the bins
+// leave no room for four (9.4 million particles on 110 x 110 bins: 135 us with
+// 768 workgroups, 129 with 240; 0.17 million in 300 tiles on 200 x 60: 47 with
+// 300, 40 with 150, 43 with float atomics).
+constexpr int PHA_CUS = 256, PHA_PER_CU = 4;
+constexpr size_t CU_LDS = 163840;
 
 struct PhaAxis {
     int quant;   // 0 x, 1 y, 2 ux, 3 uy, 4 uz
@@ -220,18 +226,23 @@ extern "C" int zpic_phasespace( const zpic_particles * p, int ntiles_x, int ntil
         // tiles above one another share their bins of x, beside one another
         // those of y
         const bool over_y = quant0 == 0 && !( two && quant1 == 1 );
-        const int n = ( nt + PHA_GROUPS - 1 ) / PHA_GROUPS;
-        a.gx = over_y ? 1 : std::min( n, ntiles_x );
-        a.gy = over_y ? std::min( n, ntiles_y ) : 1;
-        const int groups = ( ( ntiles_x + a.gx - 1 ) / a.gx ) * ( ( ntiles_y + a.gy - 1 ) / a.gy );
         // the most bins a workgroup's particles reach along each axis
         auto reach = []( const PhaAxis & x, int cells ) -> long long {
             if ( x.quant > 1 ) return x.size;
             const float r = (float) cells * x.rdx + 4.0f;
             return r < (float) x.size ? (long long) r : x.size;
         };
-        const long long most = reach( a.a0, quant0 == 0 ? a.gx * nx : a.gy * ny ) * ( two ? reach( a.a1, a.gy * ny ) : 1 );
-        const int cap = (int) std::min( most, (long long) PHA_LDS_BINS );
+        auto group = [&]( int n ) {  // of n tiles: its bins in LDS
+            a.gx = over_y ? 1 : n;
+            a.gy = over_y ? n : 1;
+            const long long most = reach( a.a0, quant0 == 0 ? a.gx * nx : a.gy * ny ) * ( two ? reach( a.a1, a.gy * ny ) : 1 );
+            return (int) std::min( most, (long long) PHA_LDS_BINS );
+        };
+        const int per_cu = std::min( (int) ( CU_LDS / ( sizeof( u64 ) * group( 1 ) ) ), PHA_PER_CU );
+        const int along = over_y ? ntiles_y : ntiles_x, across = nt / along;
+        int n = 1;
+        while ( n < along && ( along + n - 1 ) / n * across > PHA_CUS * per_cu ) n++;
+        const int cap = group( n ), groups = ( along + n - 1 ) / n * across;
         hipLaunchKernelGGL( k_phasespace, dim3( groups ), dim3( PHA_BLOCK ), sizeof( u64 ) * cap, st, a, out, cap );
     }
     ZPIC_LAUNCH_CHECK( "k_phasespace" );
