@@ -78,3 +78,36 @@ def test_field_energy_order(pair):
         sq = (f * f).reshape(fast.ntiles, -1, 3).astype(np.float64)
         tiles = np.add.accumulate(sq, axis=1)[:, -1]
         assert np.array_equal(np.add.accumulate(tiles, axis=0)[-1], got)
+
+
+@pytest.mark.parametrize("n", [64, 100, 127])
+def test_charge_of_large_tiles(n):
+    """Tiles up to the largest that the charge takes (128 KiB of LDS), larger
+    than a particle pass's, through the stage entry point."""
+    import pyzpic as zp
+    import torch
+
+    class Particles(ctypes.Structure):
+        _fields_ = [(k, ctypes.c_void_p) for k in ("np", "offset", "ix", "x", "u")] + [("max_part", ctypes.c_uint32)]
+
+    L = zp.lib()
+    L.zpic_deposit_charge.restype = ctypes.c_int
+    L.zpic_deposit_charge.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
+    g = zp.Geom()
+    assert L.zpic_geom_init(ctypes.byref(g), 2, 1, n, n, 0, 1) == 0
+    rng = np.random.default_rng(n)
+    count = 6000
+    t = dict(np=torch.tensor([count, count], dtype=torch.int32), offset=torch.tensor([0, count], dtype=torch.int32),
+             ix=torch.from_numpy(rng.integers(0, n, (2 * count, 2)).astype(np.int32)),
+             x=torch.from_numpy((rng.random((2 * count, 2)) - 0.5).astype(np.float32)), u=torch.zeros(2 * count, 3))
+    t = {k: v.cuda() for k, v in t.items()}
+    p = Particles(*(t[k].data_ptr() for k in ("np", "offset", "ix", "x", "u")), max_part=2 * count)
+    out = []
+    for det in (0, 1):
+        rho = torch.zeros(2 * g.tile_vol, device="cuda")
+        torch.cuda.synchronize()
+        assert L.zpic_deposit_charge(ctypes.byref(p), ctypes.byref(g), rho.data_ptr(), -0.25, det, None) == 0
+        torch.cuda.synchronize()
+        out.append(rho.cpu().numpy())
+    assert np.abs(out[1]).max() > 0
+    close(*out)

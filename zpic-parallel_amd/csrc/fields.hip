@@ -81,12 +81,13 @@ __global__ void __launch_bounds__( TILE_BLOCK ) k_kernel3( K3Args args, const K3
 
 // Up to CUR_FEW tiles, a workgroup of 256 threads for each, so that the tiles
 // still reach every compute unit; more tiles, two per workgroup of 128
-// threads, whose fixed costs then halve.  Microseconds a call, tiles of the
-// given cells and passes (in brackets the form that looked the neighbours up
-// for each element, ran the passes in LDS and took four tiles per 128
-// threads): 8x8 of 16x16, 0: 5 (26); 33x45 of 32x16, 5: 18 (123); 256x32 of
-// 16x16, 5: 54 (105); 128x128 of 16x16, 1: 65 (78).  On the largest, 256
-// threads and one tile take 72, 128 threads and one tile 70.
+// threads, whose fixed costs then halve.  Microseconds a call repeated on the
+// same buffers, tiles of the given cells and passes (in brackets the form with
+// branches per element, the passes in LDS and four tiles per 128 threads):
+// 8x8 of 16x16, 0: 5 (26); 33x45 of 32x16, 5: 18 (122); 256x32 of 16x16, 5:
+// 54 (104); 128x128 of 16x16, 1: 65 (78), in a step, which leaves less of the
+// 143 MB in the last-level cache, 87-95 (104-108).  On the largest, 256 threads
+// and one tile take 72, 128 threads and one tile 70.
 constexpr int CUR_FEW = 4096;
 constexpr int CUR_BLOCK_FEW = 256;
 constexpr int CUR_BLOCK = 128;

@@ -7,8 +7,8 @@
 // hold up the rest (part_rule): with one workgroup per tile, a 128x128 Weibel
 // run (64 tiles, 2 x 1M particles) took 1.18 ms a step over its first
 // thousand steps, as filaments gather up to three times the mean in a tile;
-// cut, and with the species side by side, it takes 0.10 to 0.11 ms, a 64x64
-// box of 8x8 tiles and as many particles 0.09 for 1.92.  The list of parts
+// cut, and with the species side by side, it takes 0.11 ms, a 64x64 box of 8x8
+// tiles and as many particles 0.11 for 1.96.  The list of parts
 // follows the tiles' particle counts: the sort writes it for the next pass,
 // and part_list() where the counts came about in another way.
 #pragma once
@@ -51,8 +51,8 @@ inline bool part_rule( int ntiles ) { return ntiles <= 4096; }
 // where the device is full anyway.  Microseconds a step at PART_MIN 1024, 2048
 // and 4096: 64 tiles of 2 x 16384 particles 104, 99 and 98, of one such species
 // 78, 77 and 81, 16 tiles of 16384 63, 64 and 71; 64 quiet instances in one
-// persistent launch 8970, 8700 and 8600 (8560 without parts, evolved 9600, 9350
-// and 9300).  PART_TARGET 512 instead of 1024: an evolved 512x512 run in 1024
+// persistent launch 8910, 8670 and 8570 (8490 with no tile cut), after 300 steps
+// 9600, 9350 and 9300 (9400).  PART_TARGET 512 instead of 1024: an evolved 512x512 run in 1024
 // tiles 805 for 675; 2048: 16384 particles in each of 1024 tiles 302 for 290.
 inline int part_extra( unsigned max_part ) { return (int) std::min( PART_TARGET, max_part / PART_MIN + 1 ); }
 inline int part_size( unsigned max_part, int extra ) {
